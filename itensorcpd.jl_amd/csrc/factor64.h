@@ -31,6 +31,10 @@ constexpr size_t FACTOR64_UNPIV_LDS = (size_t)(64 * 66 + 144) * 8;
 // pivoted path's up to rounding, and V^-1, invdiag, piv (identity) and finfo are
 // written; otherwise it returns false and writes nothing but V^-1 (which the
 // caller's pivoted path overwrites or leaves unused).  Uniform result.
+//
+// Bound by its serial chain (about 2 us per 16-row panel), so only the ceil(R / 16)
+// panels that hold any of V are worked on.  In the launch that it rides, us: R = 10,
+// 11 (20 with all four panels); R = 24, 17 (21); R = 37, 19 (21).
 __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, int R, double tol,
                                                    double* __restrict__ Vinv, double* __restrict__ invdiag,
                                                    int* __restrict__ piv, int* __restrict__ finfo, double* S) {
@@ -38,6 +42,7 @@ __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, 
     double* red = S + FACTOR64_RED;   // [0, 16) scalars, then 1/U(j,j) and the broadcast row
     const int t = threadIdx.x, l = t & 63, c = l & 15, g = l >> 4;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nbk = (R + 15) >> 4;   // 16-row panels that hold any of V; the rest stay the identity
     if (t == 0) red[12] = 0.0;   // set by wave 0 when a pivot is not > 0
     // V (mode order of the Hadamard as the pivoted path), identity beyond R; thread
     // (w, l) fills column l of rows w, w + 4, ...; two modes' loads in flight at once
@@ -53,9 +58,14 @@ __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, 
 #pragma unroll
             for (int k = 0; k < 16; ++k) {
                 const int i = w + 4 * k;
-                const bool in = i < R && l < R;
-                g0[k] = (in && on0) ? G0[i * R + l] : 1.0;
-                g1[k] = (in && on1) ? G1[i * R + l] : 1.0;
+                const int x = (i < R && l < R) ? i * R + l : 0;
+                g0[k] = G0[x];
+                g1[k] = G1[x];
+            }
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                if (!on0) g0[k] = 1.0;
+                if (!on1) g1[k] = 1.0;
             }
 #pragma unroll
             for (int k = 0; k < 16; ++k) v[k] = (v[k] * g0[k]) * g1[k];
@@ -85,7 +95,7 @@ __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, 
     __syncthreads();
     double* invd = red + 16;      // 1/U(j,j), 64 doubles
     double* rowj = red + 80;      // one row of the block row, 64 doubles
-    for (int kb = 0; kb < 4; ++kb) {
+    for (int kb = 0; kb < nbk; ++kb) {
         const int b0 = 16 * kb;
         if (w == 0) {
             // Block row kb (rows b0..b0+15, all 64 columns): lane l holds column l.
@@ -126,10 +136,10 @@ __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, 
         // trailing update of the upper blocks kb < ib <= jb (round-robin over waves).
         // f64 16x16x4 layout: A lane (c, g) = A[c][k0+g], B lane = B[k0+g][c], result
         // v = D[g+4v][c]
-        if (kb < 3) {
+        if (kb + 1 < nbk) {
             int idx = 0;
-            for (int ib = kb + 1; ib < 4; ++ib)
-                for (int jb = ib; jb < 4; ++jb, ++idx) {
+            for (int ib = kb + 1; ib < nbk; ++ib)
+                for (int jb = ib; jb < nbk; ++jb, ++idx) {
                     if ((idx & 3) != w) continue;
                     d4 acc;
 #pragma unroll
@@ -146,7 +156,7 @@ __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, 
     }
     // diagonal blocks of U^-1, wave w block w: lane c computes column c by
     // substitution (zero below the diagonal; the four 16-lane groups alike)
-    {
+    if (w < nbk) {
         const int b0 = 16 * w;
         double xv[16];
 #pragma unroll
@@ -168,10 +178,10 @@ __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, 
     // off-diagonal blocks of U^-1, block row bi from the bottom, wave w column
     // bi + 1 + w: X_ij = -X_ii sum_{k=i+1..j} U_ik X_kj, from row i of U and the
     // finished rows below; row i is overwritten after every wave has read it
-    for (int bi = 2; bi >= 0; --bi) {
+    for (int bi = nbk - 2; bi >= 0; --bi) {
         const int bj = bi + 1 + w;
         d4 out = (d4){0.0, 0.0, 0.0, 0.0};
-        if (bj < 4) {
+        if (bj < nbk) {
             const int i = 16 * bi + c;
             d4 acc = (d4){0.0, 0.0, 0.0, 0.0};
             for (int bk = bi + 1; bk <= bj; ++bk)
@@ -184,7 +194,7 @@ __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, 
             for (int v = 0; v < 4; ++v) out = mfma_f64(-S[(16 * bi + c) * LDT + 16 * bi + 4 * v + g], acc[v], out);
         }
         __syncthreads();
-        if (bj < 4) {
+        if (bj < nbk) {
 #pragma unroll
             for (int v = 0; v < 4; ++v) S[(16 * bi + g + 4 * v) * LDT + 16 * bj + c] = out[v];
         }
@@ -202,7 +212,7 @@ __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, 
         const int ta = ZT[w][q][0], tb = ZT[w][q][1];
         if (ta < 0 || 16 * tb >= R) continue;
         d4 acc = (d4){0.0, 0.0, 0.0, 0.0};
-        for (int k0 = 16 * tb; k0 < 64; k0 += 4)
+        for (int k0 = 16 * tb; k0 < 16 * nbk; k0 += 4)
             acc = mfma_f64(S[(16 * ta + c) * LDT + k0 + g], S[(16 * tb + c) * LDT + k0 + g], acc);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
