@@ -272,6 +272,8 @@ int itcpd_plan_create(itcpd_plan** out, int32_t order, const int64_t* dims, int6
     if ((rc = dmalloc(&p->qr_aux, (size_t)(R * R + 4 * R)))) return bail(rc);
     if ((rc = dmalloc(&p->piv, (size_t)(2 * R)))) return bail(rc);
     if ((rc = dmalloc(&p->finfo, 4))) return bail(rc);
+    if (const int64_t n = krp64_elems(p))
+        if ((rc = dmalloc(&p->Wrest, (size_t)n))) return bail(rc);
     if (p->s > 1 && (rc = dmalloc(&p->PL, (size_t)(p->ML * R)))) return bail(rc);
     if (order - p->s > 1 && (rc = dmalloc(&p->PR, (size_t)(p->MR * R)))) return bail(rc);
     {
@@ -334,7 +336,7 @@ int itcpd_plan_destroy(itcpd_plan* p) {
     dfree(p->lamprev);
     dfree(p->smp_ws);
     dfree(p->sk_ws);
-    dfree(p->T64);
+    dfree(p->Wrest);
     dfree(p->smp_iws);
     dfree(p->xg_part);
     if (p->chk_host) (void)hipHostFree(p->chk_host);

@@ -104,8 +104,6 @@ struct itcpd_plan {
     int elt_bytes = 8;
     const void* T = nullptr;
     void* T_owned = nullptr;
-    double* T64 = nullptr;     // FP64 copy of an FP32-stored tensor (FP64 GEMMs), made on first use
-    bool T64_failed = false;   // no memory for it: the FP64 GEMMs read the FP32 tensor
     int prec = ITCPD_FP64;
     int alg = ITCPD_ALG_KRP_FREE_NORMAL;
     int s = 1;               // dimension-tree split: left = modes [0, s), right = [s, N)
@@ -132,6 +130,7 @@ struct itcpd_plan {
     double* PL = nullptr;                      // ML x Rp partial of the left side (if s > 1)
     float* Af = nullptr;                       // FP32 copy of the KRP side's first factor (reduced precision)
     float* Kt = nullptr;                       // FP32-stored T, reduced precision: a side's KRP, rank-major
+    double* Wrest = nullptr;                   // a side's Khatri-Rao product or rest weights (rank fastest)
     double* PR = nullptr;                      // MR x Rp partial of the right side (if N-s > 1)
     double* parts = nullptr;                   // split-K partial buffer
     size_t parts_elems = 0;
@@ -195,6 +194,7 @@ int launch_left_gemm(itcpd_plan* p, MSrc* ms, int factor_mode = -1);
 int launch_right_gemm(itcpd_plan* p, MSrc* ms, int factor_mode = -1);
 // M of `mode` from PL / PR; with factor_mode >= 0 also that mode's factorisation
 int launch_side_ttv(itcpd_plan* p, int mode, MSrc* ms, int factor_mode = -1);
+int64_t krp64_elems(const itcpd_plan* p);      // doubles of p->Wrest
 int mttkrp_mode(itcpd_plan* p, int mode);      // full M_mode into p->M from the current factors
 // out = the sum of ms's partials; factor_mode >= 0: that mode's factorisation too
 // (in an extra workgroup for R <= 64, else as its own launch after the sum);

@@ -3,39 +3,20 @@
 // The reference computes each M_n = T_(n) (KRP of the other factors) separately,
 // one full contraction of T per rank slice (algebra/had_contract.jl:111-121).
 // Here the modes are split into a left side [0, s) and a right side [s, N):
-//   left  GEMM  P_L(mL, r) = sum_mR T(mL, mR) KRP_right(mR, r)   ("TK": output rows contiguous in T)
-//   right GEMM  P_R(mR, r) = sum_mL T(mL, mR) KRP_left(mL, r)    ("TR": reduction contiguous in T)
+//   left  GEMM  P_L(mL, r) = sum_mR T(mL, mR) KRP_right(mR, r)   (output rows contiguous in T)
+//   right GEMM  P_R(mR, r) = sum_mL T(mL, mR) KRP_left(mL, r)    (reduction contiguous in T)
 // with T viewed as an ML x MR column-major matrix (mL = left multi-index, mode 0
-// fastest).  The KRP operand is generated on the fly from the factors.  A side
+// fastest).  The KRP operand is generated on the fly from the factors (gemm64.h).  A side
 // with one mode yields its M directly; a side with several modes gets each M_n
 // from its partial by a Hadamard-reduce against the side's other (current)
 // factors.  T is read twice per sweep.
 #include "internal.h"
 #include "factor64.h"
+#include "gemm64.h"
 
 namespace itcpd {
 
 typedef double dv2 __attribute__((ext_vector_type(2)));
-
-template <typename TT>
-__device__ __forceinline__ double ld1(const TT* p) { return (double)p[0]; }
-
-// Loads MB consecutive elements (MB even; the run must be 16-byte aligned for doubles).
-template <typename TT, int MB>
-__device__ __forceinline__ void ld_run(const TT* __restrict__ p, double* out) {
-    if constexpr (sizeof(TT) == 8) {
-        const dv2* q = reinterpret_cast<const dv2*>(p);
-#pragma unroll
-        for (int k = 0; k < MB / 2; ++k) {
-            dv2 v = q[k];
-            out[2 * k] = v.x;
-            out[2 * k + 1] = v.y;
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < MB; ++k) out[k] = (double)p[k];
-    }
-}
 
 // Weight of a "rest" multi-index for the side's modes 1..nm-1 at rank r.
 // Factor layout: rank-fastest (Rp x I) when rank_fast, else column-major (I x Rp).
@@ -49,114 +30,6 @@ __device__ __forceinline__ double rest_weight(const Side& sd, int64_t rest, int 
         w *= rank_fast ? sd.fac[q][d * Rp + r] : sd.fac[q][d + sd.dim[q] * r];
     }
     return w;
-}
-
-// ---------------------------------------------------------------- TK GEMM
-// out(mL, r) = sum over reduction index mR = i + I0*rest of T(mL, mR) KRP(mR, r),
-// KRP(mR, r) = At0[i*Rp + r] * prod_{q>=1} Atq[digit_q*Rp + r].
-// Wave tile: 16*MB rows x 16*RB ranks.  Lane (g = l>>4, c = l&15) owns rows
-// m0 + MB*c .. + MB-1 (a contiguous run, loaded as vectors) at reduction index g of
-// each 4-step.  The reduction range [kk0, kk1) counts 4-steps over (rest, i).
-template <typename TT, int RB, int MB, int U, bool FAST>
-__global__ __launch_bounds__(256, 2) void k_tk(const TT* __restrict__ T, int64_t ML, Side sd,
-                                               int64_t nsteps_i, int64_t kk_per_split,
-                                               int64_t kk_total, int Rp, int R,
-                                               double* __restrict__ out, int64_t out_ld,
-                                               int64_t split_stride,
-                                               const DevCheck* __restrict__ chk) {
-    if (chk->done) return;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int c = lane & 15, g = lane >> 4;
-    const int64_t m0 = ((int64_t)blockIdx.x * 4 + wave) * (16 * MB);
-    if (m0 >= ML) return;
-    const int r0 = blockIdx.y * (16 * RB);
-    const int64_t kk0 = (int64_t)blockIdx.z * kk_per_split;
-    const int64_t kk1 = kk0 + kk_per_split < kk_total ? kk0 + kk_per_split : kk_total;
-    const int64_t I0 = sd.dim[0];
-    const double* __restrict__ At0 = sd.fac[0];
-    const int64_t mrow = m0 + MB * c;
-
-    d4 acc[RB][MB];
-#pragma unroll
-    for (int a = 0; a < RB; ++a)
-#pragma unroll
-        for (int b = 0; b < MB; ++b) acc[a][b] = (d4){0.0, 0.0, 0.0, 0.0};
-
-    int64_t kk = kk0;
-    while (kk < kk1) {
-        const int64_t rest = kk / nsteps_i;
-        const int64_t s_lo = kk - rest * nsteps_i;
-        int64_t s_hi = nsteps_i;
-        if ((rest + 1) * nsteps_i > kk1) s_hi = kk1 - rest * nsteps_i;
-        double w[RB];
-#pragma unroll
-        for (int a = 0; a < RB; ++a) w[a] = rest_weight(sd, rest, r0 + 16 * a + c, Rp, true);
-        const TT* __restrict__ Tr = T + (I0 * rest) * ML + mrow;
-
-        // two register stages: loads of the next U steps are issued before the
-        // MFMAs of the current ones
-        double ta[2][U][MB], ka[2][U][RB];
-        auto load = [&](int buf, int64_t st) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int64_t i = (st + u) * 4 + g;
-                const bool ok = (st + u < s_hi) && (FAST || i < I0);
-                if constexpr (FAST) {
-                    if (ok) {
-                        ld_run<TT, MB>(Tr + i * ML, ta[buf][u]);
-                    } else {
-#pragma unroll
-                        for (int b = 0; b < MB; ++b) ta[buf][u][b] = 0.0;
-                    }
-                } else {
-#pragma unroll
-                    for (int b = 0; b < MB; ++b)
-                        ta[buf][u][b] = (ok && mrow + b < ML) ? ld1(Tr + i * ML + b) : 0.0;
-                }
-#pragma unroll
-                for (int a = 0; a < RB; ++a)
-                    ka[buf][u][a] = ok ? At0[i * Rp + r0 + 16 * a + c] * w[a] : 0.0;
-            }
-        };
-        auto compute = [&](int buf) {
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int a = 0; a < RB; ++a)
-#pragma unroll
-                    for (int b = 0; b < MB; ++b)
-                        acc[a][b] = mfma_f64(ka[buf][u][a], ta[buf][u][b], acc[a][b]);
-        };
-        int64_t st = s_lo;
-        load(0, st);
-        while (true) {
-            const bool more1 = st + U < s_hi;
-            if (more1) load(1, st + U);
-            compute(0);
-            st += U;
-            if (!more1) break;
-            const bool more0 = st + U < s_hi;
-            if (more0) load(0, st + U);
-            compute(1);
-            st += U;
-            if (!more0) break;
-        }
-        kk = rest * nsteps_i + s_hi;
-    }
-
-    double* o = out + (int64_t)blockIdx.z * split_stride;
-#pragma unroll
-    for (int a = 0; a < RB; ++a)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int r = r0 + 16 * a + g + 4 * v;
-            if (r >= R) continue;
-#pragma unroll
-            for (int b = 0; b < MB; ++b) {
-                const int64_t row = mrow + b;
-                if (FAST || row < ML) o[row + out_ld * r] = acc[a][b][v];
-            }
-        }
 }
 
 // A mode's R <= 64 factorisation riding along with another launch: block x = 0 of
@@ -184,311 +57,14 @@ __device__ __forceinline__ bool factor_block(const FactorJob& fj) {
     return true;
 }
 
-// ------------------------------------------------- TK GEMM, LDS ring form
-// The same product for FP64 T, 64-rank blocks and 256-row workgroup tiles, with
-// T and the KRP rows staged through a ring of LDS slots filled by direct
-// global->LDS loads (global_load_lds_dwordx4: lane l of a wave writes 16 bytes at
-// slot offset + 16 l).  A stage is U = 2 four-steps, i.e. 8 consecutive
-// reduction indices i of one rest: 8 T columns of 256 rows (2 KB each, padded to
-// TKR_CST bytes) and 8 rows of At0 (64 ranks, 512 bytes each).  Stage
-// q + TKR_NS - 1 is requested while stage q is computed; the loads bypass
-// registers, so the bytes in flight no longer compete with the accumulators.
-//
-// Synchronisation per stage: each wave waits for its own loads of the stage
-// (vmcnt: loads return in order, so only the 5 loads of each later stage already
-// requested may still be pending) and for its LDS reads (lgkmcnt 0), then the
-// workgroup barrier makes every wave's loads visible; the slot refilled after
-// that barrier is the one read in the previous stage, which every wave has
-// finished.
-// Two slots: 302 us per launch at 512^3 rank 64, against 319 us with three (both at
-// two workgroups per CU, which the registers allow; 41 KB of LDS would take three).
-constexpr int TKR_NS = 2;
-constexpr int TKR_CST = 2048 + 64;
-constexpr int TKR_TBYTES = 8 * TKR_CST;
-constexpr int TKR_SLOT = TKR_TBYTES + 8 * 512;
-constexpr int TKR_LDS = TKR_NS * TKR_SLOT;
-
+// ---- direct global->LDS loads: lane l of a wave writes 16 bytes at dst + 16 l
 typedef __attribute__((address_space(3))) void lds_void_t;
 
 __device__ __forceinline__ void lds_dma16(const void* src, unsigned char* dst) {
     __builtin_amdgcn_global_load_lds(src, (lds_void_t*)dst, 16, 0, 0);
 }
 // s_waitcnt: vmcnt <= n (n < 16), lgkmcnt = 0, expcnt not waited for
-#define TKR_WAIT(n) __builtin_amdgcn_s_waitcnt(0x0000 | ((n) & 0xf) | (0x7 << 4) | (0x0 << 8))
-
-__global__ __launch_bounds__(256, 2) void k_tk_ring(const double* __restrict__ T, int64_t ML, Side sd,
-                                                    int64_t nsteps_i, int64_t kk_per_split,
-                                                    int64_t kk_total, int Rp, int R,
-                                                    double* __restrict__ out, int64_t out_ld,
-                                                    int64_t split_stride,
-                                                    const DevCheck* __restrict__ chk) {
-    constexpr int RB = 4, MB = 4, U = 2;
-    if (chk->done) return;
-    const int64_t bx = blockIdx.x;
-    extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
-    const int t = threadIdx.x, lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int c = lane & 15, g = lane >> 4;
-    const int64_t mwg = bx * 256;
-    const int r0 = blockIdx.y * 64;
-    const int64_t kk0 = (int64_t)blockIdx.z * kk_per_split;
-    const int64_t kk1 = kk0 + kk_per_split < kk_total ? kk0 + kk_per_split : kk_total;
-    const int nst = (int)((kk1 - kk0) / U);
-    const int64_t I0 = sd.dim[0];
-    const double* __restrict__ At0 = sd.fac[0];
-
-    // stage positions advance by U four-steps without divisions: (rest, step
-    // within the rest) of the next stage to request and of the stage to compute
-    int64_t rest_is = kk0 / nsteps_i, st_is = kk0 - rest_is * nsteps_i;
-    int64_t rest_c = rest_is;
-    int64_t st_c = st_is;
-    // requests the next stage into slot q % TKR_NS: wave w loads T columns 2w, 2w+1
-    // (two 1 KB halves each) and At0 rows 2w, 2w+1 of the stage
-    auto issue = [&](int q) {
-        const int64_t rest = rest_is;
-        const int64_t i0 = st_is * 4;
-        st_is += U;
-        if (st_is >= nsteps_i) { st_is -= nsteps_i; ++rest_is; }
-        unsigned char* slot = ring + (q % TKR_NS) * TKR_SLOT;
-#pragma unroll
-        for (int e2 = 0; e2 < 2; ++e2) {
-            const int e = 2 * wave + e2;
-            const double* col = T + (I0 * rest + i0 + e) * ML + mwg + 2 * lane;
-            lds_dma16(col, slot + e * TKR_CST);
-            lds_dma16(col + 128, slot + e * TKR_CST + 1024);
-        }
-        const int row = 2 * wave + (lane >> 5);
-        lds_dma16(At0 + (i0 + row) * Rp + r0 + 2 * (lane & 31), slot + TKR_TBYTES + 2 * wave * 512);
-    };
-
-    d4 acc[RB][MB];
-#pragma unroll
-    for (int a = 0; a < RB; ++a)
-#pragma unroll
-        for (int b = 0; b < MB; ++b) acc[a][b] = (d4){0.0, 0.0, 0.0, 0.0};
-
-    // the operands of the next stage to read (stages are read in order): T rows
-    // 2c, 2c+1, 32+2c, 33+2c of the wave's 64 (eight lanes read 128 contiguous
-    // bytes per instruction) and the At0 rows times the rest weights, which are
-    // reloaded when the rest changes
-    int64_t cur_rest = -1;
-    double w[RB];
-#pragma unroll
-    for (int a = 0; a < RB; ++a) w[a] = 0.0;
-    auto read_stage = [&](int q, double (&ta)[U][MB], double (&ka)[U][RB]) {
-        const int64_t rest = rest_c;
-        st_c += U;
-        if (st_c >= nsteps_i) { st_c -= nsteps_i; ++rest_c; }
-        if (rest != cur_rest) {
-            cur_rest = rest;
-#pragma unroll
-            for (int a = 0; a < RB; ++a) w[a] = rest_weight(sd, rest, r0 + 16 * a + c, Rp, true);
-        }
-        const unsigned char* slot = ring + (q % TKR_NS) * TKR_SLOT;
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const unsigned char* tp = slot + (4 * u + g) * TKR_CST + (wave * 64 + 2 * c) * 8;
-            const dv2 x0 = *reinterpret_cast<const dv2*>(tp);
-            const dv2 x1 = *reinterpret_cast<const dv2*>(tp + 256);
-            ta[u][0] = x0.x; ta[u][1] = x0.y; ta[u][2] = x1.x; ta[u][3] = x1.y;
-            const double* kp = reinterpret_cast<const double*>(slot + TKR_TBYTES) + (4 * u + g) * 64 + c;
-#pragma unroll
-            for (int a = 0; a < RB; ++a) ka[u][a] = kp[16 * a] * w[a];
-        }
-    };
-    auto mfmas = [&](const double (&ta)[U][MB], const double (&ka)[U][RB]) {
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int a = 0; a < RB; ++a)
-#pragma unroll
-                for (int b = 0; b < MB; ++b) acc[a][b] = mfma_f64(ka[u][a], ta[u][b], acc[a][b]);
-    };
-    // this wave's loads of stage q have landed once at most those of the stages
-    // requested after it (up to `last`, five loads each) are pending; then the barrier
-    auto arrive = [&](int q, int last) {
-        if (last - q >= 3) TKR_WAIT(15);
-        else if (last - q == 2) TKR_WAIT(10);
-        else if (last - q == 1) TKR_WAIT(5);
-        else TKR_WAIT(0);
-        __asm__ volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        __asm__ volatile("" ::: "memory");
-    };
-    for (int q = 0; q < TKR_NS - 1 && q < nst; ++q) issue(q);
-    for (int q = 0; q < nst; ++q) {
-        // stages up to q + TKR_NS - 2 are requested by now
-        arrive(q, q + TKR_NS - 2 < nst - 1 ? q + TKR_NS - 2 : nst - 1);
-        if (q + TKR_NS - 1 < nst) issue(q + TKR_NS - 1);
-        double ta[U][MB], ka[U][RB];
-        read_stage(q, ta, ka);
-        mfmas(ta, ka);
-    }
-
-    double* o = out + (int64_t)blockIdx.z * split_stride;
-    const int64_t mrow = mwg + wave * 64 + 2 * c;
-#pragma unroll
-    for (int a = 0; a < RB; ++a)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int r = r0 + 16 * a + g + 4 * v;
-            if (r >= R) continue;
-#pragma unroll
-            for (int b = 0; b < MB; ++b) o[mrow + 32 * (b >> 1) + (b & 1) + out_ld * r] = acc[a][b][v];
-        }
-}
-
-// ---------------------------------------------------------------- TR GEMM
-// out(mR, r) = sum over mL = i + I0*rest of T(mL, mR) KRP(mL, r),
-// KRP(mL, r) = A0[i + I0*r] * prod_{q>=1} Aq[digit_q + Iq*r] (column-major factors).
-// Workgroup tile: 16*MB output rows x 16*RB ranks; the 4 waves share the tile and
-// split the workgroup's reduction range [kk0, kk1) (in groups of 4*S indices of
-// the first left mode) into four consecutive parts, then add their accumulators
-// through LDS.  Over a group, lane (g, c) owns the run i0 + S*g .. + S-1
-// (contiguous in T and in A0).
-template <typename TT, int RB, int MB, int S, bool FAST>
-__global__ __launch_bounds__(256, 2) void k_tr(const TT* __restrict__ T, int64_t ML, int64_t MR,
-                                               Side sd, int64_t ngroups_i, int64_t kk_per_split,
-                                               int64_t kk_total, int Rp, int R,
-                                               double* __restrict__ out, int64_t split_stride,
-                                               const DevCheck* __restrict__ chk) {
-    if (chk->done) return;
-    __shared__ d4 red[2][RB * MB][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int c = lane & 15, g = lane >> 4;
-    const int64_t n0 = (int64_t)blockIdx.x * (16 * MB);
-    const int r0 = blockIdx.y * (16 * RB);
-    const int64_t kb0 = (int64_t)blockIdx.z * kk_per_split;
-    const int64_t kb1 = kb0 + kk_per_split < kk_total ? kb0 + kk_per_split : kk_total;
-    const int64_t quarter = (kb1 - kb0 + 3) / 4;
-    const int64_t kk0 = kb0 + wave * quarter < kb1 ? kb0 + wave * quarter : kb1;
-    const int64_t kk1 = kk0 + quarter < kb1 ? kk0 + quarter : kb1;
-    const int64_t I0 = sd.dim[0];
-    const double* __restrict__ A0 = sd.fac[0];
-
-    int64_t col[MB];
-    bool colok[MB];
-#pragma unroll
-    for (int b = 0; b < MB; ++b) {
-        col[b] = n0 + 16 * b + c;
-        colok[b] = FAST || col[b] < MR;
-        if (!colok[b]) col[b] = 0;
-    }
-    const double* __restrict__ Arow[RB];
-#pragma unroll
-    for (int a = 0; a < RB; ++a) Arow[a] = A0 + I0 * (int64_t)(r0 + 16 * a + c);
-
-    d4 acc[RB][MB];
-#pragma unroll
-    for (int a = 0; a < RB; ++a)
-#pragma unroll
-        for (int b = 0; b < MB; ++b) acc[a][b] = (d4){0.0, 0.0, 0.0, 0.0};
-
-    int64_t kk = kk0;
-    while (kk < kk1) {
-        const int64_t rest = kk / ngroups_i;
-        const int64_t s_lo = kk - rest * ngroups_i;
-        int64_t s_hi = ngroups_i;
-        if ((rest + 1) * ngroups_i > kk1) s_hi = kk1 - rest * ngroups_i;
-        double w[RB];
-#pragma unroll
-        for (int a = 0; a < RB; ++a) w[a] = rest_weight(sd, rest, r0 + 16 * a + c, Rp, false);
-        const TT* __restrict__ Tr = T + I0 * rest;
-
-        double tb[2][S][MB], ka[2][S][RB];
-        auto compute = [&](int buf) {
-#pragma unroll
-            for (int s = 0; s < S; ++s)
-#pragma unroll
-                for (int a = 0; a < RB; ++a)
-#pragma unroll
-                    for (int b = 0; b < MB; ++b)
-                        acc[a][b] = mfma_f64(ka[buf][s][a], tb[buf][s][b], acc[a][b]);
-        };
-        auto loads = [&](int buf, int64_t grp) {
-            const int64_t ib = grp * (4 * S) + S * g;
-            if constexpr (FAST) {
-#pragma unroll
-                for (int b = 0; b < MB; ++b) {
-                    double run[S];
-                    ld_run<TT, S>(Tr + ib + ML * col[b], run);
-#pragma unroll
-                    for (int s = 0; s < S; ++s) tb[buf][s][b] = run[s];
-                }
-#pragma unroll
-                for (int s = 0; s < S; ++s)
-#pragma unroll
-                    for (int a = 0; a < RB; ++a) ka[buf][s][a] = Arow[a][ib + s] * w[a];
-            } else {
-#pragma unroll
-                for (int s = 0; s < S; ++s) {
-                    const int64_t i = ib + s;
-                    const bool ok = i < I0;
-#pragma unroll
-                    for (int b = 0; b < MB; ++b)
-                        tb[buf][s][b] = (ok && colok[b]) ? ld1(Tr + i + ML * col[b]) : 0.0;
-#pragma unroll
-                    for (int a = 0; a < RB; ++a) ka[buf][s][a] = ok ? Arow[a][i] * w[a] : 0.0;
-                }
-            }
-        };
-        int64_t gp = s_lo;
-        loads(0, gp);
-        while (true) {
-            const bool more1 = gp + 1 < s_hi;
-            if (more1) loads(1, gp + 1);
-            compute(0);
-            gp += 1;
-            if (!more1) break;
-            const bool more0 = gp + 1 < s_hi;
-            if (more0) loads(0, gp + 1);
-            compute(1);
-            gp += 1;
-            if (!more0) break;
-        }
-        kk = rest * ngroups_i + s_hi;
-    }
-
-    // combine the four waves' partial sums: (2,3) -> (0,1), then 1 -> 0
-    if (wave >= 2) {
-#pragma unroll
-        for (int a = 0; a < RB; ++a)
-#pragma unroll
-            for (int b = 0; b < MB; ++b) red[wave - 2][a * MB + b][lane] = acc[a][b];
-    }
-    __syncthreads();
-    if (wave < 2) {
-#pragma unroll
-        for (int a = 0; a < RB; ++a)
-#pragma unroll
-            for (int b = 0; b < MB; ++b) acc[a][b] += red[wave][a * MB + b][lane];
-    }
-    __syncthreads();
-    if (wave == 1) {
-#pragma unroll
-        for (int a = 0; a < RB; ++a)
-#pragma unroll
-            for (int b = 0; b < MB; ++b) red[0][a * MB + b][lane] = acc[a][b];
-    }
-    __syncthreads();
-    if (wave != 0) return;
-#pragma unroll
-    for (int a = 0; a < RB; ++a)
-#pragma unroll
-        for (int b = 0; b < MB; ++b) acc[a][b] += red[0][a * MB + b][lane];
-
-    double* o = out + (int64_t)blockIdx.z * split_stride;
-#pragma unroll
-    for (int a = 0; a < RB; ++a)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int r = r0 + 16 * a + g + 4 * v;
-            if (r >= R) continue;
-#pragma unroll
-            for (int b = 0; b < MB; ++b)
-                if (colok[b]) o[col[b] + MR * r] = acc[a][b][v];
-        }
-}
+#define VM_WAIT(n) __builtin_amdgcn_s_waitcnt(0x0000 | ((n) & 0xf) | (0x7 << 4) | (0x0 << 8))
 
 // ------------------------------------------------- reduced-precision GEMMs
 // The same two GEMMs with FP32 arithmetic: either FP32 MFMA (v_mfma_f32_16x16x4f32)
@@ -1003,8 +579,8 @@ __global__ __launch_bounds__(512, 1) void k_lp_ring(const float* __restrict__ T,
     for (int q = 0; q < LPR_NS - 1 && q < nst; ++q) issue(q);
     for (int q = 0; q < nst; ++q) {
         // this wave's loads of stage q are done once at most the 6 of stage q+1 pend
-        if (q + 1 < nst) TKR_WAIT(6);
-        else TKR_WAIT(0);
+        if (q + 1 < nst) VM_WAIT(6);
+        else VM_WAIT(0);
         __asm__ volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         __asm__ volatile("" ::: "memory");
@@ -1136,7 +712,7 @@ __device__ __forceinline__ double w_before(const Side& sd, int pos, int64_t a, i
     return w;
 }
 
-// A == 1 (the mode is the side's fastest): thread per (i, r), split over b.
+// The side's fastest mode: thread per (i, r), split over b.
 __global__ __launch_bounds__(256) void k_ttv_lead(const double* __restrict__ P, int64_t MS,
                                                   int64_t In, int R, Side sd, int pos, int64_t B,
                                                   int64_t b_per_split, double* __restrict__ out,
@@ -1172,7 +748,7 @@ __global__ __launch_bounds__(256) void k_ttv_lead(const double* __restrict__ P, 
     out[(int64_t)blockIdx.y * split_stride + i + In * r] = sum;
 }
 
-// A > 1: one wave per JW consecutive i of one r; lanes stride over a (contiguous in
+// The other modes: one wave per JW consecutive i of one r; lanes stride over a (contiguous in
 // P), with the JW rows' loads in flight together.  Each output keeps the order of
 // its sum for any JW (per lane over a, then over b, then the wave reduction).
 template <int JW>
@@ -1292,9 +868,26 @@ __global__ void k_sum_small(const double* __restrict__ part, int n, double* __re
 }
 
 // ----------------------------------------------------------------- launchers
+// A side's Khatri-Rao product (K rows) is formed whole when writing and reading it costs at
+// most 1/16 of the tensor's bytes: the GEMM then has one operand load per rank block and
+// step instead of two.
+bool krp64_whole(const itcpd_plan* p, int64_t K) {
+    return (double)K * (double)p->Rp * 8.0 * 16.0 <= (double)p->ML * (double)p->MR * (double)p->elt_bytes;
+}
+int64_t krp64_elems(const itcpd_plan* p) {
+    int64_t rows = 0;
+    for (int left = 0; left < 2; ++left) {   // the left GEMM reduces over the right side
+        const int nm = left ? p->N - p->s : p->s;
+        const int64_t K = left ? p->MR : p->ML, d0 = left ? p->dims[p->s] : p->dims[0];
+        if (nm > 1 && krp64_whole(p, K)) rows = std::max(rows, K);
+        else if (nm > 2) rows = std::max(rows, K / d0);
+    }
+    return rows * p->Rp;
+}
+
 namespace {
 
-// ------------------------------------------------- TR GEMM, LDS ring form
+// ------------------------------------------- right GEMM, LDS ring form
 // out(mR, r) = sum_{mL} T(mL, mR) KRP(mL, r) for a left side of one or two modes,
 // mL = i + I0 rest, KRP(mL, r) = A0(i, r) w(rest, r) with w = 1 (one mode) or
 // At1(rest, r) (two modes).  FP64 T, 64-column x 64-rank tiles.  A stage is SI
@@ -1321,12 +914,12 @@ struct TrrGeom {
 // s_waitcnt vmcnt <= n (0 <= n < 16), lgkmcnt = 0
 __device__ __forceinline__ void wait_vm(int n) {
     switch (n) {
-        case 0: TKR_WAIT(0); break;   case 1: TKR_WAIT(1); break;   case 2: TKR_WAIT(2); break;
-        case 3: TKR_WAIT(3); break;   case 4: TKR_WAIT(4); break;   case 5: TKR_WAIT(5); break;
-        case 6: TKR_WAIT(6); break;   case 7: TKR_WAIT(7); break;   case 8: TKR_WAIT(8); break;
-        case 9: TKR_WAIT(9); break;   case 10: TKR_WAIT(10); break; case 11: TKR_WAIT(11); break;
-        case 12: TKR_WAIT(12); break; case 13: TKR_WAIT(13); break; case 14: TKR_WAIT(14); break;
-        default: TKR_WAIT(15); break;
+        case 0: VM_WAIT(0); break;   case 1: VM_WAIT(1); break;   case 2: VM_WAIT(2); break;
+        case 3: VM_WAIT(3); break;   case 4: VM_WAIT(4); break;   case 5: VM_WAIT(5); break;
+        case 6: VM_WAIT(6); break;   case 7: VM_WAIT(7); break;   case 8: VM_WAIT(8); break;
+        case 9: VM_WAIT(9); break;   case 10: VM_WAIT(10); break; case 11: VM_WAIT(11); break;
+        case 12: VM_WAIT(12); break; case 13: VM_WAIT(13); break; case 14: VM_WAIT(14); break;
+        default: VM_WAIT(15); break;
     }
 }
 
@@ -1468,9 +1061,6 @@ constexpr int TRR_NW = 4, TRR_NS = 2, TRR_SI = 16;
 constexpr int TRR_LDS = TRR_NS * TrrGeom<TRR_SI>::SLOT;
 constexpr int TRR_WG_PER_CU = (160 * 1024) / TRR_LDS < 4 ? (160 * 1024) / TRR_LDS : 4;
 
-// contiguous run per lane in the TR kernel (reduction indices per 4-lane group = 4 * TR_RUN)
-constexpr int TR_RUN = 2;
-
 struct Timed {
     itcpd_plan* p;
     hipEvent_t e1 = nullptr;
@@ -1537,75 +1127,175 @@ FactorJob factor_job_for(itcpd_plan* p, int mode) {
     return fj;
 }
 
-// The LDS ring form of the left GEMM applies: FP64 T, 256-row tiles, 64-rank
-// blocks, stages of 8 indices of the first right mode.
-bool tk_ring_ok(const itcpd_plan* p, const Side& sd) {
-    return p->elt_bytes == 8 && p->RB >= 4 && p->ML % 256 == 0 && p->Rp % 64 == 0 && sd.dim[0] % 8 == 0;
+// ---- the direct FP64 GEMMs (gemm64.h): configuration and launch
+// Rank blocks of 16 per wave: the fewest blocks in all (padding included; within the Rp
+// columns of the rank-fastest factors), weighed against the passes over T.
+int gemm64_rb(int64_t R, int64_t Rp) {
+    const int64_t nb = cdiv(R, 16);
+    int best = 1;
+    int64_t bestc = INT64_MAX;
+    for (int rb = 5; rb >= 1; --rb) {
+        const int64_t ny = cdiv(nb, rb), c = 2 * rb * ny + ny;
+        if (16 * rb * ny <= Rp && c < bestc) { bestc = c; best = rb; }
+    }
+    return best;
 }
 
-template <typename TT, int RB, int MB>
-int run_tk(itcpd_plan* p, const Side& sd, double* out, int64_t out_ld, int64_t nz,
-           int64_t kk_per, int64_t kk_total, int64_t nsteps_i, int64_t split_stride) {
-    constexpr int U = 2;
-    if (sizeof(TT) == 8 && tk_ring_ok(p, sd) && kk_per % 2 == 0) {
-        dim3 grid((unsigned)(p->ML / 256), (unsigned)(p->Rp / 64), (unsigned)nz);
-        hipLaunchKernelGGL(k_tk_ring, grid, dim3(256), (size_t)TKR_LDS, p->stream, (const double*)p->T, p->ML,
-                           sd, nsteps_i, kk_per, kk_total, (int)p->Rp, (int)p->R, out, out_ld, split_stride,
-                           p->chk);
-        ITCPD_HIP(hipGetLastError());
+struct Gemm64Cfg {
+    int MB, KW;
+    int64_t per, nz;    // reduction units (4-steps / 16-index stages) per split, splits
+};
+// Tiles of 16 MB outputs.  With at least three workgroups of four such tiles per CU every
+// wave takes its own tile and no reduction is split (KW = 1).  Otherwise the four waves of a
+// workgroup split one tile's reduction, and so do nz workgroups, for the fewest rounds of
+// two workgroups per CU per unit of work plus a charge for the partials' traffic; a wave
+// keeps at least `min_units`.  16-output tiles are taken when the large ones cannot give
+// every CU a workgroup, or when a slab has fewer rows than one (the large left tile is moved
+// back to end at the slab's last row).  Measured, us (KW = 1 / KW = 4): 301 x (257) x 199
+// rank 37, 398 workgroups, 60 / 42; 512 x (512) x 512 rank 64, 1024 workgroups, 338 / 347.
+Gemm64Cfg gemm64_cfg(const itcpd_plan* p, int64_t M, int64_t slabs, int64_t units, int64_t min_units, int ny,
+                     int big) {
+    Gemm64Cfg c{};
+    const int64_t slots = 2 * (int64_t)p->num_cu;
+    const int64_t out_elems = M * slabs * p->R;
+    const bool fits = M >= 16 * big;
+    if (fits && cdiv(cdiv(M, 16 * big), 4) * slabs * ny >= 3 * (int64_t)p->num_cu) return Gemm64Cfg{big, 1, units, 1};
+    const double tbytes = (double)p->ML * (double)p->MR * (double)p->elt_bytes;
+    for (int mb : {big, 1}) {
+        if (mb == big && !fits) continue;
+        const int64_t base = cdiv(M, 16 * mb) * slabs * ny;
+        double best = 1e300;
+        int64_t nz = 1;
+        for (int64_t z = 1; z <= 512; ++z) {
+            if (z > 1 && (units < 4 * min_units * z || (size_t)(z * out_elems) > p->parts_elems)) break;
+            const double cost = (double)cdiv(base * z, slots) * (double)slots / (double)(base * z) +
+                                (z > 1 ? 16.0 * (double)(z * out_elems) / tbytes : 0.0);
+            if (cost < best - 1e-9) { best = cost; nz = z; }
+        }
+        c = Gemm64Cfg{mb, 4, cdiv(units, nz), nz};
+        c.nz = cdiv(units, c.per);
+        if (base * c.nz >= p->num_cu) break;
+    }
+    return c;
+}
+
+// The rank-fastest factors of a side as the kernels' Khatri-Rao operand; *nm = 1 or 2.
+int krp64_of(itcpd_plan* p, const Side& sd, int64_t K, Krp64* kp, int* nm) {
+    kp->At0 = sd.fac[0];
+    kp->W = sd.fac[0];
+    kp->I0 = sd.dim[0];
+    kp->Rp = (int)p->Rp;
+    *nm = sd.nm < 2 ? 1 : 2;
+    if (sd.nm < 2) return ITCPD_OK;
+    const bool whole = krp64_whole(p, K);
+    if (!whole && sd.nm == 2) {
+        kp->W = sd.fac[1];
         return ITCPD_OK;
     }
-    dim3 grid((unsigned)cdiv(p->ML, 64 * MB), (unsigned)(p->Rp / (16 * RB)), (unsigned)nz);
-    const bool fast = (p->ML % (64 * MB) == 0) && (sd.dim[0] % 4 == 0) && (p->ML % 2 == 0);
-    if (fast)
-        hipLaunchKernelGGL((k_tk<TT, RB, MB, U, true>), grid, dim3(256), 0, p->stream,
-                           (const TT*)p->T, p->ML, sd, nsteps_i, kk_per, kk_total, (int)p->Rp,
-                           (int)p->R, out, out_ld, split_stride, p->chk);
-    else
-        hipLaunchKernelGGL((k_tk<TT, RB, MB, U, false>), grid, dim3(256), 0, p->stream,
-                           (const TT*)p->T, p->ML, sd, nsteps_i, kk_per, kk_total, (int)p->Rp,
-                           (int)p->R, out, out_ld, split_stride, p->chk);
+    const int64_t n = whole ? K : K / sd.dim[0];
+    hipLaunchKernelGGL(k_krp64, dim3((unsigned)cdiv(n * p->Rp, 256)), dim3(256), 0, p->stream, sd, whole ? 0 : 1, n,
+                       (int)p->Rp, p->Wrest, p->chk);
     ITCPD_HIP(hipGetLastError());
+    kp->W = p->Wrest;
+    if (whole) {
+        kp->At0 = p->Wrest;
+        kp->I0 = K;
+        *nm = 1;
+    }
     return ITCPD_OK;
 }
 
-template <typename TT, int RB, int MB>
-int run_tr(itcpd_plan* p, const Side& sd, double* out, int64_t nz, int64_t kk_per,
-           int64_t kk_total, int64_t ngroups, int64_t split_stride) {
-    constexpr int S = TR_RUN;
-    dim3 grid((unsigned)cdiv(p->MR, 16 * MB), (unsigned)(p->Rp / (16 * RB)), (unsigned)nz);
-    const bool fast = (p->MR % (16 * MB) == 0) && (sd.dim[0] % (4 * S) == 0) && (p->ML % 2 == 0);
-    if (fast)
-        hipLaunchKernelGGL((k_tr<TT, RB, MB, S, true>), grid, dim3(256), 0, p->stream,
-                           (const TT*)p->T, p->ML, p->MR, sd, ngroups, kk_per, kk_total,
-                           (int)p->Rp, (int)p->R, out, split_stride, p->chk);
+// One direct GEMM: outs x R outputs (a batch of slabs of M rows for the left form),
+// reduction length K over the operand kp.
+struct Gemm64 {
+    bool left;
+    int64_t M, slabs, K;   // outputs per slab, slabs (1 for the right form)
+    Krp64 kp;
+    int nm, rb, ny;
+    Gemm64Cfg c;
+    double* out;
+};
+
+template <typename TT, int RB, int MB, int U, int KW, int VEC, int OCC>
+void launch_left64(itcpd_plan* p, const Gemm64& q) {
+    const int64_t nt = cdiv(q.M, 16 * MB);
+    const dim3 grid((unsigned)(KW == 1 ? cdiv(nt, 4) : nt), (unsigned)(q.ny * q.slabs), (unsigned)q.c.nz);
+    const int64_t ld = q.M * q.slabs;
+    if (q.nm == 1)
+        hipLaunchKernelGGL((k_left<TT, 1, RB, MB, U, KW, VEC, OCC>), grid, dim3(256), 0, p->stream,
+                           (const TT*)p->T, q.M, q.K, q.kp, q.c.per, q.ny, (int)p->R, q.out, ld, ld * p->R, p->chk);
     else
-        hipLaunchKernelGGL((k_tr<TT, RB, MB, S, false>), grid, dim3(256), 0, p->stream,
-                           (const TT*)p->T, p->ML, p->MR, sd, ngroups, kk_per, kk_total,
-                           (int)p->Rp, (int)p->R, out, split_stride, p->chk);
-    ITCPD_HIP(hipGetLastError());
-    return ITCPD_OK;
+        hipLaunchKernelGGL((k_left<TT, 2, RB, MB, U, KW, VEC, 2>), grid, dim3(256), 0, p->stream,
+                           (const TT*)p->T, q.M, q.K, q.kp, q.c.per, q.ny, (int)p->R, q.out, ld, ld * p->R, p->chk);
+}
+template <typename TT, int RB, int MB, int KW>
+void launch_right64(itcpd_plan* p, const Gemm64& q) {
+    const int64_t nt = cdiv(q.M, 16 * MB);
+    const dim3 grid((unsigned)(KW == 1 ? cdiv(nt, 4) : nt), (unsigned)q.ny, (unsigned)q.c.nz);
+    const int64_t elems = q.M * p->R;
+    if (q.nm == 1)
+        hipLaunchKernelGGL((k_right<TT, 0, RB, MB, KW, 4, 2>), grid, dim3(256), 0, p->stream, (const TT*)p->T, q.M,
+                           q.K, q.kp, q.c.per, (int)p->R, q.out, elems, p->chk);
+    else if (q.kp.I0 % 16 == 0)
+        hipLaunchKernelGGL((k_right<TT, 1, RB, MB, KW, 4, 2>), grid, dim3(256), 0, p->stream, (const TT*)p->T, q.M,
+                           q.K, q.kp, q.c.per, (int)p->R, q.out, elems, p->chk);
+    else
+        hipLaunchKernelGGL((k_right<TT, 2, RB, MB, KW, 4, 2>), grid, dim3(256), 0, p->stream, (const TT*)p->T, q.M,
+                           q.K, q.kp, q.c.per, (int)p->R, q.out, elems, p->chk);
 }
 
-template <typename TT>
-int dispatch_tk(itcpd_plan* p, const Side& sd, double* out, int64_t out_ld, int64_t nz,
-                int64_t kk_per, int64_t kk_total, int64_t nsteps_i, int64_t split_stride) {
-    switch (p->RB) {
-        case 1: return run_tk<TT, 1, 8>(p, sd, out, out_ld, nz, kk_per, kk_total, nsteps_i, split_stride);
-        case 2: return run_tk<TT, 2, 8>(p, sd, out, out_ld, nz, kk_per, kk_total, nsteps_i, split_stride);
-        case 4: return run_tk<TT, 4, 4>(p, sd, out, out_ld, nz, kk_per, kk_total, nsteps_i, split_stride);
-        default: return run_tk<TT, 8, 2>(p, sd, out, out_ld, nz, kk_per, kk_total, nsteps_i, split_stride);
-    }
+// Tile heights (16-output tiles per wave) by rank blocks: what the accumulators and two
+// stages of operands leave of the registers of two (RB >= 3) or four waves per SIMD.
+constexpr int left64_big(int rb) { return rb <= 4 ? 4 : 2; }
+constexpr int right64_big(int rb) { return rb <= 2 ? 4 : 2; }
+
+template <typename TT, int RB>
+void run_left64(itcpd_plan* p, const Gemm64& q) {
+    constexpr int B = left64_big(RB), OCC = RB <= 2 ? 4 : 2;
+    if (q.c.KW == 1) launch_left64<TT, RB, B, 2, 1, 2, OCC>(p, q);
+    else if (q.c.MB == B) launch_left64<TT, RB, B, 2, 4, 2, OCC>(p, q);
+    else launch_left64<TT, RB, 1, 4, 4, 1, 2>(p, q);
+}
+template <typename TT, int RB>
+void run_right64(itcpd_plan* p, const Gemm64& q) {
+    constexpr int B = right64_big(RB);
+    if (q.c.KW == 1) launch_right64<TT, RB, B, 1>(p, q);
+    else if (q.c.MB == B) launch_right64<TT, RB, B, 4>(p, q);
+    else launch_right64<TT, RB, 1, 4>(p, q);
 }
 template <typename TT>
-int dispatch_tr(itcpd_plan* p, const Side& sd, double* out, int64_t nz, int64_t kk_per,
-                int64_t kk_total, int64_t ngroups, int64_t split_stride) {
-    switch (p->RB) {
-        case 1: return run_tr<TT, 1, 8>(p, sd, out, nz, kk_per, kk_total, ngroups, split_stride);
-        case 2: return run_tr<TT, 2, 8>(p, sd, out, nz, kk_per, kk_total, ngroups, split_stride);
-        case 4: return run_tr<TT, 4, 4>(p, sd, out, nz, kk_per, kk_total, ngroups, split_stride);
-        default: return run_tr<TT, 8, 2>(p, sd, out, nz, kk_per, kk_total, ngroups, split_stride);
+void dispatch_gemm64(itcpd_plan* p, const Gemm64& q) {
+    if (q.left) {
+        switch (q.rb) {
+            case 1: return run_left64<TT, 1>(p, q);
+            case 2: return run_left64<TT, 2>(p, q);
+            case 3: return run_left64<TT, 3>(p, q);
+            case 4: return run_left64<TT, 4>(p, q);
+            default: return run_left64<TT, 5>(p, q);
+        }
     }
+    switch (q.rb) {
+        case 1: return run_right64<TT, 1>(p, q);
+        case 2: return run_right64<TT, 2>(p, q);
+        case 3: return run_right64<TT, 3>(p, q);
+        case 4: return run_right64<TT, 4>(p, q);
+        default: return run_right64<TT, 5>(p, q);
+    }
+}
+// Configures and launches q (M, slabs, K, kp, nm set): into dst, or into the split partials
+// (q.c.nz > 1).
+int run_gemm64(itcpd_plan* p, Gemm64& q, double* dst) {
+    q.rb = gemm64_rb(p->R, p->Rp);
+    q.ny = (int)cdiv(cdiv(p->R, 16), q.rb);
+    q.c = q.left ? gemm64_cfg(p, q.M, q.slabs, cdiv(q.K, 4), 4, q.ny, left64_big(q.rb))
+                 : gemm64_cfg(p, q.M, 1, cdiv(q.K, 16), 2, q.ny, right64_big(q.rb));
+    q.out = q.c.nz > 1 ? p->parts : dst;
+    Timed tm(p, q.left ? 0 : 1, 2.0 * (double)p->ML * (double)p->MR * (double)p->R,
+             (double)p->ML * (double)p->MR * p->elt_bytes);
+    if (p->elt_bytes == 8) dispatch_gemm64<double>(p, q);
+    else dispatch_gemm64<float>(p, q);
+    ITCPD_HIP(hipGetLastError());
+    return ITCPD_OK;
 }
 
 template <typename TT, int RB, int MB, bool BF>
@@ -1673,8 +1363,6 @@ int convert_factor(itcpd_plan* p, const double* A, int64_t n) {
     return ITCPD_OK;
 }
 
-int mb_of(int RB) { return RB <= 2 ? 8 : RB == 4 ? 4 : 2; }
-
 }  // namespace
 
 // Parts with at most this many partials are summed by the consumer (the solve).
@@ -1709,6 +1397,8 @@ int finish_parts(itcpd_plan* p, double* parts, int64_t nz, int64_t n, double* ds
 
 // Left GEMM: rows = left multi-index (ML), reduction = right side.  Produces PL
 // (s > 1) or the M of mode 0 (s == 1).
+static int launch_ttv(itcpd_plan* p, const double* P, int64_t MS, const Side& sd, int pos, MSrc* ms,
+                      int factor_mode);
 int launch_left_gemm_lp(itcpd_plan* p, MSrc* ms);
 int launch_right_gemm_lp(itcpd_plan* p, MSrc* ms);
 
@@ -1730,87 +1420,31 @@ int launch_right_gemm(itcpd_plan* p, MSrc* ms, int factor_mode) {
     return launch_factor(p, factor_mode);
 }
 
-// FP64 arithmetic on an FP32-stored tensor: the tensor is widened once into an FP64
-// copy (exact), and the FP64 GEMMs -- the LDS ring forms where the shape allows --
-// read that copy.  While a GEMM is launched the plan presents the copy as its tensor.
-// Without memory for the copy the GEMMs read the FP32 tensor (register-staged forms).
-__global__ __launch_bounds__(256) void k_widen(const float* __restrict__ src, int64_t n,
-                                               double* __restrict__ dst) {
-    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-    if (i + 4 <= n) {
-        const float4 v = *reinterpret_cast<const float4*>(src + i);
-        *reinterpret_cast<dv2*>(dst + i) = dv2{(double)v.x, (double)v.y};
-        *reinterpret_cast<dv2*>(dst + i + 2) = dv2{(double)v.z, (double)v.w};
-    } else {
-        for (int64_t k = i; k < n; ++k) dst[k] = (double)src[k];
-    }
+// The direct FP64 GEMM of a side (gemm64.h), any shape.
+static int launch_gemm64(itcpd_plan* p, MSrc* ms, bool left, int factor_mode) {
+    const Side sd = left ? make_side(p, p->s, p->N - p->s, /*rank_fast=*/true)
+                         : make_side(p, 0, p->s, /*rank_fast=*/true);
+    const int nout = left ? p->s : p->N - p->s;   // modes on the output side
+    Gemm64 q{};
+    q.left = left;
+    q.M = left ? p->ML : p->MR;
+    q.slabs = 1;
+    q.K = left ? p->MR : p->ML;
+    int rc;
+    if ((rc = krp64_of(p, sd, q.K, &q.kp, &q.nm))) return rc;
+    double* dst = nout > 1 ? (left ? p->PL : p->PR) : p->M;
+    if ((rc = run_gemm64(p, q, dst))) return rc;
+    return finish_parts(p, p->parts, q.c.nz, q.M * p->R, dst, ms, nout == 1, factor_mode);
 }
-
-struct WidenedTensor {
-    itcpd_plan* p;
-    const void* T0 = nullptr;
-    bool on = false;
-    explicit WidenedTensor(itcpd_plan* pp) : p(pp) {
-        if (p->elt_bytes != 4 || p->prec != ITCPD_FP64 || p->T64_failed) return;
-        const int64_t n = p->ML * p->MR;
-        if (!p->T64) {
-            if (hipMalloc((void**)&p->T64, (size_t)n * 8) != hipSuccess) {
-                (void)hipGetLastError();
-                p->T64 = nullptr;
-                p->T64_failed = true;
-                return;
-            }
-            hipLaunchKernelGGL(k_widen, dim3((unsigned)cdiv(cdiv(n, 4), 256)), dim3(256), 0, p->stream,
-                               (const float*)p->T, n, p->T64);
-        }
-        T0 = p->T;
-        p->T = p->T64;
-        p->elt_bytes = 8;
-        on = true;
-    }
-    ~WidenedTensor() {
-        if (!on) return;
-        p->T = T0;
-        p->elt_bytes = 4;
-    }
-};
 
 int launch_left_gemm_impl(itcpd_plan* p, MSrc* ms) {
     if (p->prec != ITCPD_FP64) return launch_left_gemm_lp(p, ms);
-    WidenedTensor wt(p);
-    const Side sd = make_side(p, p->s, p->N - p->s, /*rank_fast=*/true);
-    const int MB = mb_of(p->RB);
-    const int64_t nsteps_i = cdiv(sd.dim[0], 4);
-    const int64_t nrest = p->MR / sd.dim[0];
-    const int64_t kk_total = nsteps_i * nrest;
-    // workgroup tiles of one split: the ring form's 256 rows x 64 ranks, else 64 MB x 16 RB
-    const int64_t base = tk_ring_ok(p, sd) ? (p->ML / 256) * (p->Rp / 64)
-                                           : cdiv(p->ML, 64 * MB) * (p->Rp / (16 * p->RB));
-    int64_t nz = pick_split(base, kk_total, 1024, 16);
-    const int64_t out_elems = p->ML * p->R;
-    if (nz > 1 && (size_t)(nz * out_elems) > p->parts_elems) nz = (int64_t)(p->parts_elems / out_elems);
-    if (nz < 1) nz = 1;
-    int64_t kk_per = cdiv(kk_total, nz);
-    if (tk_ring_ok(p, sd)) kk_per += kk_per & 1;   // whole stages of two 4-steps
-    nz = cdiv(kk_total, kk_per);
-    double* dst = (p->s > 1) ? p->PL : p->M;
-    double* out = nz > 1 ? p->parts : dst;
-    int rc;
-    {
-        Timed tm(p, 0, 2.0 * (double)p->ML * (double)p->MR * (double)p->R,
-                 (double)p->ML * (double)p->MR * p->elt_bytes);
-        rc = (p->elt_bytes == 8)
-                 ? dispatch_tk<double>(p, sd, out, p->ML, nz, kk_per, kk_total, nsteps_i, out_elems)
-                 : dispatch_tk<float>(p, sd, out, p->ML, nz, kk_per, kk_total, nsteps_i, out_elems);
-    }
-    if (rc) return rc;
-    return finish_parts(p, p->parts, nz, out_elems, dst, ms, p->s == 1);
+    return launch_gemm64(p, ms, true, -1);
 }
 
 // Right GEMM: rows = right multi-index (MR), reduction = left side.  Produces PR
 // (N-s > 1) or the M of mode N-1 (N-s == 1).
 int launch_right_gemm_impl(itcpd_plan* p, MSrc* ms, int factor_mode) {
-    WidenedTensor wt(p);
     const Side sd = make_side(p, 0, p->s, /*rank_fast=*/false);
     if (p->s <= 2 && p->elt_bytes == 8 && sd.dim[0] % TRR_SI == 0 && p->MR % 64 == 0 && p->Rp % 64 == 0) {
         // left side of one or two modes: the LDS ring form (TRR_WG_PER_CU workgroups
@@ -1859,32 +1493,8 @@ int launch_right_gemm_impl(itcpd_plan* p, MSrc* ms, int factor_mode) {
         }
         return finish_parts(p, p->parts, nz, out_elems, dst, ms, consumer_sums, factor_mode, fj.on != 0);
     }
-    const int MB = mb_of(p->RB);
-    constexpr int S = TR_RUN;
-    const int64_t ngroups = cdiv(sd.dim[0], 4 * S);
-    const int64_t nrest = p->ML / sd.dim[0];
-    const int64_t kk_total = ngroups * nrest;
-    const int64_t base = cdiv(p->MR, 16 * MB) * (p->Rp / (16 * p->RB));
-    int64_t nz = pick_split(base, kk_total, 512, 32);
-    const int64_t out_elems = p->MR * p->R;
-    if (nz > 1 && (size_t)(nz * out_elems) > p->parts_elems) nz = (int64_t)(p->parts_elems / out_elems);
-    if (nz < 1) nz = 1;
-    const int64_t kk_per = cdiv(kk_total, nz);
-    nz = cdiv(kk_total, kk_per);
-    double* dst = (p->N - p->s > 1) ? p->PR : p->M;
-    double* out = nz > 1 ? p->parts : dst;
-    int rc;
-    {
-        Timed tm(p, 1, 2.0 * (double)p->ML * (double)p->MR * (double)p->R,
-                 (double)p->ML * (double)p->MR * p->elt_bytes);
-        rc = (p->elt_bytes == 8)
-                 ? dispatch_tr<double>(p, sd, out, nz, kk_per, kk_total, ngroups, out_elems)
-                 : dispatch_tr<float>(p, sd, out, nz, kk_per, kk_total, ngroups, out_elems);
-    }
-    if (rc) return rc;
-    return finish_parts(p, p->parts, nz, out_elems, dst, ms, p->N - p->s == 1, factor_mode);
+    return launch_gemm64(p, ms, false, factor_mode);
 }
-
 
 // The LDS ring form of a reduced-precision GEMM applies: FP32-stored T, 256-row
 // (left) / 256-column (right) tiles and 32-index stages of the reduction.
@@ -2015,17 +1625,19 @@ int launch_right_gemm_lp(itcpd_plan* p, MSrc* ms) {
     return finish_parts(p, p->parts, nz, out_elems, dst, ms, p->N - p->s == 1);
 }
 
-// M of `mode` from its side's partial (only for sides with more than one mode).
-// With factor_mode >= 0 that mode's factorisation runs in an extra workgroup of the
-// same launch when it can (R <= 64), else it is launched right after.
 int launch_side_ttv(itcpd_plan* p, int mode, MSrc* ms, int factor_mode) {
     const bool left = mode < p->s;
     const int first = left ? 0 : p->s;
-    const int nm = left ? p->s : p->N - p->s;
-    const Side sd = make_side(p, first, nm, /*rank_fast=*/false);
-    const double* P = left ? p->PL : p->PR;
-    const int64_t MS = left ? p->ML : p->MR;
-    const int pos = mode - first;
+    const Side sd = make_side(p, first, left ? p->s : p->N - p->s, /*rank_fast=*/false);
+    return launch_ttv(p, left ? p->PL : p->PR, left ? p->ML : p->MR, sd, mode - first, ms, factor_mode);
+}
+
+// M of the side's mode `pos` from the partial P (leading dimension MS) by a
+// Hadamard-reduce.  With factor_mode >= 0 that mode's factorisation runs in an extra
+// workgroup of the same launch when it can (R <= 64), else it is launched right after.
+static int launch_ttv(itcpd_plan* p, const double* P, int64_t MS, const Side& sd, int pos, MSrc* ms,
+                      int factor_mode) {
+    const int nm = sd.nm;
     int64_t A = 1, B = 1;
     for (int q = 0; q < pos; ++q) A *= sd.dim[q];
     for (int q = pos + 1; q < nm; ++q) B *= sd.dim[q];
@@ -2034,7 +1646,7 @@ int launch_side_ttv(itcpd_plan* p, int mode, MSrc* ms, int factor_mode) {
     const FactorJob fj = factor_job_for(p, factor_mode);
     const size_t lds = fj.on ? FACTOR64_LDS : 0;
     int rc = ITCPD_OK;
-    if (A == 1) {
+    if (pos == 0) {
         int64_t nz = 1;
         const int64_t blocks = cdiv(nout, 256);
         while (blocks * nz < 2048 && B / (nz * 2) >= 16 && (size_t)(nz * 2 * nout) <= p->parts_elems &&

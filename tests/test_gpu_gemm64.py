@@ -1,0 +1,59 @@
+"""The direct FP64 GEMMs at the sizes where their tiles, stages and splits end."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def unfold(T, n):
+    return np.moveaxis(T, n, 0).reshape(T.shape[n], -1)
+
+
+def krp(fac):
+    out = fac[0]
+    for f in fac[1:]:
+        out = (out[:, None, :] * f[None]).reshape(-1, f.shape[1])
+    return out
+
+
+# modes at and one off multiples of the 16-output tiles, 4- and 16-index steps; slabs smaller
+# than a tile; one-element modes; orders whose Khatri-Rao product is formed whole, by rest
+# weights and on the way; ranks around every block count
+SHAPES = [((64, 64, 64), 16), ((65, 63, 33), 17), ((63, 65, 31), 33), ((17, 15, 400), 48), ((400, 16, 3), 49),
+          ((3, 5, 2), 1), ((1, 40, 30), 4), ((40, 1, 30), 4), ((50, 60), 7), ((300, 7), 65), ((31, 29, 27), 80),
+          ((33, 20, 17), 81), ((40, 30, 20), 150), ((16, 15, 14, 13), 32), ((2, 3, 5, 7, 11), 9),
+          ((130, 3, 2, 2), 20), ((2, 2, 3, 130), 20), ((9, 8, 7, 6, 5), 64)]
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("dims,R", SHAPES)
+def test_mttkrp_within_rounding_of_its_sums(itcpd, dims, R, dt):
+    """Every entry within the rounding bound of a length-K FP64 dot product with N factors:
+    (K + N + 2) 2^-53 sum |T| |KRP| for each side of the comparison (the FP32 tensor is exact
+    in FP64)."""
+    rng = np.random.default_rng(7)
+    T = np.asfortranarray(rng.standard_normal(dims).astype(dt))
+    cp = itcpd.CPD([rng.standard_normal((d, R)) for d in dims], np.ones(R))
+    with itcpd.ALSPlan(T, R) as plan:
+        plan.set_cpd(cp)
+        for n in range(len(dims)):
+            K = krp([cp.factors[m] for m in range(len(dims)) if m != n])
+            U = unfold(T.astype(np.float64), n)
+            bound = 2 * (U.shape[1] + len(dims) + 2) * 2.0**-53 * (np.abs(U) @ np.abs(K))
+            assert (np.abs(plan.mttkrp(n) - U @ K) / bound).max() <= 1.0, n
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("dims,at", [((37, 21, 18), (36, 20, 17)), ((37, 21, 18), (0, 0, 0)), ((20, 70, 5), (19, 69, 4))])
+def test_non_finite_entries_stay_in_their_rows(itcpd, dims, at, value):
+    """Reads past the end take a valid element: one that is not finite reaches only the rows
+    of M that it belongs to."""
+    rng = np.random.default_rng(8)
+    T = np.asfortranarray(rng.standard_normal(dims))
+    T[at] = value
+    cp = itcpd.CPD([rng.standard_normal((d, 6)) for d in dims], np.ones(6))
+    with itcpd.ALSPlan(T, 6) as plan:
+        plan.set_cpd(cp)
+        for n in range(3):
+            bad = ~np.isfinite(plan.mttkrp(n)).all(axis=1)
+            assert np.array_equal(np.nonzero(bad)[0], [at[n]])
