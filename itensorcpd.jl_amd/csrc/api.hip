@@ -162,7 +162,34 @@ int alloc_factor_state(itcpd_plan* p) {
 // 0's too: its V_0 is final once the previous sweep ended), and that of the right
 // GEMM's own mode in one of the launch that sums the GEMM's split-K partials; the
 // others (R > 64) run as their own launch right after mode n-1's update.
-int sweep(itcpd_plan* p) {
+//
+// Order 3 with shared partials (tree3): update u (counted from the run's start) with u even
+// contracts T over the mode updated last, and that partial serves updates u and u + 1.  When
+// only one update is left for a partial (the last of an odd number of sweeps), M_2 comes
+// from the right GEMM, as in the plain tree.
+int sweep3(itcpd_plan* p, int64_t k, bool last) {
+    int rc;
+    MSrc ms{};
+    const bool rides = p->R <= 64 && !p->v_override;
+    if (!rides && (rc = launch_factor(p, 0))) return rc;
+    for (int n = 0; n < 3; ++n) {
+        const int64_t u = 3 * k + n;
+        if (u % 2 == 0 && n == 2 && last && p->s == 2) {
+            if ((rc = launch_right_gemm(p, &ms, rides ? n : -1))) return rc;
+        } else {
+            const int c = u % 2 == 0 ? (n + 2) % 3 : (n + 1) % 3;
+            if (u % 2 == 0 && (rc = launch_tree3_gemm(p, c))) return rc;
+            if ((rc = launch_tree3_ttv(p, n, c, &ms, rides ? n : -1))) return rc;
+        }
+        const int next = n + 1 < 3 && !rides ? n + 1 : -1;
+        if ((rc = launch_solve(p, n, ms.ptr, ms.nparts, ms.stride, true, n == 2, next))) return rc;
+    }
+    if (p->profiling && p->timer.ev.size() >= 64) return collect_timer(p, false);
+    return ITCPD_OK;
+}
+
+int sweep(itcpd_plan* p, int64_t k, bool last) {
+    if (p->tree3) return sweep3(p, k, last);
     int rc;
     const int N = p->N;
     MSrc ms{};
@@ -337,6 +364,7 @@ int itcpd_plan_destroy(itcpd_plan* p) {
     dfree(p->smp_ws);
     dfree(p->sk_ws);
     dfree(p->Wrest);
+    dfree(p->P3);
     dfree(p->smp_iws);
     dfree(p->xg_part);
     if (p->chk_host) (void)hipHostFree(p->chk_host);
@@ -462,6 +490,12 @@ int itcpd_run(itcpd_plan* p, itcpd_check* c, double* fit_trace) {
     c->sweeps_run = 0;
     c->converged = 0;
     if (nsweeps <= 0) return ITCPD_OK;
+    p->tree3 = nsweeps > 1 && tree3_pays(p);
+    if (p->tree3 && !p->P3 && hipMalloc((void**)&p->P3, (size_t)tree3_elems(p) * 8) != hipSuccess) {
+        (void)hipGetLastError();   // no memory for it: the plain tree
+        p->P3 = nullptr;
+        p->tree3 = false;
+    }
     if (nsweeps > p->trace_cap) {
         dfree(p->fit_trace);
         p->fit_trace = nullptr;
@@ -502,7 +536,7 @@ int itcpd_run(itcpd_plan* p, itcpd_check* c, double* fit_trace) {
     for (int64_t k = 0; k < nsweeps;) {
         const int64_t nb = std::min<int64_t>(batch, nsweeps - k);
         for (int64_t b = 0; b < nb; ++b)
-            if ((rc = sweep(p))) return rc;
+            if ((rc = sweep(p, k + b, k + b == nsweeps - 1))) return rc;
         k += nb;
         if (c->kind == ITCPD_CHECK_NONE || k >= nsweeps) continue;
         const int slot = (int)(polls_issued % ITCPD_POLL_SLOTS);

@@ -131,6 +131,8 @@ struct itcpd_plan {
     float* Af = nullptr;                       // FP32 copy of the KRP side's first factor (reduced precision)
     float* Kt = nullptr;                       // FP32-stored T, reduced precision: a side's KRP, rank-major
     double* Wrest = nullptr;                   // a side's Khatri-Rao product or rest weights (rank fastest)
+    double* P3 = nullptr;                      // order 3: the partial that serves two mode updates (tree3)
+    bool tree3 = false;                        // order 3: partials shared across sweeps
     double* PR = nullptr;                      // MR x Rp partial of the right side (if N-s > 1)
     double* parts = nullptr;                   // split-K partial buffer
     size_t parts_elems = 0;
@@ -194,6 +196,11 @@ int launch_left_gemm(itcpd_plan* p, MSrc* ms, int factor_mode = -1);
 int launch_right_gemm(itcpd_plan* p, MSrc* ms, int factor_mode = -1);
 // M of `mode` from PL / PR; with factor_mode >= 0 also that mode's factorisation
 int launch_side_ttv(itcpd_plan* p, int mode, MSrc* ms, int factor_mode = -1);
+// order 3 across sweeps: the partial of T contracted over mode c, and a mode's M from it
+bool tree3_pays(const itcpd_plan* p);
+int64_t tree3_elems(const itcpd_plan* p);
+int launch_tree3_gemm(itcpd_plan* p, int c);
+int launch_tree3_ttv(itcpd_plan* p, int mode, int c, MSrc* ms, int factor_mode);
 int64_t krp64_elems(const itcpd_plan* p);      // doubles of p->Wrest
 int mttkrp_mode(itcpd_plan* p, int mode);      // full M_mode into p->M from the current factors
 // out = the sum of ms's partials; factor_mode >= 0: that mode's factorisation too

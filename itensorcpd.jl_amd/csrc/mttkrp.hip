@@ -9,7 +9,8 @@
 // fastest).  The KRP operand is generated on the fly from the factors (gemm64.h).  A side
 // with one mode yields its M directly; a side with several modes gets each M_n
 // from its partial by a Hadamard-reduce against the side's other (current)
-// factors.  T is read twice per sweep.
+// factors.  T is read twice per sweep; at order 3 three times per two sweeps where the
+// partials are shared across sweeps (launch_tree3_gemm).
 #include "internal.h"
 #include "factor64.h"
 #include "gemm64.h"
@@ -1435,6 +1436,56 @@ static int launch_gemm64(itcpd_plan* p, MSrc* ms, bool left, int factor_mode) {
     double* dst = nout > 1 ? (left ? p->PL : p->PR) : p->M;
     if ((rc = run_gemm64(p, q, dst))) return rc;
     return finish_parts(p, p->parts, q.c.nz, q.M * p->R, dst, ms, nout == 1, factor_mode);
+}
+
+// ---- order 3, across sweeps: one contraction of T per two mode updates
+// P_c(a, b, r) = sum over mode c of T A_c gives M of both other modes by Hadamard-reduces,
+// and the updates cycle 0, 1, 2, 0, ..., so the partial formed for update u (contracting the
+// mode updated last) also serves update u + 1: 3 passes over T per two sweeps instead of 4.
+// Contracting mode 2 or mode 1 is a left GEMM (mode 1: a batch of K slabs), mode 0 a right
+// one, each against one factor.  The price is one and a half partials written and three read
+// per sweep instead of one and two: taken when half a pass over T (the tensor's read or
+// 2 n R flops, at the rates the GEMMs reach) costs more than that.  Per sweep, us: 512^3
+// rank 64 684 (755 with two passes); 301 x 257 x 199 rank 37 166 (206).
+bool tree3_pays(const itcpd_plan* p) {
+    if (p->N != 3 || p->prec != ITCPD_FP64) return false;
+    const double n = (double)p->ML * (double)p->MR;
+    const double pair = ((double)p->dims[0] * p->dims[1] + (double)p->dims[0] * p->dims[2] +
+                         (double)p->dims[1] * p->dims[2]) / 3.0;
+    const double gemm = std::max(n * p->elt_bytes / 5.2e12, 2.0 * n * 16.0 * (double)cdiv(p->R, 16) / 5.0e13);
+    // the batched left GEMM has one grid row per slab and rank block
+    if (p->dims[2] * cdiv(p->R, 16) > 65535) return false;
+    return 0.5 * gemm > 1.5 * 8.0 * pair * (double)p->R / 4.5e12;
+}
+int64_t tree3_elems(const itcpd_plan* p) {
+    return std::max(p->dims[0] * std::max(p->dims[1], p->dims[2]), p->dims[1] * p->dims[2]) * p->R;
+}
+int launch_tree3_gemm(itcpd_plan* p, int c) {
+    Gemm64 q{};
+    q.left = c != 0;
+    q.slabs = c == 1 ? p->dims[2] : 1;
+    q.M = c == 2 ? p->dims[0] * p->dims[1] : (c == 1 ? p->dims[0] : p->dims[1] * p->dims[2]);
+    q.K = p->dims[c];
+    q.kp = Krp64{p->At[c], p->At[c], p->dims[c], (int)p->Rp};
+    q.nm = 1;
+    int rc;
+    if ((rc = run_gemm64(p, q, p->P3))) return rc;
+    if (q.c.nz == 1) return ITCPD_OK;
+    const int64_t n = q.M * q.slabs * p->R;
+    return launch_sum_parts(p, MSrc{p->parts, (int)q.c.nz, n}, n, p->P3);
+}
+int launch_tree3_ttv(itcpd_plan* p, int mode, int c, MSrc* ms, int factor_mode) {
+    Side sd{};
+    sd.nm = 2;
+    int pos = 0;
+    for (int m = 0, q = 0; m < 3; ++m) {
+        if (m == c) continue;
+        if (m == mode) pos = q;
+        sd.dim[q] = p->dims[m];
+        sd.fac[q] = p->A[m];
+        ++q;
+    }
+    return launch_ttv(p, p->P3, sd.dim[0] * sd.dim[1], sd, pos, ms, factor_mode);
 }
 
 int launch_left_gemm_impl(itcpd_plan* p, MSrc* ms) {

@@ -1,6 +1,9 @@
-"""The direct FP64 GEMMs at the sizes where their tiles, stages and splits end."""
+"""The direct FP64 GEMMs and the order-3 sweeps that share partials, at the sizes where
+their tiles, stages and splits end."""
 import numpy as np
 import pytest
+
+import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +60,19 @@ def test_non_finite_entries_stay_in_their_rows(itcpd, dims, at, value):
         for n in range(3):
             bad = ~np.isfinite(plan.mttkrp(n)).all(axis=1)
             assert np.array_equal(np.nonzero(bad)[0], [at[n]])
+
+
+@pytest.mark.parametrize("sweeps", [1, 2, 3, 4])
+@pytest.mark.parametrize("dims,R", [((48, 40, 32), 5), ((33, 70, 90), 6), ((90, 31, 47), 17), ((80, 81, 82), 66)])
+def test_shared_partials_match_oracle(itcpd, dims, R, sweeps):
+    """Odd and even numbers of sweeps (the last partial of an odd run serves one update), both
+    splits of the plain tree, ranks with and without the factorisation riding along."""
+    rng = np.random.default_rng(9)
+    true = [rng.standard_normal((d, R)) for d in dims]
+    T = np.einsum("ir,jr,kr->ijk", *true) + 1e-3 * rng.standard_normal(dims)
+    init = O.random_CPD(T, R, np.random.default_rng(10))
+    ref = O.als_optimize(T, init, check=O.NoCheck(sweeps), form="gemm")
+    got = itcpd.als_optimize(T, itcpd.CPD(init.factors, init.lam), check=itcpd.NoCheck(sweeps))
+    for a, b in zip(got.factors, ref.factors):
+        assert np.linalg.norm(a - b) <= 1e-10 * np.linalg.norm(b)
+    assert np.linalg.norm(got.lam - ref.lam) <= 1e-10 * np.linalg.norm(ref.lam)
