@@ -294,6 +294,11 @@ int itcpd_plan_create(itcpd_plan** out, int32_t order, const int64_t* dims, int6
     if (R <= 64) {
         p->RT = R <= 16 ? 16 : (R <= 32 ? 32 : 64);
         if ((rc = dmalloc(&p->Upad, (size_t)(R * R)))) return bail(rc);   // V^-1
+    } else {
+        const int64_t nb = cdiv(R, 64);
+        if ((rc = dmalloc(&p->inv_buf, (size_t)(2 * 4096 * nb * nb)))) return bail(rc);
+        if ((rc = dmalloc(&p->inv_P, (size_t)2 * 4096))) return bail(rc);
+        if ((rc = dmalloc(&p->inv_stat, (size_t)(3 * nb * nb + nb)))) return bail(rc);
     }
     if ((rc = dmalloc(&p->invdiag, (size_t)R))) return bail(rc);
     if ((rc = dmalloc(&p->qr_aux, (size_t)(R * R + 4 * R)))) return bail(rc);
@@ -350,6 +355,9 @@ int itcpd_plan_destroy(itcpd_plan* p) {
     dfree(p->Af);
     dfree(p->Kt);
     dfree(p->Upad);
+    dfree(p->inv_buf);
+    dfree(p->inv_P);
+    dfree(p->inv_stat);
     dfree(p->PL);
     dfree(p->PR);
     dfree(p->parts);

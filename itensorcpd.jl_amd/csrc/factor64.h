@@ -12,87 +12,19 @@ constexpr size_t FACTOR64_LDS = (size_t)(2 * 64 * 66) * 8;
 constexpr int FACTOR64_RED = 64 * 66;
 constexpr size_t FACTOR64_UNPIV_LDS = (size_t)(64 * 66 + 144) * 8;
 
-// Unpivoted blocked Cholesky V = U^T U and V^-1 = U^-1 U^-T for the R <= 64 row
-// solves (one 256-thread workgroup; V padded to 64 with the identity, ld 66 in S,
-// then U, then U^-1 in place; red = S + FACTOR64_RED, FACTOR64_UNPIV_LDS bytes in
-// all).  Per 16-row panel kb: wave 0 factors the whole block row in registers
-// (lane l holds column l; row j comes through LDS), the trailing update A(ib, jb)
+// The blocked inverse of a symmetric positive definite matrix of at most 64 rows in LDS (one
+// 256-thread workgroup; S: the matrix padded to 64 with the identity, ld 66; nbk = its
+// 16-row panels; red = S + FACTOR64_RED with red[12] = 0 on entry).  Unpivoted Cholesky
+// V = U^T U, then U^-1 in place.  Per 16-row panel kb: wave 0 factors the whole block row in
+// registers (lane l holds column l; row j comes through LDS), the trailing update A(ib, jb)
 // -= U(kb, ib)^T U(kb, jb) runs on FP64 MFMA.  Then the diagonal blocks of U^-1 by
-// substitution (one wave each), the off-diagonal blocks block row by block row
-// from the bottom, X(i, j) = -X(i, i) sum_{i<k<=j} U(i, k) X(k, j) (row i of U is
-// read before it is overwritten), and the upper tiles of U^-1 U^-T on MFMA.
-//
-// It stands in for the pivoted factorisation (xPSTRF, absolute tolerance tol) only
-// when that one provably keeps every pivot: each pivoted pivot is a diagonal entry
-// of a Schur complement of V, hence >= lambda_min(V), and lambda_min(V) >=
-// 1 / ||V^-1||_F.  The computed inverse is trusted while ||V||_F ||V^-1||_F < 1e12;
-// the bound must exceed 2 tol plus the pivots' rounding (64 R eps max V_ii); every
-// unpivoted pivot must be > 0.  Then the solution (the unique minimiser) is the
-// pivoted path's up to rounding, and V^-1, invdiag, piv (identity) and finfo are
-// written; otherwise it returns false and writes nothing but V^-1 (which the
-// caller's pivoted path overwrites or leaves unused).  Uniform result.
-//
-// Bound by its serial chain (about 2 us per 16-row panel), so only the ceil(R / 16)
-// panels that hold any of V are worked on.  In the launch that it rides, us: R = 10,
-// 11 (20 with all four panels); R = 24, 17 (21); R = 37, 19 (21).
-__device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, int R, double tol,
-                                                   double* __restrict__ Vinv, double* __restrict__ invdiag,
-                                                   int* __restrict__ piv, int* __restrict__ finfo, double* S) {
+// substitution (one wave each), the off-diagonal blocks block row by block row from the
+// bottom, X(i, j) = -X(i, i) sum_{i<k<=j} U(i, k) X(k, j) (row i of U is read before it is
+// overwritten).  red[12] = 1 when a pivot was not > 0; 1/U(j,j) in red[16 + j].
+__device__ __forceinline__ void inv64_core(double* S, double* red, int nbk) {
     constexpr int LDT = 66;
-    double* red = S + FACTOR64_RED;   // [0, 16) scalars, then 1/U(j,j) and the broadcast row
     const int t = threadIdx.x, l = t & 63, c = l & 15, g = l >> 4;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int nbk = (R + 15) >> 4;   // 16-row panels that hold any of V; the rest stay the identity
-    if (t == 0) red[12] = 0.0;   // set by wave 0 when a pivot is not > 0
-    // V (mode order of the Hadamard as the pivoted path), identity beyond R; thread
-    // (w, l) fills column l of rows w, w + 4, ...; two modes' loads in flight at once
-    {
-        double v[16];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) v[k] = 1.0;
-        for (int m0 = 0; m0 < gs.N; m0 += 2) {
-            const bool on0 = m0 != mode, on1 = m0 + 1 < gs.N && m0 + 1 != mode;
-            const double* __restrict__ G0 = gs.G[m0];
-            const double* __restrict__ G1 = on1 ? gs.G[m0 + 1] : G0;
-            double g0[16], g1[16];
-#pragma unroll
-            for (int k = 0; k < 16; ++k) {
-                const int i = w + 4 * k;
-                const int x = (i < R && l < R) ? i * R + l : 0;
-                g0[k] = G0[x];
-                g1[k] = G1[x];
-            }
-#pragma unroll
-            for (int k = 0; k < 16; ++k) {
-                if (!on0) g0[k] = 1.0;
-                if (!on1) g1[k] = 1.0;
-            }
-#pragma unroll
-            for (int k = 0; k < 16; ++k) v[k] = (v[k] * g0[k]) * g1[k];
-        }
-        double vsq = 0.0, dmax = 0.0;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const int i = w + 4 * k;
-            const bool in = i < R && l < R;
-            const double x = in ? v[k] : (i == l ? 1.0 : 0.0);
-            S[i * LDT + l] = x;
-            if (in) {
-                vsq = fma(x, x, vsq);
-                if (i == l) dmax = fmax(dmax, x);
-            }
-        }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            vsq += __shfl_xor(vsq, o);
-            dmax = fmax(dmax, __shfl_xor(dmax, o));
-        }
-        if (l == 0) {
-            red[w] = vsq;
-            red[4 + w] = dmax;
-        }
-    }
-    __syncthreads();
     double* invd = red + 16;      // 1/U(j,j), 64 doubles
     double* rowj = red + 80;      // one row of the block row, 64 doubles
     for (int kb = 0; kb < nbk; ++kb) {
@@ -200,30 +132,116 @@ __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, 
         }
         __syncthreads();
     }
-    // upper tiles of Z = U^-1 U^-T (Z(a, b) sums over k >= max(a, b)), both halves to
-    // V^-1, and ||V^-1||_F^2 over the R x R block
+}
+
+// The upper 16 x 16 tiles of Z = U^-1 U^-T from inv64_core's S on FP64 MFMA (Z(a, b) sums
+// over k >= max(a, b)): store(ra, rb, value, ta != tb) for the tiles ta <= tb below nbk.
+template <typename F>
+__device__ __forceinline__ void inv64_tiles(const double* S, int nbk, F store) {
+    constexpr int LDT = 66;
+    const int t = threadIdx.x, l = t & 63, c = l & 15, g = l >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
     constexpr int ZT[4][3][2] = {{{0, 0}, {0, 3}, {-1, -1}},
                                  {{0, 1}, {1, 3}, {2, 3}},
                                  {{1, 1}, {0, 2}, {-1, -1}},
                                  {{1, 2}, {2, 2}, {3, 3}}};
-    double zsq = 0.0;
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
         const int ta = ZT[w][q][0], tb = ZT[w][q][1];
-        if (ta < 0 || 16 * tb >= R) continue;
+        if (ta < 0 || tb >= nbk) continue;
         d4 acc = (d4){0.0, 0.0, 0.0, 0.0};
         for (int k0 = 16 * tb; k0 < 16 * nbk; k0 += 4)
             acc = mfma_f64(S[(16 * ta + c) * LDT + k0 + g], S[(16 * tb + c) * LDT + k0 + g], acc);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int ra = 16 * ta + g + 4 * v, rb = 16 * tb + c;
-            if (ra < R && rb < R) {
-                Vinv[ra * R + rb] = acc[v];
-                if (ta != tb) Vinv[rb * R + ra] = acc[v];
-                zsq = fma((ta != tb ? 2.0 : 1.0) * acc[v], acc[v], zsq);
+        for (int v = 0; v < 4; ++v) store(16 * ta + g + 4 * v, 16 * tb + c, acc[v], ta != tb);
+    }
+}
+
+// Unpivoted V = U^T U and V^-1 = U^-1 U^-T for the R <= 64 row solves (one 256-thread
+// workgroup; V, then U, then U^-1 in S, FACTOR64_UNPIV_LDS bytes with red behind it).
+//
+// It stands in for the pivoted factorisation (xPSTRF, absolute tolerance tol) only
+// when that one provably keeps every pivot: each pivoted pivot is a diagonal entry
+// of a Schur complement of V, hence >= lambda_min(V), and lambda_min(V) >=
+// 1 / ||V^-1||_F.  The computed inverse is trusted while ||V||_F ||V^-1||_F < 1e12;
+// the bound must exceed 2 tol plus the pivots' rounding (64 R eps max V_ii); every
+// unpivoted pivot must be > 0.  Then the solution (the unique minimiser) is the
+// pivoted path's up to rounding, and V^-1, invdiag, piv (identity) and finfo are
+// written; otherwise it returns false and writes nothing but V^-1 (which the
+// caller's pivoted path overwrites or leaves unused).  Uniform result.
+//
+// Bound by its serial chain (about 2 us per 16-row panel), so only the ceil(R / 16)
+// panels that hold any of V are worked on.  In the launch that it rides, us: R = 10,
+// 11 (20 with all four panels); R = 24, 17 (21); R = 37, 19 (21).
+__device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, int R, double tol,
+                                                   double* __restrict__ Vinv, double* __restrict__ invdiag,
+                                                   int* __restrict__ piv, int* __restrict__ finfo, double* S) {
+    constexpr int LDT = 66;
+    double* red = S + FACTOR64_RED;   // [0, 16) scalars, then 1/U(j,j) and the broadcast row
+    const int t = threadIdx.x, l = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nbk = (R + 15) >> 4;   // 16-row panels that hold any of V; the rest stay the identity
+    if (t == 0) red[12] = 0.0;   // set by wave 0 when a pivot is not > 0
+    // V (mode order of the Hadamard as the pivoted path), identity beyond R; thread
+    // (w, l) fills column l of rows w, w + 4, ...; two modes' loads in flight at once
+    {
+        double v[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) v[k] = 1.0;
+        for (int m0 = 0; m0 < gs.N; m0 += 2) {
+            const bool on0 = m0 != mode, on1 = m0 + 1 < gs.N && m0 + 1 != mode;
+            const double* __restrict__ G0 = gs.G[m0];
+            const double* __restrict__ G1 = on1 ? gs.G[m0 + 1] : G0;
+            double g0[16], g1[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const int i = w + 4 * k;
+                const int x = (i < R && l < R) ? i * R + l : 0;
+                g0[k] = G0[x];
+                g1[k] = G1[x];
+            }
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                if (!on0) g0[k] = 1.0;
+                if (!on1) g1[k] = 1.0;
+            }
+#pragma unroll
+            for (int k = 0; k < 16; ++k) v[k] = (v[k] * g0[k]) * g1[k];
+        }
+        double vsq = 0.0, dmax = 0.0;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const int i = w + 4 * k;
+            const bool in = i < R && l < R;
+            const double x = in ? v[k] : (i == l ? 1.0 : 0.0);
+            S[i * LDT + l] = x;
+            if (in) {
+                vsq = fma(x, x, vsq);
+                if (i == l) dmax = fmax(dmax, x);
             }
         }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            vsq += __shfl_xor(vsq, o);
+            dmax = fmax(dmax, __shfl_xor(dmax, o));
+        }
+        if (l == 0) {
+            red[w] = vsq;
+            red[4 + w] = dmax;
+        }
     }
+    __syncthreads();
+    inv64_core(S, red, nbk);
+    const double* invd = red + 16;
+    // both halves of V^-1, and ||V^-1||_F^2 over the R x R block
+    double zsq = 0.0;
+    inv64_tiles(S, nbk, [&](int ra, int rb, double z, bool off) {
+        if (ra < R && rb < R) {
+            Vinv[ra * R + rb] = z;
+            if (off) Vinv[rb * R + ra] = z;
+            zsq = fma((off ? 2.0 : 1.0) * z, z, zsq);
+        }
+    });
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) zsq += __shfl_xor(zsq, o);
     if (l == 0) red[8 + w] = zsq;

@@ -50,7 +50,7 @@ struct Krp64 {
 
 // W[j][r] = prod_{q >= q0} At_q[digit_q(j)][r]: a side's whole Khatri-Rao product (q0 = 0)
 // or the rest weights of its GEMM (q0 = 1), as one rank-fastest array.
-__global__ __launch_bounds__(256) void k_krp64(Side sd, int q0, int64_t n, int Rp, double* __restrict__ W,
+static __global__ __launch_bounds__(256) void k_krp64(Side sd, int q0, int64_t n, int Rp, double* __restrict__ W,
                                                const DevCheck* __restrict__ chk) {
     const int64_t x = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (x >= n * Rp) return;

@@ -122,6 +122,9 @@ struct itcpd_plan {
     double* qr_aux = nullptr;                  // QR fallback workspace (tau, Z reflectors)
     double* invdiag = nullptr;                 // R: 1 / U(j,j) of the pivoted Cholesky
     double* Upad = nullptr;                    // R <= 64: V^-1 (R x R) from the factor kernel
+    double* inv_buf = nullptr;                 // R > 64: two (64 nb)^2 buffers of the blocked inverse
+    double* inv_P = nullptr;                   // the pivot block's inverse (two of 64 x 64)
+    double* inv_stat = nullptr;                // norms and flags of the certificate
     int RT = 0;                                // 16, 32 or 64 for R <= 64, else 0
     double* Msum = nullptr;                    // maxI x R: summed MTTKRP of the last mode (fit)
     unsigned* counters = nullptr;              // arrival counters of last-block reductions

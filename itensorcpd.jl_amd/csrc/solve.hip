@@ -18,8 +18,25 @@
 //    converge_checks.jl:5-11).
 #include "dense_la.h"
 #include "factor64.h"
+#include "inverse.h"
 
 namespace itcpd {
+
+// The certified inverse of inverse.h stands for the pivoted factorisation: its status,
+// finfo[3] = 1, and true; else finfo[3] = 0 and the pivoted kernel goes on.
+__device__ __forceinline__ bool wide_exit(const double* __restrict__ stat, int nb, int R, double tol,
+                                          int* __restrict__ finfo) {
+    const bool ok = wide_certified(stat, nb, R, tol);
+    if (threadIdx.x == 0) {
+        finfo[3] = ok ? 1 : 0;
+        if (ok) {
+            finfo[0] = R;
+            finfo[1] = 0;
+            finfo[2] = R;
+        }
+    }
+    return ok;
+}
 
 // ------------------------------------------------------------ factorisation
 // One workgroup.  Builds V = Hadamard of the Grams of modes != mode, factors it
@@ -38,15 +55,15 @@ __global__ __launch_bounds__(FACTOR_THREADS) void k_factor(GramSet gs, int mode,
                                                            double* __restrict__ qtau,
                                                            double* __restrict__ ztau,
                                                            int* __restrict__ jpvt, double* vwork,
-                                                           int use_lds,
+                                                           const double* __restrict__ stat, int nb,
                                                            const DevCheck* __restrict__ chk) {
     if (chk->done) return;
-    extern __shared__ double lds[];
+    if (wide_exit(stat, nb, R, tol, finfo)) return;
     __shared__ double redv[FACTOR_THREADS];
     __shared__ int redi[FACTOR_THREADS];
     const int t = threadIdx.x;
     constexpr int NT = FACTOR_THREADS;
-    double* S = use_lds ? lds : U;  // full symmetric R x R, row-major
+    double* S = U;  // full symmetric R x R, row-major
     int* pv = piv;
 
     // V = ones .* G_m for m != mode, in mode order (MttkrpAlgorithm.jl:38-47)
@@ -128,8 +145,10 @@ __global__ __launch_bounds__(1024) void k_factor128(GramSet gs, int mode, int R,
                                                     int* __restrict__ piv, int* __restrict__ finfo,
                                                     double* __restrict__ W, double* __restrict__ qtau,
                                                     double* __restrict__ ztau, int* __restrict__ jpvt,
-                                                    double* vwork, const DevCheck* __restrict__ chk) {
+                                                    double* vwork, const double* __restrict__ stat, int nb,
+                                                    const DevCheck* __restrict__ chk) {
     if (chk->done) return;
+    if (wide_exit(stat, nb, R, tol, finfo)) return;
     constexpr int LDT = F128_LDT;
     extern __shared__ double UbT[];   // UbT(l, j) = U(j, l), 128 x LDT
     __shared__ double diagU[128];
@@ -407,11 +426,10 @@ __global__ __launch_bounds__(256) void k_solve(
     const double* __restrict__ Ug, const double* __restrict__ invdiag, const int* __restrict__ piv,
     const int* __restrict__ finfo, const double* __restrict__ W, const double* __restrict__ qtau,
     const double* __restrict__ ztau, const int* __restrict__ jpvt, int u_in_lds,
-    double* __restrict__ X, double* __restrict__ Msum, double* __restrict__ gram_part, int grams,
-    const DevCheck* __restrict__ chk) {
-    if (chk->done) return;
-    solve_rows_dev<RQ, RPW>(Msrc, In, R, Ug, invdiag, piv, finfo, W, qtau, ztau, jpvt, u_in_lds, X, Msum,
-                            gram_part, grams);
+    double* __restrict__ X, const DevCheck* __restrict__ chk) {
+    if (chk->done || finfo[3] == 1) return;   // certified: k_solve_inv solved the rows
+    solve_rows_dev<RQ, RPW>(Msrc, In, R, Ug, invdiag, piv, finfo, W, qtau, ztau, jpvt, u_in_lds, X, nullptr,
+                            nullptr, 0);
 }
 
 // Row solves for R <= RT <= 64.  Cholesky case: X = M V^-1 on FP64 MFMA with the
@@ -1295,15 +1313,24 @@ int launch_factor_on(itcpd_plan* p, int mode_in, hipStream_t st) {
         hipLaunchKernelGGL(k_factor64, dim3(1), dim3(256), FACTOR64_LDS,
                            st, gs, mode, R, 1e-6, p->U, p->Upad, p->invdiag, p->piv,
                            p->finfo, W, qtau, ztau, p->piv + R, vwork, p->chk);
-    } else if (R <= 128) {
-        hipLaunchKernelGGL(k_factor128, dim3(1), dim3(1024), F128_LDS, st, gs, mode, R, 1e-6,
-                           p->U, p->invdiag, p->piv, p->finfo, W, qtau, ztau, p->piv + R, vwork, p->chk);
     } else {
-        // right-looking, all threads; V in LDS up to R = 128, else in the U buffer
-        const bool lds = R <= 128;
-        hipLaunchKernelGGL(k_factor, dim3(1), dim3(FACTOR_THREADS), lds ? (size_t)R * R * 8 : 0, st,
-                           gs, mode, R, 1e-6, p->U, p->invdiag, p->piv, p->finfo, W, qtau,
-                           ztau, p->piv + R, vwork, lds ? 1 : 0, p->chk);
+        // V^-1 by blocks; the pivoted factorisation only when it is not certified
+        const int nb = (int)cdiv(R, 64);
+        const size_t half = (size_t)(64 * nb) * (64 * nb);
+        const dim3 grid((unsigned)nb, (unsigned)nb);
+        hipLaunchKernelGGL(k_inv_first, grid, dim3(256), FACTOR64_UNPIV_LDS, st, gs, mode, R, nb, p->inv_buf,
+                           p->inv_P, p->inv_stat, p->chk);
+        for (int k = 0; k < nb; ++k)
+            hipLaunchKernelGGL(k_inv_step, grid, dim3(256), INV_LDS, st, k, R, nb, p->inv_buf + (k & 1) * half,
+                               p->inv_buf + ((k + 1) & 1) * half, p->inv_P + (k & 1) * 4096,
+                               p->inv_P + ((k + 1) & 1) * 4096, p->inv_stat, p->chk);
+        ITCPD_HIP(hipGetLastError());
+        if (R <= 128)
+            hipLaunchKernelGGL(k_factor128, dim3(1), dim3(1024), F128_LDS, st, gs, mode, R, 1e-6, p->U, p->invdiag,
+                               p->piv, p->finfo, W, qtau, ztau, p->piv + R, vwork, p->inv_stat, nb, p->chk);
+        else
+            hipLaunchKernelGGL(k_factor, dim3(1), dim3(FACTOR_THREADS), 0, st, gs, mode, R, 1e-6, p->U, p->invdiag,
+                               p->piv, p->finfo, W, qtau, ztau, p->piv + R, vwork, p->inv_stat, nb, p->chk);
     }
     ITCPD_HIP(hipGetLastError());
     return ITCPD_OK;
@@ -1328,24 +1355,42 @@ int solve_nb(int64_t In, int R) {
     const int64_t nb = cdiv(In, R <= 64 ? 16 : rpb_of(R));
     return (int)(nb < cap ? nb : cap);
 }
-int finalize_nb(int64_t In) {
+// R <= 64: 32 rows a block, at most 16.  Above, also 256 Gram entries a block (one per
+// thread), at most 128 blocks: 7.9 us at R = 128, I = 224 (45 us with 7 blocks and 56 partials).
+int finalize_nb(int64_t In, int R) {
     const int64_t nb = cdiv(In, 32);
+    if (R > 64) return (int)std::min<int64_t>(128, std::max(nb, cdiv((int64_t)R * R, 256)));
     return (int)(nb < 16 ? (nb < 1 ? 1 : nb) : 16);
 }
 
+// Row ranges of the Gram products: one up to 2048 rows, at most 64 (and within gram_part).
+int gram_parts(int64_t In, int R) {
+    const int64_t cap = std::max<int64_t>(1, ((int64_t)1 << 25) / ((int64_t)R * R));
+    return (int)std::min<int64_t>(std::min<int64_t>(64, cap), std::max<int64_t>(1, cdiv(In, 2048)));
+}
+unsigned gram_tiles(int R) {
+    const unsigned nt = (unsigned)cdiv(R, 16);
+    return nt * (nt + 1) / 2;
+}
+
+// R > 64: X = M V^-1 when the inverse is certified, else the substitution / QR row solves;
+// one of the two launches finds that the other has the rows.
 template <int RQ>
-int run_solve_k(itcpd_plan* p, int mode, const double* Msrc, int nparts, int64_t stride,
-                bool grams, bool keep_m) {
+int run_solve_k(itcpd_plan* p, int mode, const double* Msrc) {
     const int64_t In = p->dims[mode];
     const int R = (int)p->R;
-    const int nb = solve_nb(In, R);
+    const int nbq = (int)cdiv(R, 64);
+    const int64_t Rq = 64 * (int64_t)nbq;
+    hipLaunchKernelGGL(k_solve_inv, dim3((unsigned)cdiv(In, 16), (unsigned)cdiv(cdiv(R, 16), 4)), dim3(256), 0,
+                       p->stream, Msrc, In, R, p->inv_buf + (nbq & 1) * (size_t)(Rq * Rq), Rq, p->finfo, p->X,
+                       p->chk);
     const bool u_lds = R <= 128;
     constexpr int RPW = rpw_of<RQ>();
     const size_t lds = (size_t)4 * RPW * R * 8 + (u_lds ? (size_t)R * (R + 1) * 8 : 0);
     double* W = p->qr_aux;
-    hipLaunchKernelGGL((k_solve<RQ, RPW>), dim3(nb), dim3(256), lds, p->stream, Msrc, In, R, p->U, p->invdiag, p->piv, p->finfo, W, W + (size_t)R * R,
-                       W + (size_t)R * R + R, (const int*)(p->piv + R), u_lds ? 1 : 0, p->X,
-                       keep_m ? p->Msum : (double*)nullptr, p->gram_part, grams ? 1 : 0, p->chk);
+    hipLaunchKernelGGL((k_solve<RQ, RPW>), dim3(solve_nb(In, R)), dim3(256), lds, p->stream, Msrc, In, R, p->U,
+                       p->invdiag, p->piv, p->finfo, W, W + (size_t)R * R, W + (size_t)R * R + R,
+                       (const int*)(p->piv + R), u_lds ? 1 : 0, p->X, p->chk);
     ITCPD_HIP(hipGetLastError());
     return ITCPD_OK;
 }
@@ -1374,11 +1419,10 @@ int run_apply(itcpd_plan* p, int mode, const double* Msrc, int nparts, int64_t s
     if (p->RT == 16) return run_solve_rows<16>(p, mode, Msrc, nparts, stride, grams, keep_m);
     if (p->RT == 32) return run_solve_rows<32>(p, mode, Msrc, nparts, stride, grams, keep_m);
     if (p->RT == 64) return run_solve_rows<64>(p, mode, Msrc, nparts, stride, grams, keep_m);
-    if (R <= 64) return run_solve_k<1>(p, mode, Msrc, nparts, stride, grams, keep_m);
-    if (R <= 128) return run_solve_k<2>(p, mode, Msrc, nparts, stride, grams, keep_m);
-    if (R <= 256) return run_solve_k<4>(p, mode, Msrc, nparts, stride, grams, keep_m);
-    if (R <= 512) return run_solve_k<8>(p, mode, Msrc, nparts, stride, grams, keep_m);
-    return run_solve_k<16>(p, mode, Msrc, nparts, stride, grams, keep_m);
+    if (R <= 128) return run_solve_k<2>(p, mode, Msrc);
+    if (R <= 256) return run_solve_k<4>(p, mode, Msrc);
+    if (R <= 512) return run_solve_k<8>(p, mode, Msrc);
+    return run_solve_k<16>(p, mode, Msrc);
 }
 
 }  // namespace
@@ -1398,11 +1442,21 @@ int launch_solve(itcpd_plan* p, int mode, const double* Msrc, int nparts, int64_
     rc = run_apply(p, mode, Msrc, nparts, stride, finalize, fit_after);
     if (rc || !finalize) return rc;
     const int64_t In = p->dims[mode];
-    const int nb = solve_nb(In, R);
-    const int nbf = finalize_nb(In);
+    int nb = solve_nb(In, R);
+    const double* Mkept = p->Msum;
+    if (!p->RT) {   // R > 64: the Gram of X by its own launch; M is still where the solve read it
+        GramJobs gj{};
+        gj.X[0] = p->X;
+        gj.S[0] = p->gram_part;
+        gj.I[0] = In;
+        nb = gram_parts(In, R);
+        hipLaunchKernelGGL(k_gram_mfma, dim3(gram_tiles(R), (unsigned)nb), dim3(256), 0, p->stream, gj, R, nb, p->chk);
+        Mkept = Msrc;
+    }
+    const int nbf = finalize_nb(In, R);
     const bool one_rt = nb <= 32 && R <= 256 && cdiv((int64_t)R * R, nbf) <= 256 && cdiv(In, nbf) * R <= 2048;
     hipLaunchKernelGGL(one_rt ? k_finalize_1rt : k_finalize, dim3(nbf), dim3(256), one_rt ? 0 : (size_t)R * 8,
-                       p->stream, p->gram_part, nb, p->X, p->Msum, In, R, (int)p->Rp, p->A[mode], p->At[mode],
+                       p->stream, p->gram_part, nb, p->X, Mkept, In, R, (int)p->Rp, p->A[mode], p->At[mode],
                        p->lam, p->G[mode], (fit_after && !cp_check) ? p->inner_part : (double*)nullptr, p->chk);
     ITCPD_HIP(hipGetLastError());
     if (fit_after && cp_check) {
@@ -1448,21 +1502,42 @@ int launch_normalize(itcpd_plan* p, int mode, const double* Xsrc, bool fit_after
 
 // Gram cache seeding (optimizers/als_optimizers/standard/tensor.jl:12) and the
 // rank-fastest copies of the factors.
+//
+// One launch for the copies and one for the Grams of every mode of at most 2048 rows; longer
+// modes sum row ranges.  Was a row-normalisation and a single-workgroup sum per mode: 3 x 89
+// us at 512^3 rank 64, 3 x 290 us at 200^3 rank 150.
 int launch_seed_grams(itcpd_plan* p) {
     const int R = (int)p->R;
-    const int rpb = rows_per_block_for(R);
+    TransposeJobs tj{};
+    GramJobs gj{};
+    int64_t imax = 0;
     for (int m = 0; m < p->N; ++m) {
-        const int64_t In = p->dims[m];
-        const int nb2 = norm_blocks(In, R, rpb);
-        const size_t lds = (size_t)(R + rpb * R) * 8;
-        hipLaunchKernelGGL(k_normalize, dim3(nb2), dim3(256), lds, p->stream, p->A[m], In, R,
-                           (int)p->Rp, p->sumsq_part, 0, rpb, p->A[m], p->At[m], p->lam,
-                           p->gram_part, p->M, 0, p->inner_part, 0, (const DevCheck*)nullptr);
+        tj.A[m] = gj.X[m] = p->A[m];
+        tj.At[m] = p->At[m];
+        tj.I[m] = gj.I[m] = p->dims[m];
+        gj.S[m] = p->G[m];
+        imax = std::max(imax, p->dims[m]);
+    }
+    hipLaunchKernelGGL(k_rank_fast, dim3((unsigned)cdiv(imax, 32), (unsigned)cdiv(R, 32), (unsigned)p->N), dim3(256),
+                       0, p->stream, tj, R, (int)p->Rp);
+    ITCPD_HIP(hipGetLastError());
+    if (gram_parts(imax, R) == 1) {
+        hipLaunchKernelGGL(k_gram_mfma, dim3(gram_tiles(R), 1, (unsigned)p->N), dim3(256), 0, p->stream, gj, R, 1,
+                           (const DevCheck*)nullptr);
         ITCPD_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_gram_final, dim3(1), dim3(256), 0, p->stream, p->gram_part, nb2, R,
-                           p->G[m], grams_of(p), m, p->lam, p->inner_part, 0, p->scal,
-                           (DevCheck*)nullptr, (double*)nullptr, 0);
+        return ITCPD_OK;
+    }
+    for (int m = 0; m < p->N; ++m) {
+        const int nb = gram_parts(p->dims[m], R);
+        GramJobs one{};
+        one.X[0] = p->A[m];
+        one.I[0] = p->dims[m];
+        one.S[0] = nb == 1 ? p->G[m] : p->gram_part;
+        hipLaunchKernelGGL(k_gram_mfma, dim3(gram_tiles(R), (unsigned)nb), dim3(256), 0, p->stream, one, R, nb,
+                           (const DevCheck*)nullptr);
         ITCPD_HIP(hipGetLastError());
+        if (nb == 1) continue;
+        if (int rc = launch_sum_parts(p, MSrc{p->gram_part, nb, (int64_t)R * R}, (int64_t)R * R, p->G[m])) return rc;
     }
     return ITCPD_OK;
 }

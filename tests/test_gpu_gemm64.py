@@ -76,3 +76,40 @@ def test_shared_partials_match_oracle(itcpd, dims, R, sweeps):
     for a, b in zip(got.factors, ref.factors):
         assert np.linalg.norm(a - b) <= 1e-10 * np.linalg.norm(b)
     assert np.linalg.norm(got.lam - ref.lam) <= 1e-10 * np.linalg.norm(ref.lam)
+
+
+@pytest.mark.parametrize("R", [65, 80, 127, 128, 129, 191, 192, 193, 257])
+def test_blocked_inverse_solves(itcpd, R):
+    """R > 64: one to five pivot blocks, the last of 1 to 64 rows.  Forward error of an
+    inverse-based solve: 8 R 2^-53 cond(V) of the solution's norm; and a V of deficient rank
+    goes to the QR path."""
+    rng = np.random.default_rng(11)
+    dims = (R + 40, R + 30, 40)
+    T = np.asfortranarray(rng.standard_normal(dims))
+    fac = [rng.standard_normal((d, R)) / np.sqrt(d) for d in dims]
+    with itcpd.ALSPlan(T, R) as plan:
+        plan.set_cpd(itcpd.CPD(fac, np.ones(R)))
+        M = rng.standard_normal((40, R))
+        V = (fac[0].T @ fac[0]) * (fac[1].T @ fac[1])
+        X, fell = plan.solve_ls(2, M)
+        ref = np.linalg.solve(V, M.T).T
+        assert not fell
+        assert np.linalg.norm(X - ref) <= 8 * R * 2.0**-53 * np.linalg.cond(V) * np.linalg.norm(ref)
+        fac[0][:, 1], fac[1][:, 1] = fac[0][:, 0], fac[1][:, 0]
+        plan.set_cpd(itcpd.CPD(fac, np.ones(R)))
+        assert plan.solve_ls(2, M)[1]
+
+
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 63, 2048, 2049, 5000])
+@pytest.mark.parametrize("R", [1, 16, 17, 70])
+def test_seeded_grams(itcpd, rows, R):
+    """G_n = A_n^T A_n after set_cpd, through V of the modes of a two-mode tensor: the
+    rounding bound of its sums."""
+    rng = np.random.default_rng(12)
+    A = [rng.standard_normal((rows, R)), rng.standard_normal((3, R))]
+    with itcpd.ALSPlan(np.asfortranarray(rng.standard_normal((rows, 3))), R) as plan:
+        plan.set_cpd(itcpd.CPD(A, np.ones(R)))
+        for mode in (0, 1):
+            B = A[1 - mode]
+            bound = 2 * (B.shape[0] + 2) * 2.0**-53 * (np.abs(B).T @ np.abs(B))
+            assert (np.abs(plan.compute_krp(mode) - B.T @ B) / bound).max() <= 1.0, mode
