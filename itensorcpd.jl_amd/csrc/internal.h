@@ -304,8 +304,6 @@ struct MlpDev {
     int64_t step = 0;
 };
 
-int mlp_gemm(hipStream_t st, bool ta, bool tb, int M, int N, int K, float alpha, const float* A, int lda,
-             const float* B, int ldb, float beta, float* C, int ldc);
 int mlp_forward(const MlpDev& m, int batch, const float* X, hipStream_t st);
 int mlp_backward(const MlpDev& m, int batch, const float* X, const float* Yt, const float* mask,
                  double* loss_dev, hipStream_t st);

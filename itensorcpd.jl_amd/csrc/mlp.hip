@@ -16,76 +16,158 @@
 namespace itcpd {
 namespace {
 
-constexpr int TB = 64;    // output tile (TB x TB) per workgroup
-constexpr int TKB = 16;   // reduction slab
-constexpr int GT = 256;   // threads: 16 x 16, each a 4 x 4 micro-tile
+typedef float mf4 __attribute__((ext_vector_type(4)));
+typedef float mfu4 __attribute__((ext_vector_type(4), aligned(4)));
 
-// C(MxN) = alpha * op(A)(MxK) * op(B)(KxN) + beta * C, all row-major.
-// op(A) = A (lda) or A^T (A stored KxM); op(B) likewise.  LDS tiles padded by
-// one column against bank conflicts; every global access is bounds-checked.
-template <bool TA, bool TBt>
-__global__ __launch_bounds__(GT) void k_sgemm(int M, int N, int K, float alpha,
-                                              const float* __restrict__ A, int lda,
-                                              const float* __restrict__ B, int ldb, float beta,
-                                              float* __restrict__ C, int ldc) {
-    __shared__ float As[TKB][TB + 1];
-    __shared__ float Bs[TKB][TB + 1];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int m0 = blockIdx.y * TB, n0 = blockIdx.x * TB;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < K; k0 += TKB) {
-        for (int e = threadIdx.x; e < TKB * TB; e += GT) {
-            // A tile element (kk, mm) = op(A)(m0 + mm, k0 + kk)
-            const int kk = TA ? e / TB : e % TKB;
-            const int mm = TA ? e % TB : e / TKB;
-            const int m = m0 + mm, k = k0 + kk;
-            float v = 0.f;
-            if (m < M && k < K) v = TA ? A[(size_t)k * lda + m] : A[(size_t)m * lda + k];
-            As[kk][mm] = v;
-            // B tile element (kk, nn) = op(B)(k0 + kk, n0 + nn)
-            const int kb = TBt ? e % TKB : e / TB;
-            const int nb = TBt ? e / TKB : e % TB;
-            const int n = n0 + nb, k2 = k0 + kb;
-            float w = 0.f;
-            if (n < N && k2 < K) w = TBt ? B[(size_t)n * ldb + k2] : B[(size_t)k2 * ldb + n];
-            Bs[kb][nb] = w;
-        }
-        __syncthreads();
+// One product of the network, C(M x N) = op(A)(M x K) op(B)(K x N), row-major, and what is
+// done to it on the way out.
+struct MlpProduct {
+    const float *A, *B;
+    float* C;
+    int M, N, K, lda, ldb;      // C has leading dimension N
+    const float* bias;          // added to every row (null: none)
+    int relu;                   // then negative values are set to 0
+    const float* gate;          // M x N: the result is 0 where the gate is not > 0 (null: none)
+    float* colsum;              // N column sums of op(B) (null: none)
+};
+
+// A wave's 16 T x 16 T tile (tile row tm, column tn) of a product on v_mfma_f32_16x16x4_f32,
+// operands straight from global memory (a network's matrices live in L2).  A stage is 16
+// reduction indices, lane (c, g) taking 4 g .. 4 g + 3: one 16-byte run where the index is
+// contiguous, else four rows of which the 16 lanes read 64 bytes each.  Eight stages (T = 1;
+// four for T = 2) are in flight together: these products are bound by latency, 256 x 256 x 256
+// having one tile per CU, so every round trip to L2 shows.  Rows past the end read the last
+// one, stages past the last whole one are zeroed after the load.
+template <bool TA, bool TB, int T>
+__device__ __forceinline__ void mlp_tile(const MlpProduct& q, int tm, int tn) {
+    constexpr int U = T == 1 ? 8 : 4;
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    int m[T], n[T];
 #pragma unroll
-        for (int kk = 0; kk < TKB; ++kk) {
-            float a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[kk][ty + 16 * i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * b[j];
-        }
-        __syncthreads();
+    for (int i = 0; i < T; ++i) {
+        const int mm = 16 * (T * tm + i) + c, nn = 16 * (T * tn + i) + c;
+        m[i] = mm < q.M ? mm : q.M - 1;
+        n[i] = nn < q.N ? nn : q.N - 1;
     }
+    auto loadA = [&](int i, int k, float (&x)[4]) {   // op(A)(m[i], k .. k + 3)
+        if constexpr (TA) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty + 16 * i;
-        if (m >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx + 16 * j;
-            if (n >= N) continue;
-            float* c = C + (size_t)m * ldc + n;
-            *c = alpha * acc[i][j] + (beta == 0.f ? 0.f : beta * *c);
+            for (int s = 0; s < 4; ++s) x[s] = q.A[(size_t)(k + s) * q.lda + m[i]];
+        } else {
+            const mfu4 v = *reinterpret_cast<const mfu4*>(q.A + (size_t)m[i] * q.lda + k);
+            x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
         }
+    };
+    auto loadB = [&](int j, int k, float (&x)[4]) {   // op(B)(k .. k + 3, n[j])
+        if constexpr (!TB) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) x[s] = q.B[(size_t)(k + s) * q.ldb + n[j]];
+        } else {
+            const mfu4 v = *reinterpret_cast<const mfu4*>(q.B + (size_t)n[j] * q.ldb + k);
+            x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+        }
+    };
+    mf4 acc[T][T];
+    float cs[T];
+#pragma unroll
+    for (int i = 0; i < T; ++i) {
+        cs[i] = 0.f;
+#pragma unroll
+        for (int j = 0; j < T; ++j) acc[i][j] = (mf4){0.f, 0.f, 0.f, 0.f};
+    }
+    const int full = q.K / 16;
+    for (int s0 = 0; s0 < full; s0 += U) {
+        float a[U][T][4], b[U][T][4];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = 16 * (s0 + u < full ? s0 + u : full - 1) + 4 * g;
+#pragma unroll
+            for (int i = 0; i < T; ++i) loadA(i, k, a[u][i]);
+#pragma unroll
+            for (int j = 0; j < T; ++j) loadB(j, k, b[u][j]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool in = s0 + u < full;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+#pragma unroll
+                for (int j = 0; j < T; ++j) {
+                    const float bv = in ? b[u][j][s] : 0.f;
+                    cs[j] += bv;
+#pragma unroll
+                    for (int i = 0; i < T; ++i)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? a[u][i][s] : 0.f, bv, acc[i][j], 0, 0, 0);
+                }
+            }
+        }
+    }
+    if (16 * full < q.K) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int k = 16 * full + 4 * g + s, kc = k < q.K ? k : q.K - 1;
+            float a[T], b[T];
+#pragma unroll
+            for (int i = 0; i < T; ++i) {
+                a[i] = TA ? q.A[(size_t)kc * q.lda + m[i]] : q.A[(size_t)m[i] * q.lda + kc];
+                b[i] = TB ? q.B[(size_t)n[i] * q.ldb + kc] : q.B[(size_t)kc * q.ldb + n[i]];
+                if (k >= q.K) a[i] = b[i] = 0.f;
+                cs[i] += b[i];
+            }
+#pragma unroll
+            for (int i = 0; i < T; ++i)
+#pragma unroll
+                for (int j = 0; j < T; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+    }
+    // result: lane (c, g), register v holds row 4 g + v, column c
+#pragma unroll
+    for (int j = 0; j < T; ++j) {
+        const int col = 16 * (T * tn + j) + c;
+        if (q.colsum && tm == 0) {
+            float s = cs[j];
+            s += __shfl_xor(s, 16);
+            s += __shfl_xor(s, 32);
+            if (g == 0 && col < q.N) q.colsum[col] = s;
+        }
+        if (col >= q.N) continue;
+        const float bias = q.bias ? q.bias[col] : 0.f;
+#pragma unroll
+        for (int i = 0; i < T; ++i)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int row = 16 * (T * tm + i) + 4 * g + v;
+                if (row >= q.M) continue;
+                float x = acc[i][j][v] + bias;
+                if (q.relu && x < 0.f) x = 0.f;
+                if (q.gate && !(q.gate[(size_t)row * q.N + col] > 0.f)) x = 0.f;
+                q.C[(size_t)row * q.N + col] = x;
+            }
     }
 }
 
-// H = act(H + b) in place (row-major, width N)
-__global__ __launch_bounds__(256) void k_bias_act(float* __restrict__ H, const float* __restrict__ b,
-                                                  int64_t n, int N, int relu) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    float v = H[i] + b[i % N];
-    H[i] = (relu && v < 0.f) ? 0.f : v;
+// H = act(X W + b): wave w of a block takes tile 4 blockIdx.x + w, row by row of tiles.
+template <int T>
+__global__ __launch_bounds__(256) void k_mlp_forward(MlpProduct q) {
+    const int tiles_n = (q.N + 16 * T - 1) / (16 * T);
+    const int64_t tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int tm = (int)(tile / tiles_n);
+    if (tm * 16 * T >= q.M) return;
+    mlp_tile<false, false, T>(q, tm, (int)(tile % tiles_n));
+}
+
+// A layer's two backward products in one launch: blocks below nw the weight gradient
+// dW = H^T dZ (and db, the column sums of dZ), the others dH = dZ W^T gated by H > 0.
+template <int T>
+__global__ __launch_bounds__(256) void k_mlp_backward(MlpProduct dw, MlpProduct dh, unsigned nw) {
+    const bool weight = blockIdx.x < nw;
+    const MlpProduct& q = weight ? dw : dh;
+    const int tiles_n = (q.N + 16 * T - 1) / (16 * T);
+    const int64_t tile = (int64_t)(weight ? blockIdx.x : blockIdx.x - nw) * 4 + (threadIdx.x >> 6);
+    const int tm = (int)(tile / tiles_n), tn = (int)(tile % tiles_n);
+    if (tm * 16 * T >= q.M) return;
+    if (weight) mlp_tile<true, false, T>(q, tm, tn);
+    else mlp_tile<false, true, T>(q, tm, tn);
 }
 
 // dZ = mask .* (Y - Y*) / batch (output layer), and the per-block loss partials
@@ -108,21 +190,6 @@ __global__ __launch_bounds__(256) void k_mse_grad(const float* __restrict__ Y, c
         __syncthreads();
     }
     if (threadIdx.x == 0) loss_part[blockIdx.x] = red[0];
-}
-
-// dZ .*= (H > 0)  (ReLU derivative from the activation output)
-__global__ __launch_bounds__(256) void k_relu_bwd(float* __restrict__ dZ, const float* __restrict__ H, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n && !(H[i] > 0.f)) dZ[i] = 0.f;
-}
-
-// db(j) = sum_i dZ(i, j): one thread per column, rows in order
-__global__ __launch_bounds__(256) void k_colsum(const float* __restrict__ dZ, int rows, int N, float* __restrict__ db) {
-    const int j = blockIdx.x * 256 + threadIdx.x;
-    if (j >= N) return;
-    float s = 0.f;
-    for (int i = 0; i < rows; ++i) s += dZ[(size_t)i * N + j];
-    db[j] = s;
 }
 
 __global__ __launch_bounds__(256) void k_adam(float* __restrict__ p, const float* __restrict__ g,
@@ -341,30 +408,27 @@ int launch_gauss_sketch(itcpd_plan* p, int mode, int K, uint64_t seed, double* S
 }
 
 
-
-
-int mlp_gemm(hipStream_t st, bool ta, bool tb, int M, int N, int K, float alpha, const float* A, int lda,
-             const float* B, int ldb, float beta, float* C, int ldc) {
-    dim3 grid((unsigned)((N + TB - 1) / TB), (unsigned)((M + TB - 1) / TB));
-    if (!ta && !tb) hipLaunchKernelGGL((k_sgemm<false, false>), grid, dim3(GT), 0, st, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
-    else if (ta && !tb) hipLaunchKernelGGL((k_sgemm<true, false>), grid, dim3(GT), 0, st, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
-    else if (!ta && tb) hipLaunchKernelGGL((k_sgemm<false, true>), grid, dim3(GT), 0, st, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
-    else hipLaunchKernelGGL((k_sgemm<true, true>), grid, dim3(GT), 0, st, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
-    ITCPD_HIP(hipGetLastError());
-    return ITCPD_OK;
-}
-
 // ---------------------------------------------------------------- network
+namespace {
+int64_t mlp_tiles(const MlpProduct& q, int T) {
+    return (int64_t)((q.M + 16 * T - 1) / (16 * T)) * ((q.N + 16 * T - 1) / (16 * T));
+}
+// 32 x 32 tiles (half the operand loads per flop) once 16 x 16 ones would give every SIMD
+// four waves; below that more, smaller tiles hide the latency better.
+bool mlp_wide(const MlpProduct& q) { return mlp_tiles(q, 1) >= 4096; }
+unsigned mlp_blocks(const MlpProduct& q, int T) { return (unsigned)((mlp_tiles(q, T) + 3) / 4); }
+}  // namespace
+
+// Network 200 -> 256 -> 256 -> 200, batch 256: forward 3 launches of 9.8 us (6 of 30 before,
+// 64 x 64 VALU tiles on 16 workgroups), backward 3 of 7.4 us beside the loss (10 of 30).
 int mlp_forward(const MlpDev& m, int batch, const float* X, hipStream_t st) {
     const float* in = X;
     for (int l = 0; l < m.nlayers; ++l) {
         const int K = m.widths[l], N = m.widths[l + 1];
         float* H = m.act[l];
-        int rc;
-        if ((rc = mlp_gemm(st, false, false, batch, N, K, 1.f, in, K, m.W[l], N, 0.f, H, N))) return rc;
-        const int64_t n = (int64_t)batch * N;
-        hipLaunchKernelGGL(k_bias_act, dim3(nblk(n)), dim3(256), 0, st, H, m.b[l], n, N,
-                           l + 1 < m.nlayers ? 1 : 0);
+        const MlpProduct q{in, m.W[l], H, batch, N, K, K, N, m.b[l], l + 1 < m.nlayers ? 1 : 0, nullptr, nullptr};
+        if (mlp_wide(q)) hipLaunchKernelGGL(k_mlp_forward<2>, dim3(mlp_blocks(q, 2)), dim3(256), 0, st, q);
+        else hipLaunchKernelGGL(k_mlp_forward<1>, dim3(mlp_blocks(q, 1)), dim3(256), 0, st, q);
         ITCPD_HIP(hipGetLastError());
         in = H;
     }
@@ -383,20 +447,17 @@ int mlp_backward(const MlpDev& m, int batch, const float* X, const float* Yt, co
     ITCPD_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_sum_loss, dim3(1), dim3(256), 0, st, m.loss_part, (int)nblk(nout), loss_dev);
     ITCPD_HIP(hipGetLastError());
-    int rc;
     for (int l = L - 1; l >= 0; --l) {
         const int K = m.widths[l], N = m.widths[l + 1];
         const float* in = l == 0 ? X : m.act[l - 1];
-        // dW_l = in^T dZ, db_l = colsum(dZ)
-        if ((rc = mlp_gemm(st, true, false, K, N, batch, 1.f, in, K, dZ, N, 0.f, m.gW[l], N))) return rc;
-        hipLaunchKernelGGL(k_colsum, dim3(nblk(N)), dim3(256), 0, st, dZ, batch, N, m.gb[l]);
-        ITCPD_HIP(hipGetLastError());
-        if (l == 0) break;
-        // dZ_{l-1} = (dZ W_l^T) .* relu'(act[l-1])
         float* dPrev = (dZ == m.dA) ? m.dB : m.dA;
-        if ((rc = mlp_gemm(st, false, true, batch, K, N, 1.f, dZ, N, m.W[l], N, 0.f, dPrev, K))) return rc;
-        const int64_t np = (int64_t)batch * K;
-        hipLaunchKernelGGL(k_relu_bwd, dim3(nblk(np)), dim3(256), 0, st, dPrev, m.act[l - 1], np);
+        // dW_l = in^T dZ, db_l = colsum(dZ); dZ_{l-1} = (dZ W_l^T) .* relu'(act[l-1])
+        const MlpProduct dw{in, dZ, m.gW[l], K, N, batch, K, N, nullptr, 0, nullptr, m.gb[l]};
+        const MlpProduct dh{dZ, m.W[l], dPrev, batch, K, N, N, N, nullptr, 0, l > 0 ? m.act[l - 1] : nullptr, nullptr};
+        const int T = mlp_wide(dw) && (l == 0 || mlp_wide(dh)) ? 2 : 1;
+        const unsigned nw = mlp_blocks(dw, T), nh = l > 0 ? mlp_blocks(dh, T) : 0;
+        if (T == 2) hipLaunchKernelGGL(k_mlp_backward<2>, dim3(nw + nh), dim3(256), 0, st, dw, dh, nw);
+        else hipLaunchKernelGGL(k_mlp_backward<1>, dim3(nw + nh), dim3(256), 0, st, dw, dh, nw);
         ITCPD_HIP(hipGetLastError());
         dZ = dPrev;
     }
