@@ -102,15 +102,13 @@ hipError_t create_streams(itcpd_plan* p) {
 }
 
 // Buffers of the reduced-precision GEMMs, allocated on the first switch away from
-// FP64: the converted first factor; for an FP32-stored tensor also a side's
-// Khatri-Rao product (rank padded to 128, 4 bytes per element) and room for 8
-// split-K partials of the larger side's output.
+// FP64: a side's Khatri-Rao product (4 bytes per element); for an FP32-stored tensor
+// also room for 8 split-K partials of the larger side's output.
 int ensure_lp_buffers(itcpd_plan* p) {
     int rc;
-    if (!p->Af && (rc = dmalloc(&p->Af, (size_t)(p->maxI * p->R)))) return rc;
+    if (!p->Kt && (rc = dmalloc(&p->Kt, (size_t)lp_krp_elems(p)))) return rc;
     if (p->elt_bytes != 4) return ITCPD_OK;
     const int64_t Mmax = std::max(p->ML, p->MR);
-    if (!p->Kt && (rc = dmalloc(&p->Kt, (size_t)(Mmax * cdiv(p->R, 128) * 128)))) return rc;
     const size_t want = std::min<size_t>((size_t)8 * (size_t)(Mmax * p->R), (size_t)1 << 27);
     if (p->parts_elems < want) {
         ITCPD_HIP(hipStreamSynchronize(p->stream));
@@ -352,7 +350,6 @@ int itcpd_plan_destroy(itcpd_plan* p) {
     dfree(p->qr_aux);
     dfree(p->piv);
     dfree(p->finfo);
-    dfree(p->Af);
     dfree(p->Kt);
     dfree(p->Upad);
     dfree(p->inv_buf);

@@ -131,8 +131,7 @@ struct itcpd_plan {
     int* piv = nullptr;                        // R
     int* finfo = nullptr;                      // [0] = rank, [1] = used fallback, [2] = QR rank
     double* PL = nullptr;                      // ML x Rp partial of the left side (if s > 1)
-    float* Af = nullptr;                       // FP32 copy of the KRP side's first factor (reduced precision)
-    float* Kt = nullptr;                       // FP32-stored T, reduced precision: a side's KRP, rank-major
+    float* Kt = nullptr;                       // reduced precision: a side's Khatri-Rao product, rank-major
     double* Wrest = nullptr;                   // a side's Khatri-Rao product or rest weights (rank fastest)
     double* P3 = nullptr;                      // order 3: the partial that serves two mode updates (tree3)
     bool tree3 = false;                        // order 3: partials shared across sweeps
@@ -204,6 +203,7 @@ bool tree3_pays(const itcpd_plan* p);
 int64_t tree3_elems(const itcpd_plan* p);
 int launch_tree3_gemm(itcpd_plan* p, int c);
 int launch_tree3_ttv(itcpd_plan* p, int mode, int c, MSrc* ms, int factor_mode);
+int64_t lp_krp_elems(const itcpd_plan* p);     // 4-byte elements of p->Kt
 int64_t krp64_elems(const itcpd_plan* p);      // doubles of p->Wrest
 int mttkrp_mode(itcpd_plan* p, int mode);      // full M_mode into p->M from the current factors
 // out = the sum of ms's partials; factor_mode >= 0: that mode's factorisation too
