@@ -7,158 +7,182 @@
 namespace itcpd {
 
 constexpr size_t FACTOR64_LDS = (size_t)(2 * 64 * 66) * 8;
-// LDS of the unpivoted form alone: V / U / U^-1 (64 x 66) and 144 doubles of
-// reductions, 1/U(j,j) and the broadcast row
-constexpr int FACTOR64_RED = 64 * 66;
-constexpr size_t FACTOR64_UNPIV_LDS = (size_t)(64 * 66 + 144) * 8;
+// LDS of the unpivoted form alone: four broadcast rows and 16 doubles of reductions
+constexpr size_t FACTOR64_UNPIV_LDS = (size_t)(4 * 128 + 16) * 8;
 
-// The blocked inverse of a symmetric positive definite matrix of at most 64 rows in LDS (one
-// 256-thread workgroup; S: the matrix padded to 64 with the identity, ld 66; nbk = its
-// 16-row panels; red = S + FACTOR64_RED with red[12] = 0 on entry).  Unpivoted Cholesky
-// V = U^T U, then U^-1 in place.  Per 16-row panel kb: wave 0 factors the whole block row in
-// registers (lane l holds column l; row j comes through LDS), the trailing update A(ib, jb)
-// -= U(kb, ib)^T U(kb, jb) runs on FP64 MFMA.  Then the diagonal blocks of U^-1 by
-// substitution (one wave each), the off-diagonal blocks block row by block row from the
-// bottom, X(i, j) = -X(i, i) sum_{i<k<=j} U(i, k) X(k, j) (row i of U is read before it is
-// overwritten).  red[12] = 1 when a pivot was not > 0; 1/U(j,j) in red[16 + j].
-__device__ __forceinline__ void inv64_core(double* S, double* red, int nbk) {
-    constexpr int LDT = 66;
-    const int t = threadIdx.x, l = t & 63, c = l & 15, g = l >> 4;
-    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-    double* invd = red + 16;      // 1/U(j,j), 64 doubles
-    double* rowj = red + 80;      // one row of the block row, 64 doubles
-    for (int kb = 0; kb < nbk; ++kb) {
-        const int b0 = 16 * kb;
-        if (w == 0) {
-            // Block row kb (rows b0..b0+15, all 64 columns): lane l holds column l.
-            // Step j: row j goes through LDS (lane l writes A(b0+j, l)); d =
-            // A(b0+j, b0+j), 1/sqrt(d) from the hardware estimate and two Newton
-            // steps, U(b0+j, l) = A(b0+j, l)/sqrt(d) for l > b0+j, and rows i > j take
-            // A(b0+i, l) -= A(b0+j, b0+i) A(b0+j, l) / d.  Lanes l < b0 (finished
-            // columns) compute along on values nobody reads and store zeros.
-            double col[16];
+// LDS written by lanes of one wave, then read by other lanes of the same wave: the wave's LDS
+// operations complete in order, so only the compiler must keep them so.
+__device__ __forceinline__ void lds_wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Inverse of a symmetric positive definite n x n matrix by symmetric sweeps, in registers.
+// A thread holds 16 rows (16 grp ..) of one column col; rows and columns >= n are zero.
+// Sweeping index k, with r the k-th row (= column) and d = r_k: the element (i, l) takes
+// a - r_i r_l / d, row and column k become r / d and (k, k) -1 / d.  After n sweeps the matrix
+// is -A^-1; it stays symmetric throughout, so the rows being swept, handed to every thread
+// through LDS, are all that a step needs.  The d are the pivots of the unpivoted
+// factorisation; false when one was not > 0.
+//
+// A step sweeps k and k + 1 together: p, q their rows, B = [d1 c; c e] their 2 x 2 block, (T1,
+// T2) = B^-1 (p_l, q_l): the element (i, l) takes a - p_i T1 - q_i T2, rows k and k + 1 become
+// T1 and T2.  With an odd n the index n is a 1 on the diagonal.  The step's critical chain is
+// 1 / det B, the next two rows' multiply-adds and their way through LDS: those rows go first
+// and their reads are issued before the other rows are updated; d1 and e come from a running
+// copy of the diagonal by readlane, not from the rows.
+//
+// The loop body is short on purpose: unrolled over all steps it is straight-line code that
+// every launch fetches anew (27 us at n = 64).  So that registers are not indexed by k, every
+// step rotates the rows by two (position j holds row 16 grp + (j + k) mod 16, the rows being
+// swept sit at positions 0 and 1, the next ones at 2 and 3), and each row in LDS keeps its
+// 16-entry groups twice in a row, so a rotated group is one run.
+//
+// WAVES = 1: one wave, n <= 32, grp = lane >> 5, col = lane & 31, rows in LDS order, no
+// barrier; WAVES = 4: a 256-thread workgroup, n <= 64, grp = wave, col = lane, one barrier a
+// step (two row buffers), and p_i, q_i, which a wave's lanes share, by readlane from one
+// LDS read (delivered to every lane they would take 512 cycles of the LDS port a step).
+// rows: SWEEP_ROWS doubles of LDS.  On return position j holds row sweep_row(n, grp, j).
+constexpr int SWEEP_ROWS = 4 * 128;
+
+__device__ __forceinline__ int sweep_row(int n, int grp, int j) { return 16 * grp + ((j + n + (n & 1)) & 15); }
+
+__device__ __forceinline__ double lane_double(double v, int k) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), k),
+                            __builtin_amdgcn_readlane(__double2loint(v), k));
+}
+// Wave-wide sum / maximum by DPP row rotations and the four rows' values (uniform result):
+// shorter chains than LDS shuffles.
+template <int CTRL>
+__device__ __forceinline__ double dpp_double(double v) {
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false));
+}
+__device__ __forceinline__ double wave_sum_dpp(double v) {
+    v += dpp_double<0x128>(v);   // row_ror:8
+    v += dpp_double<0x124>(v);
+    v += dpp_double<0x122>(v);
+    v += dpp_double<0x121>(v);
+    return (lane_double(v, 0) + lane_double(v, 16)) + (lane_double(v, 32) + lane_double(v, 48));
+}
+__device__ __forceinline__ double wave_max_dpp(double v) {
+    v = fmax(v, dpp_double<0x128>(v));
+    v = fmax(v, dpp_double<0x124>(v));
+    v = fmax(v, dpp_double<0x122>(v));
+    v = fmax(v, dpp_double<0x121>(v));
+    return fmax(fmax(lane_double(v, 0), lane_double(v, 16)), fmax(lane_double(v, 32), lane_double(v, 48)));
+}
+__device__ __forceinline__ double newton_rcp(double d) {
+    // the estimate's error e (< 2^-20) cubed
+    const double y = __builtin_amdgcn_rcp(d), e = fma(-d, y, 1.0);
+    return fma(y, fma(e, e, e), y);
+}
+
+template <int WAVES>
+__device__ __forceinline__ bool sweep_inverse(double (&a)[16], int n, int grp, int col, double* rows) {
+    auto sync = [] {
+        if (WAVES == 1) lds_wave_order();
+        else __syncthreads();
+    };
+    const int at = 32 * (col >> 4) + (col & 15);   // this column's place in a row in LDS
+    auto put = [&](double* row, double v) {
+        row[at] = v;
+        row[at + 16] = v;
+    };
+    double dg = 0.0;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) col[i] = S[(b0 + i) * LDT + l];
-            bool pos = true;
+    for (int i = 0; i < 16; ++i) {
+        const bool here = 16 * grp + i == col;
+        a[i] = here && (n & 1) && col == n ? 1.0 : a[i];
+        dg = here ? a[i] : dg;
+    }
+    if (col >> 4 == grp) rows[256 + at] = dg;
+    if (grp == 0) {
+        put(rows, a[0]);
+        put(rows + 128, a[1]);
+    }
+    sync();
+    dg = rows[256 + at];
+    const int lane = threadIdx.x & 63;
+    // the rows' entries of this column and of this group
+    double pl, ql;
+    auto fetch = [&](const double* row, int k, double (&p)[16], double (&q)[16]) {
+        const double* run = row + 32 * grp + (k & 15);
+        pl = row[at];
+        ql = row[128 + at];
+        if (WAVES == 4) {
+            p[0] = run[(lane & 15) + 8 * (lane & 16)];   // lane j: p_j, lane 16 + j: q_j
+        } else {
 #pragma unroll
             for (int j = 0; j < 16; ++j) {
-                rowj[l] = col[j];
-                const double d = rowj[b0 + j];
-                double bi[16];
-#pragma unroll
-                for (int i = j + 1; i < 16; ++i) bi[i] = rowj[b0 + i];
-                pos = pos && d > 0.0;
-                const double dc = fmax(d, 0x1p-1020);
-                const double h = 0.5 * dc;
-                double y = __builtin_amdgcn_rsq(dc);
-                y = fma(y, fma(-h * y, y, 0.5), y);
-                y = fma(y, fma(-h * y, y, 0.5), y);
-                const double u = l > b0 + j ? col[j] * y : (l == b0 + j ? dc * y : 0.0);
-                const double ncu = -(u * y);
-#pragma unroll
-                for (int i = j + 1; i < 16; ++i) col[i] = fma(bi[i], ncu, col[i]);
-                col[j] = u;
-                invd[b0 + j] = y;
+                p[j] = run[j];
+                q[j] = run[128 + j];
             }
-#pragma unroll
-            for (int i = 0; i < 16; ++i) S[(b0 + i) * LDT + l] = l >= b0 + i ? col[i] : 0.0;
-            if (!pos) red[12] = 1.0;
         }
-        __syncthreads();
-        // trailing update of the upper blocks kb < ib <= jb (round-robin over waves).
-        // f64 16x16x4 layout: A lane (c, g) = A[c][k0+g], B lane = B[k0+g][c], result
-        // v = D[g+4v][c]
-        if (kb + 1 < nbk) {
-            int idx = 0;
-            for (int ib = kb + 1; ib < nbk; ++ib)
-                for (int jb = ib; jb < nbk; ++jb, ++idx) {
-                    if ((idx & 3) != w) continue;
-                    d4 acc;
+    };
+    double pa[16], qa[16], pb[16], qb[16];
+    fetch(rows, 0, pa, qa);
+    sync();   // the diagonal's place is the next rows'
+    bool pos = true;
+    // the step of rows k, k + 1 in (p, q); the next two go to (pn, qn)
+    auto step = [&](int k, double (&p)[16], double (&q)[16], double (&pn)[16], double (&qn)[16]) {
+        const double d1 = lane_double(dg, k), e = lane_double(dg, k + 1), c = lane_double(pl, k + 1);
+        const double det = fma(d1, e, -c * c);
+        pos = pos && d1 > 0.0 && det > 0.0;
+        const double inv = newton_rcp(det);
+        double t1 = fma(e, pl, -c * ql) * inv, t2 = fma(d1, ql, -c * pl) * inv;
+        dg = fma(-pl, t1, fma(-ql, t2, dg));
+        const bool c1 = col == k, c2 = col == k + 1;
+        t1 = c1 ? -e * inv : (c2 ? c * inv : t1);
+        t2 = c1 ? c * inv : (c2 ? -d1 * inv : t2);
+        const double keep = c1 || c2 ? 0.0 : 1.0;
+        if (WAVES == 4) {
+            const double pq = p[0];
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[v] = S[(16 * ib + g + 4 * v) * LDT + 16 * jb + c];
-#pragma unroll
-                    for (int k0 = 0; k0 < 16; k0 += 4)
-                        acc = mfma_f64(-S[(b0 + k0 + g) * LDT + 16 * ib + c], S[(b0 + k0 + g) * LDT + 16 * jb + c],
-                                       acc);
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) S[(16 * ib + g + 4 * v) * LDT + 16 * jb + c] = acc[v];
-                }
-            __syncthreads();
-        }
-    }
-    // diagonal blocks of U^-1, wave w block w: lane c computes column c by
-    // substitution (zero below the diagonal; the four 16-lane groups alike)
-    if (w < nbk) {
-        const int b0 = 16 * w;
-        double xv[16];
-#pragma unroll
-        for (int i = 15; i >= 0; --i) {
-            double acc0 = (i == c) ? 1.0 : 0.0, acc1 = 0.0;
-#pragma unroll
-            for (int k = i + 1; k < 16; ++k) {
-                const double uik = S[(b0 + i) * LDT + b0 + k];
-                if (k & 1) acc1 -= uik * xv[k];
-                else acc0 -= uik * xv[k];
+            for (int j = 0; j < 16; ++j) {
+                p[j] = lane_double(pq, j);
+                q[j] = lane_double(pq, 16 + j);
             }
-            xv[i] = (i <= c) ? (acc0 + acc1) * invd[b0 + i] : 0.0;
         }
-        // (the wave's own reads of U(w, w) precede these writes)
+        double* next = rows + 256 * ((k / 2 + 1) & 1);
+        if ((k + 2) >> 4 == grp) {
+            const double v2 = fma(-p[2], t1, a[2] * keep), v3 = fma(-p[3], t1, a[3] * keep);
+            put(next, fma(-q[2], t2, v2));
+            put(next + 128, fma(-q[3], t2, v3));
+        }
+        sync();
+        fetch(next, k + 2, pn, qn);
+        // a <- a keep - p t1 - q t2 in passes of 16 independent operations
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) S[(b0 + i) * LDT + b0 + c] = xv[i];
+        for (int j = 0; j < 16; ++j) a[j] *= keep;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) a[j] = fma(-p[j], t1, a[j]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) a[j] = fma(-q[j], t2, a[j]);
+        __builtin_amdgcn_sched_barrier(0);
+        const bool own = k >> 4 == grp;
+        const double r0 = own ? t1 : a[0], r1 = own ? t2 : a[1];
+#pragma unroll
+        for (int j = 0; j < 14; ++j) a[j] = a[j + 2];
+        a[14] = r0;
+        a[15] = r1;
+    };
+#pragma unroll 1
+    for (int k = 0;; k += 4) {
+        step(k, pa, qa, pb, qb);
+        if (k + 2 >= n) break;
+        step(k + 2, pb, qb, pa, qa);
+        if (k + 4 >= n) break;
     }
-    __syncthreads();
-    // off-diagonal blocks of U^-1, block row bi from the bottom, wave w column
-    // bi + 1 + w: X_ij = -X_ii sum_{k=i+1..j} U_ik X_kj, from row i of U and the
-    // finished rows below; row i is overwritten after every wave has read it
-    for (int bi = nbk - 2; bi >= 0; --bi) {
-        const int bj = bi + 1 + w;
-        d4 out = (d4){0.0, 0.0, 0.0, 0.0};
-        if (bj < nbk) {
-            const int i = 16 * bi + c;
-            d4 acc = (d4){0.0, 0.0, 0.0, 0.0};
-            for (int bk = bi + 1; bk <= bj; ++bk)
-#pragma unroll
-                for (int k0 = 0; k0 < 16; k0 += 4) {
-                    const int kk = 16 * bk + k0 + g;
-                    acc = mfma_f64(S[i * LDT + kk], S[kk * LDT + 16 * bj + c], acc);
-                }
-#pragma unroll
-            for (int v = 0; v < 4; ++v) out = mfma_f64(-S[(16 * bi + c) * LDT + 16 * bi + 4 * v + g], acc[v], out);
-        }
-        __syncthreads();
-        if (bj < nbk) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) S[(16 * bi + g + 4 * v) * LDT + 16 * bj + c] = out[v];
-        }
-        __syncthreads();
-    }
+    return pos;
 }
 
-// The upper 16 x 16 tiles of Z = U^-1 U^-T from inv64_core's S on FP64 MFMA (Z(a, b) sums
-// over k >= max(a, b)): store(ra, rb, value, ta != tb) for the tiles ta <= tb below nbk.
-template <typename F>
-__device__ __forceinline__ void inv64_tiles(const double* S, int nbk, F store) {
-    constexpr int LDT = 66;
-    const int t = threadIdx.x, l = t & 63, c = l & 15, g = l >> 4;
-    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-    constexpr int ZT[4][3][2] = {{{0, 0}, {0, 3}, {-1, -1}},
-                                 {{0, 1}, {1, 3}, {2, 3}},
-                                 {{1, 1}, {0, 2}, {-1, -1}},
-                                 {{1, 2}, {2, 2}, {3, 3}}};
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        const int ta = ZT[w][q][0], tb = ZT[w][q][1];
-        if (ta < 0 || tb >= nbk) continue;
-        d4 acc = (d4){0.0, 0.0, 0.0, 0.0};
-        for (int k0 = 16 * tb; k0 < 16 * nbk; k0 += 4)
-            acc = mfma_f64(S[(16 * ta + c) * LDT + k0 + g], S[(16 * tb + c) * LDT + k0 + g], acc);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) store(16 * ta + g + 4 * v, 16 * tb + c, acc[v], ta != tb);
-    }
-}
-
-// Unpivoted V = U^T U and V^-1 = U^-1 U^-T for the R <= 64 row solves (one 256-thread
-// workgroup; V, then U, then U^-1 in S, FACTOR64_UNPIV_LDS bytes with red behind it).
+// Unpivoted V^-1 for the R <= 64 row solves (one 256-thread workgroup; the first wave alone
+// up to R = 32).
 //
 // It stands in for the pivoted factorisation (xPSTRF, absolute tolerance tol) only
 // when that one provably keeps every pivot: each pivoted pivot is a diagonal entry
@@ -166,99 +190,90 @@ __device__ __forceinline__ void inv64_tiles(const double* S, int nbk, F store) {
 // 1 / ||V^-1||_F.  The computed inverse is trusted while ||V||_F ||V^-1||_F < 1e12;
 // the bound must exceed 2 tol plus the pivots' rounding (64 R eps max V_ii); every
 // unpivoted pivot must be > 0.  Then the solution (the unique minimiser) is the
-// pivoted path's up to rounding, and V^-1, invdiag, piv (identity) and finfo are
-// written; otherwise it returns false and writes nothing but V^-1 (which the
-// caller's pivoted path overwrites or leaves unused).  Uniform result.
+// pivoted path's up to rounding, and V^-1 and finfo are written; otherwise it returns
+// false and writes nothing but V^-1 (which the caller's pivoted path overwrites or leaves
+// unused).  Uniform result.
 //
-// Bound by its serial chain (about 2 us per 16-row panel), so only the ceil(R / 16)
-// panels that hold any of V are worked on.  In the launch that it rides, us: R = 10,
-// 11 (20 with all four panels); R = 24, 17 (21); R = 37, 19 (21).
+// Bound by its chain of R / 2 steps on one wave per SIMD (about 165 instructions of 5 cycles).
+// Gram loads to V^-1, us: R = 1 3.9, 10 5.2, 24 7.7, 37 13.6, 64 19.7; the blocked Cholesky,
+// triangular inverse and product of them that this replaces took 11 (R = 10), 17 (R = 24), 19
+// (R = 37), 29 (R = 64) in the Hadamard-reduce launch that carries them, where this takes 7,
+// 14, 17 and 28.
 __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, int R, double tol,
-                                                   double* __restrict__ Vinv, double* __restrict__ invdiag,
-                                                   int* __restrict__ piv, int* __restrict__ finfo, double* S) {
-    constexpr int LDT = 66;
-    double* red = S + FACTOR64_RED;   // [0, 16) scalars, then 1/U(j,j) and the broadcast row
+                                                   double* __restrict__ Vinv, int* __restrict__ finfo,
+                                                   double* S) {
+    double* red = S + SWEEP_ROWS;   // behind the broadcast rows
     const int t = threadIdx.x, l = t & 63;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int nbk = (R + 15) >> 4;   // 16-row panels that hold any of V; the rest stay the identity
-    if (t == 0) red[12] = 0.0;   // set by wave 0 when a pivot is not > 0
-    // V (mode order of the Hadamard as the pivoted path), identity beyond R; thread
-    // (w, l) fills column l of rows w, w + 4, ...; two modes' loads in flight at once
-    {
-        double v[16];
+    const bool one = R <= 32;
+    if (!one || w == 0) {
+        const int grp = one ? l >> 5 : w, col = one ? l & 31 : l;
+        // V in the mode order of the pivoted path's Hadamard; two modes' loads in flight
+        double a[16];
 #pragma unroll
-        for (int k = 0; k < 16; ++k) v[k] = 1.0;
+        for (int i = 0; i < 16; ++i) a[i] = 1.0;
         for (int m0 = 0; m0 < gs.N; m0 += 2) {
             const bool on0 = m0 != mode, on1 = m0 + 1 < gs.N && m0 + 1 != mode;
             const double* __restrict__ G0 = gs.G[m0];
             const double* __restrict__ G1 = on1 ? gs.G[m0 + 1] : G0;
             double g0[16], g1[16];
 #pragma unroll
-            for (int k = 0; k < 16; ++k) {
-                const int i = w + 4 * k;
-                const int x = (i < R && l < R) ? i * R + l : 0;
-                g0[k] = G0[x];
-                g1[k] = G1[x];
+            for (int i = 0; i < 16; ++i) {
+                const int r = 16 * grp + i, x = (r < R && col < R) ? r * R + col : 0;
+                g0[i] = G0[x];
+                g1[i] = G1[x];
             }
 #pragma unroll
-            for (int k = 0; k < 16; ++k) {
-                if (!on0) g0[k] = 1.0;
-                if (!on1) g1[k] = 1.0;
-            }
-#pragma unroll
-            for (int k = 0; k < 16; ++k) v[k] = (v[k] * g0[k]) * g1[k];
-        }
-        double vsq = 0.0, dmax = 0.0;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const int i = w + 4 * k;
-            const bool in = i < R && l < R;
-            const double x = in ? v[k] : (i == l ? 1.0 : 0.0);
-            S[i * LDT + l] = x;
-            if (in) {
-                vsq = fma(x, x, vsq);
-                if (i == l) dmax = fmax(dmax, x);
+            for (int i = 0; i < 16; ++i) {
+                if (!on0) g0[i] = 1.0;
+                if (!on1) g1[i] = 1.0;
+                a[i] = (a[i] * g0[i]) * g1[i];
             }
         }
+        double vsq = 0.0, dmax = 0.0, zsq = 0.0;
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            vsq += __shfl_xor(vsq, o);
-            dmax = fmax(dmax, __shfl_xor(dmax, o));
+        for (int i = 0; i < 16; ++i) {
+            const int r = 16 * grp + i;
+            if (r >= R || col >= R) a[i] = 0.0;
+            vsq = fma(a[i], a[i], vsq);
+            if (r == col) dmax = fmax(dmax, a[i]);
         }
+        const bool pos = one ? sweep_inverse<1>(a, R, grp, col, S) : sweep_inverse<4>(a, R, grp, col, S);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int r = sweep_row(R, grp, i);
+            if (r < R && col < R) {
+                Vinv[r * R + col] = -a[i];
+                zsq = fma(a[i], a[i], zsq);
+            }
+        }
+        vsq = wave_sum_dpp(vsq);
+        zsq = wave_sum_dpp(zsq);
+        dmax = wave_max_dpp(dmax);
         if (l == 0) {
             red[w] = vsq;
             red[4 + w] = dmax;
+            red[8 + w] = zsq;
+            if (w == 0) red[12] = pos ? 0.0 : 1.0;
         }
     }
     __syncthreads();
-    inv64_core(S, red, nbk);
-    const double* invd = red + 16;
-    // both halves of V^-1, and ||V^-1||_F^2 over the R x R block
-    double zsq = 0.0;
-    inv64_tiles(S, nbk, [&](int ra, int rb, double z, bool off) {
-        if (ra < R && rb < R) {
-            Vinv[ra * R + rb] = z;
-            if (off) Vinv[rb * R + ra] = z;
-            zsq = fma((off ? 2.0 : 1.0) * z, z, zsq);
+    double vs = red[0], dmax = red[4], zs = red[8];
+    if (!one)
+        for (int q = 1; q < 4; ++q) {
+            vs += red[q];
+            dmax = fmax(dmax, red[4 + q]);
+            zs += red[8 + q];
         }
-    });
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) zsq += __shfl_xor(zsq, o);
-    if (l == 0) red[8 + w] = zsq;
-    __syncthreads();
-    const double vF = sqrt((red[0] + red[1]) + (red[2] + red[3]));
-    const double dmax = fmax(fmax(red[4], red[5]), fmax(red[6], red[7]));
-    const double zF = sqrt((red[8] + red[9]) + (red[10] + red[11]));
+    const double vF = sqrt(vs), zF = sqrt(zs);
     const bool cert = red[12] == 0.0 && zF > 0.0 && zF < __builtin_inf() &&
                       1.0 / zF > 2.0 * tol + 64.0 * R * 0x1p-52 * dmax && vF * zF < 1e12;
-    if (cert) {
-        for (int j = t; j < R; j += 256) {
-            invdiag[j] = invd[j];
-            piv[j] = j;
-        }
-        if (t == 0) { finfo[0] = R; finfo[1] = 0; finfo[2] = R; }
+    if (cert && t == 0) {
+        finfo[0] = R;
+        finfo[1] = 0;
+        finfo[2] = R;
     }
-    __syncthreads();   // red and S are reused by the pivoted path
+    __syncthreads();   // S is reused by the pivoted path
     return cert;
 }
 
@@ -295,7 +310,7 @@ __device__ __forceinline__ void factor64_dev(GramSet gs, int mode, int R, double
     double* UbT = S + 64 * LDT;
     const int t = threadIdx.x, l = t & 63;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-    if (Vinv && try_unpivoted && factor64_unpivoted(gs, mode, R, tol, Vinv, invdiag, piv, finfo, S)) return;
+    if (Vinv && try_unpivoted && factor64_unpivoted(gs, mode, R, tol, Vinv, finfo, S)) return;
     fill_hadamard<256>(S, gs, mode, R * R);
     __syncthreads();
     d16 sr;

@@ -122,8 +122,8 @@ __device__ __forceinline__ void lp_flush(f4 (&acc)[N], d4 (&tot)[N]) {
 // LEFT: outputs are rows (VEC of them consecutive per lane, the tile moved back to end at the
 // last row when VEC > 1, which then needs outs >= 16 MB); else columns.  Grid: x rank blocks
 // (the workgroups that share a tensor tile run together) times tiles, z reduction splits.
-template <bool LEFT, typename TT, bool BF, int RB, int MB, int KW, int VEC>
-__global__ __launch_bounds__(256, 2) void k_gemm_lp(const TT* __restrict__ T, int64_t outs, int64_t K,
+template <bool LEFT, typename TT, bool BF, int RB, int MB, int KW, int VEC, int D, int OCC>
+__global__ __launch_bounds__(256, OCC) void k_gemm_lp(const TT* __restrict__ T, int64_t outs, int64_t K,
                                                     const void* __restrict__ Kt, int64_t Kp, int64_t lo_off,
                                                     int64_t stages_per_split, int ny, int R,
                                                     double* __restrict__ out, int64_t split_stride,
@@ -167,8 +167,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_lp(const TT* __restrict__ T, in
         acc[a] = (f4){0.f, 0.f, 0.f, 0.f};
         tot[a] = (d4){0.0, 0.0, 0.0, 0.0};
     }
-    KrpRun<BF> kr[2][RB];
-    float x[2][MB][E];
+    KrpRun<BF> kr[D][RB];
+    float x[D][MB][E];
     auto load = [&](int buf, int64_t st) {
         const int64_t k = st * ST + E * g;
         if constexpr (LEFT) {
@@ -198,15 +198,16 @@ __global__ __launch_bounds__(256, 2) void k_gemm_lp(const TT* __restrict__ T, in
     };
     const int64_t full = K / ST < s1 ? K / ST : s1;
     int64_t st = s0;
-    if (st < full) {
-        load(0, st);
-        while (true) {
-            if (st + 1 < full) load(1, st + 1);
-            compute(0);
-            if (++st == full) break;
-            if (st + 1 < full) load(0, st + 1);
-            compute(1);
-            if (++st == full) break;
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d)
+        if (st + d < full) load(d, st + d);
+    while (st < full) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            if (st >= full) break;
+            if (st + D - 1 < full) load((d + D - 1) % D, st + D - 1);
+            compute(d);
+            ++st;
         }
     }
     // the last, partial stage: indices past the end read the last one and become zeros

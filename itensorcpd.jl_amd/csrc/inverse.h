@@ -10,7 +10,7 @@
 // (k_inv_step) reads the blocks of buffer k & 1, the inverse P of the pivot block (k, k), and
 // writes buffer (k + 1) & 1:
 //   (k, k) <- P,  (k, j) <- P A_kj,  (i, k) <- -A_ik P,  (i, j) <- A_ij - A_ik P A_kj,
-// one workgroup per block; the one of block (k + 1, k + 1) goes on to invert it (inv64_core).
+// one workgroup per block; the one of block (k + 1, k + 1) goes on to invert it (sweep_inverse).
 // After nb launches the buffer holds V^-1.  The pivot blocks are the Schur complements of
 // the unpivoted block factorisation, so their Cholesky pivots are those of V.
 //
@@ -26,8 +26,8 @@ namespace itcpd {
 
 constexpr int INV_LD = 66;
 constexpr int INV_TILE = 64 * INV_LD;
-// three 64 x 64 tiles and the inverse's reductions
-constexpr size_t INV_LDS = (size_t)(3 * INV_TILE + 144) * 8;
+// three 64 x 64 tiles and the inverse's broadcast rows
+constexpr size_t INV_LDS = (size_t)(3 * INV_TILE + SWEEP_ROWS) * 8;
 
 
 // Sums (or maxima) of v over the workgroup's four waves by red[0..3]; thread 0 gets it.
@@ -42,23 +42,23 @@ __device__ __forceinline__ double block4_sum(double v, double* red) {
     return v;
 }
 
-// Inverts the 64 x 64 pivot block in S (rows and columns >= rb are the identity) into P.
-__device__ __forceinline__ void inv_pivot(double* S, int rb, double* __restrict__ P, double* __restrict__ flag) {
-    double* red = S + FACTOR64_RED;
-    const int t = threadIdx.x;
-    const int nbk = (rb + 15) >> 4;
-    if (t == 0) red[12] = 0.0;
-    __syncthreads();
-    inv64_core(S, red, nbk);
-    inv64_tiles(S, nbk, [&](int ra, int rc, double z, bool off) {
-        P[ra * 64 + rc] = z;
-        if (off) P[rc * 64 + ra] = z;
-    });
-    for (int x = t; x < 64 * 64; x += 256) {
-        const int i = x >> 6, j = x & 63;
-        if (i >= 16 * nbk || j >= 16 * nbk) P[x] = i == j ? 1.0 : 0.0;
+// Inverts the rb x rb pivot block of the 64 x 64 tile S into P (identity beyond rb).
+__device__ __forceinline__ void inv_pivot(const double* S, double* rows, int rb, double* __restrict__ P,
+                                          double* __restrict__ flag) {
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    double a[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int r = 16 * w + i;
+        a[i] = r < rb && l < rb ? S[r * INV_LD + l] : 0.0;
     }
-    if (t == 0) flag[0] = red[12];
+    const bool pos = sweep_inverse<4>(a, rb, w, l, rows);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int r = sweep_row(rb, w, i);
+        P[r * 64 + l] = r < rb && l < rb ? -a[i] : (r == l ? 1.0 : 0.0);
+    }
+    if (threadIdx.x == 0) flag[0] = pos ? 0.0 : 1.0;
 }
 
 // V = Hadamard of the Grams of modes != mode in blocks, identity beyond R; block (0, 0) is
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256) void k_inv_first(GramSet gs, int mode, int R, 
         stat[bi * nb + bj] = vsq;
         stat[nb * nb + bi * nb + bj] = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
     }
-    if (bi == 0 && bj == 0) inv_pivot(S, R < 64 ? R : 64, P, stat + 3 * nb * nb);
+    if (bi == 0 && bj == 0) inv_pivot(S, S + INV_TILE, R < 64 ? R : 64, P, stat + 3 * nb * nb);
 }
 
 __global__ __launch_bounds__(256) void k_inv_step(int k, int R, int nb, const double* __restrict__ src,
@@ -118,9 +118,10 @@ __global__ __launch_bounds__(256) void k_inv_step(int k, int R, int nb, const do
     if (chk->done) return;
     extern __shared__ __attribute__((aligned(16))) double S[];
     __shared__ double red[4];
-    double* Pt = S;                     // P, later the next pivot block (with the reductions behind it)
-    double* At = S + INV_TILE + 144;    // A_ik, then A_ik P
-    double* Bt = At + INV_TILE;         // A_kj
+    double* Pt = S;                // P, later the next pivot block
+    double* At = S + INV_TILE;     // A_ik, then A_ik P
+    double* Bt = At + INV_TILE;    // A_kj
+    double* rows = Bt + INV_TILE;
     const int t = threadIdx.x, l = t & 63, c = l & 15, g = l >> 4;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int bi = blockIdx.x, bj = blockIdx.y;
@@ -208,7 +209,7 @@ __global__ __launch_bounds__(256) void k_inv_step(int k, int R, int nb, const do
             for (int v = 0; v < 4; ++v) Pt[(16 * w + g + 4 * v) * INV_LD + 16 * b + c] = acc[b][v];
         __syncthreads();
         const int rb = R - 64 * (k + 1) < 64 ? R - 64 * (k + 1) : 64;
-        inv_pivot(Pt, rb, Pnext, stat + 3 * nb * nb + k + 1);
+        inv_pivot(Pt, rows, rb, Pnext, stat + 3 * nb * nb + k + 1);
     }
 }
 

@@ -536,8 +536,7 @@ __global__ __launch_bounds__(NW * 64, 4) void k_tr_ring(const double* __restrict
     if (fj.on && blockIdx.x == 0) {
         // the unpivoted factorisation of mode fj.mode in this launch's LDS (no
         // done test, as factor_block)
-        const bool ok = factor64_unpivoted(fj.gs, fj.mode, fj.R, fj.tol, fj.Vinv, fj.invdiag, fj.piv, fj.finfo,
-                                           reinterpret_cast<double*>(ring));
+        const bool ok = factor64_unpivoted(fj.gs, fj.mode, fj.R, fj.tol, fj.Vinv, fj.finfo, reinterpret_cast<double*>(ring));
         if (threadIdx.x == 0) fj.finfo[3] = ok ? 1 : 0;
         return;
     }
@@ -905,6 +904,10 @@ int lp_rb(int64_t R) {
 }
 constexpr int lp_big(bool bf, int rb) { return rb <= (bf ? 2 : 3) ? 4 : 2; }
 
+// Register stages: three where they fit (160^4-like shapes, FP32, us with two / three: rank 32
+// 231 / 208, rank 64 397 / 360); at rank 48 the third costs more than it hides (252 / 263).
+constexpr int lp_depth(bool bf, int rb) { return !bf && (rb == 2 || rb == 4) ? 3 : 2; }
+
 struct GemmLp {
     bool left;
     int64_t outs, K, Kp, lo;
@@ -916,7 +919,7 @@ template <bool LEFT, typename TT, bool BF, int RB, int MB, int KW, int VEC>
 void launch_lp(itcpd_plan* p, const GemmLp& q) {
     const int64_t nt = cdiv(q.outs, 16 * MB);
     const dim3 grid((unsigned)((KW == 1 ? cdiv(nt, 4) : nt) * q.ny), 1, (unsigned)q.c.nz);
-    hipLaunchKernelGGL((k_gemm_lp<LEFT, TT, BF, RB, MB, KW, VEC>), grid, dim3(256), 0, p->stream, (const TT*)p->T,
+    hipLaunchKernelGGL((k_gemm_lp<LEFT, TT, BF, RB, MB, KW, VEC, lp_depth(BF, RB), 2>), grid, dim3(256), 0, p->stream, (const TT*)p->T,
                        q.outs, q.K, (const void*)p->Kt, q.Kp, q.lo, q.c.per, q.ny, (int)p->R, q.out, q.outs * p->R,
                        p->chk);
 }

@@ -1318,7 +1318,7 @@ int launch_factor_on(itcpd_plan* p, int mode_in, hipStream_t st) {
         const int nb = (int)cdiv(R, 64);
         const size_t half = (size_t)(64 * nb) * (64 * nb);
         const dim3 grid((unsigned)nb, (unsigned)nb);
-        hipLaunchKernelGGL(k_inv_first, grid, dim3(256), FACTOR64_UNPIV_LDS, st, gs, mode, R, nb, p->inv_buf,
+        hipLaunchKernelGGL(k_inv_first, grid, dim3(256), (size_t)(INV_TILE + SWEEP_ROWS) * 8, st, gs, mode, R, nb, p->inv_buf,
                            p->inv_P, p->inv_stat, p->chk);
         for (int k = 0; k < nb; ++k)
             hipLaunchKernelGGL(k_inv_step, grid, dim3(256), INV_LDS, st, k, R, nb, p->inv_buf + (k & 1) * half,
