@@ -53,17 +53,8 @@ int put_factor(itcpd_plan* p, int m, const double* src, int mem) {
     return copy_in(p->A[m], src, (size_t)In * p->R * 8, mem, p->stream);
 }
 
-int reset_check_flags(itcpd_plan* p) {
-    // clear done / nan so that hook calls after a converged run execute
-    DevCheck* h = p->chk_host;
-    ITCPD_HIP(hipMemcpyAsync(h, p->chk, sizeof(DevCheck), hipMemcpyDeviceToHost, p->stream));
-    ITCPD_HIP(hipStreamSynchronize(p->stream));
-    h->done = 0;
-    h->nan_flag = 0;
-    ITCPD_HIP(hipMemcpyAsync(p->chk, h, sizeof(DevCheck), hipMemcpyHostToDevice, p->stream));
-    ITCPD_HIP(hipStreamSynchronize(p->stream));
-    return ITCPD_OK;
-}
+// Clears done / nan so that hook calls after a converged run execute.
+int reset_check_flags(itcpd_plan* p) { return launch_reset_flags(p); }
 
 // Folds finished begin/end event pairs into the per-kernel totals.  With
 // wait == false only pairs whose end event has already completed are taken
@@ -104,12 +95,14 @@ hipError_t create_streams(itcpd_plan* p) {
 // Buffers of the reduced-precision GEMMs, allocated on the first switch away from
 // FP64: a side's Khatri-Rao product (4 bytes per element); for an FP32-stored tensor
 // also room for 8 split-K partials of the larger side's output.
+size_t lp_parts(const itcpd_plan* p) {
+    if (p->elt_bytes != 4) return 0;
+    return std::min<size_t>((size_t)8 * (size_t)(std::max(p->ML, p->MR) * p->R), (size_t)1 << 27);
+}
 int ensure_lp_buffers(itcpd_plan* p) {
     int rc;
     if (!p->Kt && (rc = dmalloc(&p->Kt, (size_t)lp_krp_elems(p)))) return rc;
-    if (p->elt_bytes != 4) return ITCPD_OK;
-    const int64_t Mmax = std::max(p->ML, p->MR);
-    const size_t want = std::min<size_t>((size_t)8 * (size_t)(Mmax * p->R), (size_t)1 << 27);
+    const size_t want = lp_parts(p);
     if (p->parts_elems < want) {
         ITCPD_HIP(hipStreamSynchronize(p->stream));
         dfree(p->parts);
@@ -121,34 +114,72 @@ int ensure_lp_buffers(itcpd_plan* p) {
     return ITCPD_OK;
 }
 
-// Per-mode factor state shared by plans and the plan-free random init.
-int alloc_factor_state(itcpd_plan* p) {
-    int rc;
+// A plan's device buffers come from one allocation: requests are collected, then laid out in
+// order at 256-byte steps (about 25 hipMalloc / hipFree pairs a plan otherwise, most of a
+// short als_optimize call).
+struct Arena {
+    std::vector<std::pair<void**, size_t>> req;
+    size_t bytes = 0;
+    template <typename T>
+    void add(T** ptr, size_t count) {
+        *ptr = nullptr;
+        req.emplace_back((void**)ptr, bytes);
+        bytes += (std::max<size_t>(count, 1) * sizeof(T) + 255) / 256 * 256;
+    }
+    int alloc(char** base) {
+        const int rc = dmalloc(base, bytes);
+        if (rc) return rc;
+        for (auto& r : req) *r.first = *base + r.second;
+        return ITCPD_OK;
+    }
+};
+
+// Per-mode factor state shared by plans and the plan-free random init.  The factors and
+// lambda come first, then the other buffers that start at zero: p->cpd_bytes covers the CPD
+// (what set_cpd and get_cpd move in one copy), p->zero_bytes all that is cleared.
+void factor_state(itcpd_plan* p, Arena& ar) {
     const int64_t R = p->R, Rp = p->Rp, maxI = p->maxI;
-    for (int q = 0; q < p->N; ++q) {
-        if ((rc = dmalloc(&p->A[q], (size_t)(p->dims[q] * Rp)))) return rc;
-        if ((rc = dmalloc(&p->At[q], (size_t)(p->dims[q] * Rp)))) return rc;
-        if ((rc = dmalloc(&p->G[q], (size_t)(R * R)))) return rc;
-        ITCPD_HIP(hipMemset(p->A[q], 0, (size_t)(p->dims[q] * Rp) * 8));
-        ITCPD_HIP(hipMemset(p->At[q], 0, (size_t)(p->dims[q] * Rp) * 8));
-    }
-    if ((rc = dmalloc(&p->lam, (size_t)Rp))) return rc;
-    ITCPD_HIP(hipMemset(p->lam, 0, (size_t)Rp * 8));
-    if ((rc = dmalloc(&p->X, (size_t)(maxI * Rp)))) return rc;
-    if ((rc = dmalloc(&p->M, (size_t)(maxI * Rp)))) return rc;
-    if ((rc = dmalloc(&p->Msum, (size_t)(maxI * Rp)))) return rc;
-    if ((rc = dmalloc(&p->counters, 64))) return rc;
-    ITCPD_HIP(hipMemset(p->counters, 0, 64 * sizeof(unsigned)));
-    if ((rc = dmalloc(&p->sumsq_part, (size_t)(128 * R)))) return rc;
-    {
-        // Gram partials: one per row block of the fused solve / normalisation kernels,
-        // at most 256 blocks and at most 2^25 doubles
-        int64_t nb = std::min<int64_t>(256, std::max<int64_t>(1, ((int64_t)1 << 25) / (R * R)));
-        if ((rc = dmalloc(&p->gram_part, (size_t)(nb * R * R)))) return rc;
-        if ((rc = dmalloc(&p->inner_part, 256))) return rc;
-    }
-    if ((rc = dmalloc(&p->scal, 8))) return rc;
+    for (int q = 0; q < p->N; ++q) ar.add(&p->A[q], (size_t)(p->dims[q] * Rp));
+    ar.add(&p->lam, (size_t)Rp);
+    p->cpd_bytes = ar.bytes;
+    for (int q = 0; q < p->N; ++q) ar.add(&p->At[q], (size_t)(p->dims[q] * Rp));
+    ar.add(&p->counters, 64);
+    ar.add(&p->chk, 1);
+    p->zero_bytes = ar.bytes;
+    for (int q = 0; q < p->N; ++q) ar.add(&p->G[q], (size_t)(R * R));
+    ar.add(&p->X, (size_t)(maxI * Rp));
+    ar.add(&p->M, (size_t)(maxI * Rp));
+    ar.add(&p->Msum, (size_t)(maxI * Rp));
+    ar.add(&p->sumsq_part, (size_t)(128 * R));
+    // Gram partials: one per 16-row tile of the R <= 64 row solves (at most 256), else per
+    // row range of the Gram or normalisation kernels (at most 64); at most 2^25 doubles
+    const int64_t most = R <= 64 ? std::min<int64_t>(256, std::max<int64_t>(64, cdiv(maxI, 16))) : 64;
+    const int64_t nb = std::min<int64_t>(most, std::max<int64_t>(1, ((int64_t)1 << 25) / (R * R)));
+    ar.add(&p->gram_part, (size_t)(nb * R * R));
+    ar.add(&p->inner_part, 256);
+    ar.add(&p->scal, 8);
+}
+int alloc_arena(itcpd_plan* p, Arena& ar) {
+    const int rc = ar.alloc(&p->arena);
+    if (rc) return rc;
+    ITCPD_HIP(hipMemsetAsync(p->arena, 0, p->zero_bytes, p->stream));
     return ITCPD_OK;
+}
+
+// Pinned mirror of the CPD region for host factors (up to 8 MiB): one copy instead of N + 1
+// from pageable memory.  Null where there is none; its padding columns stay zero.
+char* cpd_stage(itcpd_plan* p) {
+    if (!p->stage && !p->stage_failed) {
+        p->stage_failed = p->cpd_bytes > ((size_t)8 << 20) ||
+                          hipHostMalloc((void**)&p->stage, p->cpd_bytes, hipHostMallocDefault) != hipSuccess;
+        if (p->stage_failed) {
+            (void)hipGetLastError();
+            p->stage = nullptr;
+        } else {
+            std::memset(p->stage, 0, p->cpd_bytes);
+        }
+    }
+    return p->stage;
 }
 
 // One ALS sweep (optimize.jl:17-30), every launch on the plan's stream.  Mode n's
@@ -287,44 +318,47 @@ int itcpd_plan_create(itcpd_plan** out, int32_t order, const int64_t* dims, int6
         if (((uintptr_t)tensor) % 16 != 0) return bail(fail(ITCPD_E_ARG, "device tensor must be 16-byte aligned"));
         p->T = tensor;
     }
-    if ((rc = alloc_factor_state(p))) return bail(rc);
-    if ((rc = dmalloc(&p->U, (size_t)(R * R)))) return bail(rc);
+    Arena ar;
+    factor_state(p, ar);
+    ar.add(&p->U, (size_t)(R * R));
     if (R <= 64) {
         p->RT = R <= 16 ? 16 : (R <= 32 ? 32 : 64);
-        if ((rc = dmalloc(&p->Upad, (size_t)(R * R)))) return bail(rc);   // V^-1
+        ar.add(&p->Upad, (size_t)(R * R));   // V^-1
     } else {
         const int64_t nb = cdiv(R, 64);
-        if ((rc = dmalloc(&p->inv_buf, (size_t)(2 * 4096 * nb * nb)))) return bail(rc);
-        if ((rc = dmalloc(&p->inv_P, (size_t)2 * 4096))) return bail(rc);
-        if ((rc = dmalloc(&p->inv_stat, (size_t)(3 * nb * nb + nb)))) return bail(rc);
+        ar.add(&p->inv_buf, (size_t)(2 * 4096 * nb * nb));
+        ar.add(&p->inv_P, (size_t)2 * 4096);
+        ar.add(&p->inv_stat, (size_t)(3 * nb * nb + nb));
     }
-    if ((rc = dmalloc(&p->invdiag, (size_t)R))) return bail(rc);
-    if ((rc = dmalloc(&p->qr_aux, (size_t)(R * R + 4 * R)))) return bail(rc);
-    if ((rc = dmalloc(&p->piv, (size_t)(2 * R)))) return bail(rc);
-    if ((rc = dmalloc(&p->finfo, 4))) return bail(rc);
-    if (const int64_t n = krp64_elems(p))
-        if ((rc = dmalloc(&p->Wrest, (size_t)n))) return bail(rc);
-    if (p->s > 1 && (rc = dmalloc(&p->PL, (size_t)(p->ML * R)))) return bail(rc);
-    if (order - p->s > 1 && (rc = dmalloc(&p->PR, (size_t)(p->MR * R)))) return bail(rc);
+    ar.add(&p->invdiag, (size_t)R);
+    ar.add(&p->qr_aux, (size_t)(R * R + 4 * R));
+    ar.add(&p->piv, (size_t)(2 * R));
+    ar.add(&p->finfo, 4);
+    if (const int64_t n = krp64_elems(p)) ar.add(&p->Wrest, (size_t)n);
+    if (p->s > 1) ar.add(&p->PL, (size_t)(p->ML * R));
+    if (order - p->s > 1) ar.add(&p->PR, (size_t)(p->MR * R));
+    p->trace_cap = 1024;
+    ar.add(&p->fit_trace, (size_t)p->trace_cap);
+    if ((rc = alloc_arena(p, ar))) return bail(rc);
     {
+        // split-K partials: what 512 splits of the larger side could use, up to half of the
+        // tensor's elements (their traffic is weighed against the tensor's) and 128 MiB, and
+        // the 16 partials of the longest mode's Hadamard-reduce
         const size_t outmax = (size_t)std::max<int64_t>(std::max(p->ML, p->MR), maxI) * R;
         size_t want = std::min<size_t>((size_t)1 << 24, outmax * 512);
+        want = std::min<size_t>(want, std::max<size_t>(nel / 2, (size_t)(16 * maxI * R)));
         want = std::max<size_t>(want, 1024 * 4);
+        if (prec != ITCPD_FP64) want = std::max(want, lp_parts(p));
         p->parts_elems = want;
         if ((rc = dmalloc(&p->parts, want))) return bail(rc);
     }
     if (prec != ITCPD_FP64 && (rc = ensure_lp_buffers(p))) return bail(rc);
-    if ((rc = dmalloc(&p->chk, 1))) return bail(rc);
     e = hipHostMalloc((void**)&p->chk_host, sizeof(DevCheck) * (1 + ITCPD_POLL_SLOTS),
                       hipHostMallocDefault);
     if (e != hipSuccess) return bail(hip_fail(e, "hipHostMalloc"));
     std::memset(p->chk_host, 0, sizeof(DevCheck) * (1 + ITCPD_POLL_SLOTS));
-    e = hipMemcpy(p->chk, p->chk_host, sizeof(DevCheck), hipMemcpyHostToDevice);
-    if (e != hipSuccess) return bail(hip_fail(e, "hipMemcpy(check)"));
-    p->trace_cap = 1024;
-    if ((rc = dmalloc(&p->fit_trace, (size_t)p->trace_cap))) return bail(rc);
-    e = hipDeviceSynchronize();
-    if (e != hipSuccess) return bail(hip_fail(e, "hipDeviceSynchronize"));
+    e = hipStreamSynchronize(p->stream);
+    if (e != hipSuccess) return bail(hip_fail(e, "hipStreamSynchronize"));
     *out = p;
     return ITCPD_OK;
 }
@@ -335,44 +369,19 @@ int itcpd_plan_destroy(itcpd_plan* p) {
     if (p->stream) (void)hipStreamSynchronize(p->stream);
     for (hipEvent_t e : p->timer.ev) (void)hipEventDestroy(e);
     dfree(p->T_owned);
-    for (int q = 0; q < ITCPD_MAX_ORDER; ++q) {
-        dfree(p->A[q]);
-        dfree(p->At[q]);
-        dfree(p->G[q]);
-    }
-    dfree(p->lam);
-    dfree(p->X);
-    dfree(p->M);
-    dfree(p->U);
-    dfree(p->invdiag);
-    dfree(p->Msum);
-    dfree(p->counters);
-    dfree(p->qr_aux);
-    dfree(p->piv);
-    dfree(p->finfo);
+    dfree(p->arena);
     dfree(p->Kt);
-    dfree(p->Upad);
-    dfree(p->inv_buf);
-    dfree(p->inv_P);
-    dfree(p->inv_stat);
-    dfree(p->PL);
-    dfree(p->PR);
     dfree(p->parts);
-    dfree(p->sumsq_part);
-    dfree(p->gram_part);
-    dfree(p->inner_part);
-    dfree(p->scal);
-    dfree(p->chk);
-    dfree(p->fit_trace);
+    dfree(p->trace_owned);
     for (int q = 0; q < ITCPD_MAX_ORDER; ++q) dfree(p->Atprev[q]);
     dfree(p->lamprev);
     dfree(p->smp_ws);
     dfree(p->sk_ws);
-    dfree(p->Wrest);
     dfree(p->P3);
     dfree(p->smp_iws);
     dfree(p->xg_part);
     if (p->chk_host) (void)hipHostFree(p->chk_host);
+    if (p->stage) (void)hipHostFree(p->stage);
     for (int q = 0; q < ITCPD_POLL_SLOTS; ++q)
         if (p->ev_poll[q]) (void)hipEventDestroy(p->ev_poll[q]);
     if (p->stream) (void)hipStreamDestroy(p->stream);
@@ -384,11 +393,19 @@ int itcpd_set_cpd(itcpd_plan* p, const double* const* factors, const double* lam
     if (!p || !factors) return fail(ITCPD_E_ARG, "null argument");
     DeviceGuard dg(p->device);
     int rc;
-    for (int m = 0; m < p->N; ++m) {
+    for (int m = 0; m < p->N; ++m)
         if (!factors[m]) return fail(ITCPD_E_ARG, "null factor pointer");
-        if ((rc = put_factor(p, m, factors[m], mem))) return rc;
+    char* const stage = mem == ITCPD_MEM_HOST && lambda ? cpd_stage(p) : nullptr;
+    if (stage) {
+        for (int m = 0; m < p->N; ++m)
+            std::memcpy(stage + ((char*)p->A[m] - p->arena), factors[m], (size_t)(p->dims[m] * p->R) * 8);
+        std::memcpy(stage + ((char*)p->lam - p->arena), lambda, (size_t)p->R * 8);
+        if ((rc = copy_in(p->arena, stage, p->cpd_bytes, mem, p->stream))) return rc;
+    } else {
+        for (int m = 0; m < p->N; ++m)
+            if ((rc = put_factor(p, m, factors[m], mem))) return rc;
+        if (lambda && (rc = copy_in(p->lam, lambda, (size_t)p->R * 8, mem, p->stream))) return rc;
     }
-    if (lambda && (rc = copy_in(p->lam, lambda, (size_t)p->R * 8, mem, p->stream))) return rc;
     if ((rc = reset_check_flags(p))) return rc;
     if ((rc = launch_seed_grams(p))) return rc;
     ITCPD_HIP(hipStreamSynchronize(p->stream));
@@ -438,7 +455,9 @@ int itcpd_random_factors(int32_t order, const int64_t* dims, int64_t rank, uint6
     int rc;
     hipError_t e = hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking);
     if (e != hipSuccess) return bail(hip_fail(e, "hipStreamCreate"));
-    if ((rc = alloc_factor_state(p))) return bail(rc);
+    Arena ar;
+    factor_state(p, ar);
+    if ((rc = alloc_arena(p, ar))) return bail(rc);
     if ((rc = launch_random_init(p, seed))) return bail(rc);
     p->have_cpd = true;
     rc = itcpd_get_cpd(p, factors, lambda, mem);
@@ -450,6 +469,15 @@ int itcpd_get_cpd(itcpd_plan* p, double* const* factors, double* lambda, int32_t
     if (!p->have_cpd) return fail(ITCPD_E_STATE, "no CPD set on this plan");
     DeviceGuard dg(p->device);
     int rc;
+    if (char* const stage = mem == ITCPD_MEM_HOST && factors ? cpd_stage(p) : nullptr) {
+        if ((rc = copy_out(stage, p->arena, p->cpd_bytes, mem, p->stream))) return rc;
+        ITCPD_HIP(hipStreamSynchronize(p->stream));
+        for (int m = 0; m < p->N; ++m)
+            if (factors[m])
+                std::memcpy(factors[m], stage + ((char*)p->A[m] - p->arena), (size_t)(p->dims[m] * p->R) * 8);
+        if (lambda) std::memcpy(lambda, stage + ((char*)p->lam - p->arena), (size_t)p->R * 8);
+        return ITCPD_OK;
+    }
     for (int m = 0; factors && m < p->N; ++m) {
         if (!factors[m]) continue;
         if ((rc = copy_out(factors[m], p->A[m], (size_t)p->dims[m] * p->R * 8, mem, p->stream)))
@@ -502,11 +530,16 @@ int itcpd_run(itcpd_plan* p, itcpd_check* c, double* fit_trace) {
         p->tree3 = false;
     }
     if (nsweeps > p->trace_cap) {
-        dfree(p->fit_trace);
-        p->fit_trace = nullptr;
+        dfree(p->trace_owned);
+        p->trace_owned = nullptr;
+        const int rc = dmalloc(&p->trace_owned, (size_t)nsweeps);
+        if (rc) {
+            p->trace_cap = 0;
+            p->fit_trace = nullptr;
+            return rc;
+        }
+        p->fit_trace = p->trace_owned;
         p->trace_cap = (int)nsweeps;
-        int rc = dmalloc(&p->fit_trace, (size_t)p->trace_cap);
-        if (rc) return rc;
     }
     DevCheck* h = p->chk_host;
     std::memset(h, 0, sizeof(DevCheck));
@@ -525,8 +558,8 @@ int itcpd_run(itcpd_plan* p, itcpd_check* c, double* fit_trace) {
         h->has_prev = c->has_prev ? 1 : 0;
     }
     p->check_kind = c->kind;
+    // h is written again only by the copy back at the run's end, behind this one on the stream
     ITCPD_HIP(hipMemcpyAsync(p->chk, h, sizeof(DevCheck), hipMemcpyHostToDevice, p->stream));
-    ITCPD_HIP(hipStreamSynchronize(p->stream));
 
     // FitCheck: every POLL_EVERY sweeps a snapshot of the device check state is
     // copied to a pinned slot behind an event.  The host keeps enqueueing and

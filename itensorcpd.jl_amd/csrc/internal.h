@@ -111,7 +111,12 @@ struct itcpd_plan {
     int64_t maxI = 0;
     bool have_cpd = false;
 
-    // device state
+    // device state: one allocation (arena), the CPD (factors, lambda) at its start
+    char* arena = nullptr;
+    size_t cpd_bytes = 0, zero_bytes = 0;
+    char* stage = nullptr;                     // pinned mirror of the CPD region (made on first use)
+    bool stage_failed = false;
+    double* trace_owned = nullptr;             // fit trace of a run longer than the arena's
     double* A[ITCPD_MAX_ORDER] = {nullptr};    // I_n x Rp column-major (zero beyond R)
     double* At[ITCPD_MAX_ORDER] = {nullptr};   // Rp x I_n (rank fastest, zero beyond R)
     double* G[ITCPD_MAX_ORDER] = {nullptr};    // R x R
@@ -226,6 +231,7 @@ int launch_solve(itcpd_plan* p, int mode, const double* Msrc, int nparts, int64_
                  bool finalize, bool fit_after, int next_factor = -1);
 int launch_normalize(itcpd_plan* p, int mode, const double* Xsrc, bool fit_after);
 int launch_seed_grams(itcpd_plan* p);
+int launch_reset_flags(itcpd_plan* p);         // chk->done = chk->nan_flag = 0
 int launch_random_init(itcpd_plan* p, uint64_t seed);
 int launch_fit_only(itcpd_plan* p, const double* Mlast, double ref_norm);
 int launch_hadamard(itcpd_plan* p, int mode, double* V);

@@ -1542,6 +1542,16 @@ int launch_seed_grams(itcpd_plan* p) {
     return ITCPD_OK;
 }
 
+__global__ void k_reset_flags(DevCheck* __restrict__ chk) {
+    chk->done = 0;
+    chk->nan_flag = 0;
+}
+int launch_reset_flags(itcpd_plan* p) {
+    hipLaunchKernelGGL(k_reset_flags, dim3(1), dim3(1), 0, p->stream, p->chk);
+    ITCPD_HIP(hipGetLastError());
+    return ITCPD_OK;
+}
+
 // random_factors (cpd.jl:48-60): draw, row_norm, lambda from the last mode.
 int launch_random_init(itcpd_plan* p, uint64_t seed) {
     const int R = (int)p->R;
