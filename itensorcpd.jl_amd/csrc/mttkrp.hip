@@ -283,70 +283,69 @@ __global__ __launch_bounds__(512, 1) void k_lp_ring(const float* __restrict__ T,
 // M(i, r) = sum_{a<A, b<B} P(a + A*i + A*In*b, r) * Wa(a, r) * Wb(b, r)
 // Wa = product over the side's modes before `pos`, Wb over the modes after it
 // (column-major factors).  P has leading dimension MS.
-__device__ __forceinline__ double w_after(const Side& sd, int pos, int64_t b, int r) {
-    double w = 1.0;
-    int64_t t = b;
-    for (int q = pos + 1; q < sd.nm; ++q) {
-        const int64_t d = t % sd.dim[q];
-        t /= sd.dim[q];
-        w *= sd.fac[q][d + sd.dim[q] * r];
+// w[k] *= the product over the side's modes [q0, q1) at the flattened index x[k] (x is used
+// up), mode by mode so that the U loads of one are in flight together.
+template <int U, typename I>
+__device__ __forceinline__ void side_weights(const Side& sd, int q0, int q1, int r, I (&x)[U], double (&w)[U]) {
+    for (int q = q0; q < q1; ++q) {
+        const I d = (I)sd.dim[q];
+        const double* __restrict__ f = sd.fac[q] + sd.dim[q] * r;
+        double fv[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const I t = q + 1 < q1 ? x[k] / d : (I)0;
+            fv[k] = f[x[k] - t * d];
+            x[k] = t;
+        }
+#pragma unroll
+        for (int k = 0; k < U; ++k) w[k] *= fv[k];
     }
-    return w;
-}
-__device__ __forceinline__ double w_before(const Side& sd, int pos, int64_t a, int r) {
-    double w = 1.0;
-    int64_t t = a;
-    for (int q = 0; q < pos; ++q) {
-        const int64_t d = t % sd.dim[q];
-        t /= sd.dim[q];
-        w *= sd.fac[q][d + sd.dim[q] * r];
-    }
-    return w;
 }
 
-// The side's fastest mode: thread per (i, r), split over b.
+// The side's fastest mode: thread per (i, r), split over b; 8 steps of b in flight.  Bound by
+// HBM when large (512 x 512 x 64: 32 us, 4.2 TB/s).  When small, by the factorisation in the
+// same launch: In = 20, B = 342, R = 24 takes 11.1 us, 14.1 with the steps one by one.
+template <typename I>
 __global__ __launch_bounds__(256) void k_ttv_lead(const double* __restrict__ P, int64_t MS,
-                                                  int64_t In, int R, Side sd, int pos, int64_t B,
-                                                  int64_t b_per_split, double* __restrict__ out,
-                                                  int64_t split_stride, FactorJob fj,
-                                                  const DevCheck* __restrict__ chk) {
+                                                  int64_t In, int R, Side sd, I B, I b_per_split,
+                                                  double* __restrict__ out, int64_t split_stride,
+                                                  FactorJob fj, const DevCheck* __restrict__ chk) {
     if (factor_block(fj)) return;
     if (chk->done) return;
     const int64_t idx = ((int64_t)blockIdx.x - (fj.on ? 1 : 0)) * 256 + threadIdx.x;
     if (idx >= In * R) return;
     const int64_t i = idx % In;
     const int r = (int)(idx / In);
-    const int64_t b0 = (int64_t)blockIdx.y * b_per_split;
-    const int64_t b1 = b0 + b_per_split < B ? b0 + b_per_split : B;
+    const I b0 = (I)blockIdx.y * b_per_split;
+    const I b1 = b0 + b_per_split < B ? b0 + b_per_split : B;
     const double* __restrict__ Pc = P + MS * r + i;
     double sum = 0.0;
-    if (sd.nm - pos - 1 == 1) {
-        const double* __restrict__ f = sd.fac[pos + 1] + sd.dim[pos + 1] * r;
-        int64_t b = b0;
-        for (; b + 8 <= b1; b += 8) {
-            double pv[8], fv[8];
+    for (I b = b0; b < b1; b += 8) {
+        I x[8];
+        double pv[8], w[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                pv[k] = Pc[In * (b + k)];
-                fv[k] = f[b + k];
-            }
-#pragma unroll
-            for (int k = 0; k < 8; ++k) sum += pv[k] * fv[k];
+        for (int k = 0; k < 8; ++k) {   // past the end: a valid element, not added
+            x[k] = b + k < b1 ? b + k : b1 - 1;
+            pv[k] = Pc[In * x[k]];
+            w[k] = 1.0;
         }
-        for (; b < b1; ++b) sum += Pc[In * b] * f[b];
-    } else {
-        for (int64_t b = b0; b < b1; ++b) sum += Pc[In * b] * w_after(sd, pos, b, r);
+        side_weights<8, I>(sd, 1, sd.nm, r, x, w);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (b + k < b1) sum += pv[k] * w[k];
     }
     out[(int64_t)blockIdx.y * split_stride + i + In * r] = sum;
 }
 
-// The other modes: one wave per JW consecutive i of one r; lanes stride over a (contiguous in
-// P), with the JW rows' loads in flight together.  Each output keeps the order of
-// its sum for any JW (per lane over a, then over b, then the wave reduction).
-template <int JW>
+// The other modes: one wave per JW consecutive i of one r; lanes stride over the flattened
+// (a, b) with U steps and the JW rows' loads in flight together, and share the weights over
+// the rows.  Bound as k_ttv_lead (512 x 512 x 64: 30 us).  Lanes over a alone, b one by one,
+// left most lanes idle behind one load at a time where A is short: A = 20, In = 19, B = 18,
+// R = 24 took 18.6 us, now 10.8 with its factorisation.
+template <int JW, int U, typename I>
 __global__ __launch_bounds__(256) void k_ttv_inner(const double* __restrict__ P, int64_t MS,
-                                                   int64_t In, int R, Side sd, int pos, int64_t A,
-                                                   int64_t B, double* __restrict__ out, FactorJob fj,
+                                                   int64_t In, int R, Side sd, int pos, I A, I B,
+                                                   double* __restrict__ out, FactorJob fj,
                                                    const DevCheck* __restrict__ chk) {
     if (factor_block(fj)) return;
     if (chk->done) return;
@@ -356,58 +355,41 @@ __global__ __launch_bounds__(256) void k_ttv_inner(const double* __restrict__ P,
     if (wid >= ngi * R) return;
     const int64_t i0 = (wid % ngi) * JW;
     const int r = (int)(wid / ngi);
-    bool ok[JW];
-#pragma unroll
-    for (int jj = 0; jj < JW; ++jj) ok[jj] = i0 + jj < In;
+    const double* __restrict__ Pr[JW];   // rows past the end read the last one
     double sum[JW];
 #pragma unroll
-    for (int jj = 0; jj < JW; ++jj) sum[jj] = 0.0;
-    const bool one_before = (pos == 1);
-    const double* __restrict__ f0 = sd.fac[0] + sd.dim[0] * r;
-    for (int64_t b = 0; b < B; ++b) {
-        const double wb = w_after(sd, pos, b, r);
-        const double* __restrict__ Pc = P + MS * r + A * i0 + A * In * b;
-        double part[JW];
+    for (int j = 0; j < JW; ++j) {
+        Pr[j] = P + MS * r + (int64_t)A * (i0 + j < In ? i0 + j : In - 1);
+        sum[j] = 0.0;
+    }
+    const I n = A * B;
+    const int64_t skip = (int64_t)A * (In - 1);   // x = a + A b is at x + skip b
+    for (I x0 = lane; x0 < n; x0 += 64 * U) {
+        I xa[U], xb[U];
+        double w[U], pv[JW][U];
 #pragma unroll
-        for (int jj = 0; jj < JW; ++jj) part[jj] = 0.0;
-        if (one_before) {
-            int64_t a = lane;
-            for (; a + 64 * 7 < A; a += 64 * 8) {
-                double fv[8], pv[JW][8];
+        for (int k = 0; k < U; ++k) {
+            const I x = x0 + 64 * k < n ? x0 + 64 * k : n - 1;
+            xb[k] = B > 1 ? x / A : (I)0;
+            xa[k] = x - xb[k] * A;
+            const int64_t off = x + skip * xb[k];
 #pragma unroll
-                for (int k = 0; k < 8; ++k) fv[k] = f0[a + 64 * k];
-#pragma unroll
-                for (int jj = 0; jj < JW; ++jj)
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) pv[jj][k] = ok[jj] ? Pc[A * jj + a + 64 * k] : 0.0;
-#pragma unroll
-                for (int jj = 0; jj < JW; ++jj)
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) part[jj] += pv[jj][k] * fv[k];
-            }
-            for (; a < A; a += 64) {
-                const double f = f0[a];
-#pragma unroll
-                for (int jj = 0; jj < JW; ++jj)
-                    if (ok[jj]) part[jj] += Pc[A * jj + a] * f;
-            }
-        } else {
-            for (int64_t a = lane; a < A; a += 64) {
-                const double wa = w_before(sd, pos, a, r);
-#pragma unroll
-                for (int jj = 0; jj < JW; ++jj)
-                    if (ok[jj]) part[jj] += Pc[A * jj + a] * wa;
-            }
+            for (int j = 0; j < JW; ++j) pv[j][k] = Pr[j][off];
+            w[k] = 1.0;
         }
+        side_weights<U, I>(sd, 0, pos, r, xa, w);
+        side_weights<U, I>(sd, pos + 1, sd.nm, r, xb, w);
 #pragma unroll
-        for (int jj = 0; jj < JW; ++jj) sum[jj] += part[jj] * wb;
+        for (int k = 0; k < U; ++k)
+            if (x0 + 64 * k < n) {
+#pragma unroll
+                for (int j = 0; j < JW; ++j) sum[j] += pv[j][k] * w[k];
+            }
     }
 #pragma unroll
-    for (int jj = 0; jj < JW; ++jj) {
-        double v = sum[jj];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-        if (lane == 0 && ok[jj]) out[i0 + jj + In * r] = v;
+    for (int j = 0; j < JW; ++j) {
+        const double v = wave_sum_dpp(sum[j]);
+        if (lane == 0 && i0 + j < In) out[i0 + j + In * r] = v;
     }
 }
 
@@ -1270,6 +1252,7 @@ static int launch_ttv(itcpd_plan* p, const double* P, int64_t MS, const Side& sd
     const int64_t nout = In * p->R;
     const FactorJob fj = factor_job_for(p, factor_mode);
     const size_t lds = fj.on ? FACTOR64_LDS : 0;
+    const bool small = A * B < ((int64_t)1 << 30);   // 32-bit digits
     int rc = ITCPD_OK;
     if (pos == 0) {
         int64_t nz = 1;
@@ -1280,15 +1263,23 @@ static int launch_ttv(itcpd_plan* p, const double* P, int64_t MS, const Side& sd
         const int64_t bper = cdiv(B, nz);
         nz = cdiv(B, bper);
         double* out = nz > 1 ? p->parts : p->M;
-        hipLaunchKernelGGL(k_ttv_lead, dim3((unsigned)(blocks + fj.on), (unsigned)nz), dim3(256), lds, p->stream,
-                           P, MS, In, (int)p->R, sd, pos, B, bper, out, nout, fj, p->chk);
+        const dim3 grid((unsigned)(blocks + fj.on), (unsigned)nz);
+        if (small)
+            hipLaunchKernelGGL(k_ttv_lead<int>, grid, dim3(256), lds, p->stream, P, MS, In, (int)p->R, sd, (int)B,
+                               (int)bper, out, nout, fj, p->chk);
+        else
+            hipLaunchKernelGGL(k_ttv_lead<int64_t>, grid, dim3(256), lds, p->stream, P, MS, In, (int)p->R, sd, B,
+                               bper, out, nout, fj, p->chk);
         ITCPD_HIP(hipGetLastError());
         rc = finish_parts(p, p->parts, nz, nout, p->M, ms, true);
     } else {
-        constexpr int JW = 4;
-        const int64_t waves = cdiv(In, JW) * p->R;
-        hipLaunchKernelGGL(k_ttv_inner<JW>, dim3((unsigned)(cdiv(waves, 4) + fj.on)), dim3(256), lds, p->stream, P,
-                           MS, In, (int)p->R, sd, pos, A, B, p->M, fj, p->chk);
+        auto run = [&](auto kern, int jw, auto a, auto b) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)(cdiv(cdiv(In, jw) * p->R, 4) + fj.on)), dim3(256), lds,
+                               p->stream, P, MS, In, (int)p->R, sd, pos, a, b, p->M, fj, p->chk);
+        };
+        if (!small) run(k_ttv_inner<4, 4, int64_t>, 4, A, B);
+        else if (A * B <= 128) run(k_ttv_inner<4, 2, int>, 4, (int)A, (int)B);
+        else run(k_ttv_inner<4, 4, int>, 4, (int)A, (int)B);
         ITCPD_HIP(hipGetLastError());
         *ms = MSrc{p->M, 1, nout};
     }

@@ -1355,12 +1355,12 @@ int solve_nb(int64_t In, int R) {
     const int64_t nb = cdiv(In, R <= 64 ? 16 : rpb_of(R));
     return (int)(nb < cap ? nb : cap);
 }
-// R <= 64: 32 rows a block, at most 16.  Above, also 256 Gram entries a block (one per
-// thread), at most 128 blocks: 7.9 us at R = 128, I = 224 (45 us with 7 blocks and 56 partials).
+// 32 rows and 256 Gram entries (one per thread) a block, which is k_finalize_1rt's form while
+// the partials are few; at most 16 blocks for R <= 64, 128 above.  Measured: R = 24, I = 20
+// 5.2 us (5.8 with one block); R = 128, I = 224 with 64 blocks 7.9 us (45 with 7 blocks and
+// 56 partials).
 int finalize_nb(int64_t In, int R) {
-    const int64_t nb = cdiv(In, 32);
-    if (R > 64) return (int)std::min<int64_t>(128, std::max(nb, cdiv((int64_t)R * R, 256)));
-    return (int)(nb < 16 ? (nb < 1 ? 1 : nb) : 16);
+    return (int)std::min<int64_t>(R > 64 ? 128 : 16, std::max(cdiv(In, 32), cdiv((int64_t)R * R, 256)));
 }
 
 // Row ranges of the Gram products: one up to 2048 rows, at most 64 (and within gram_part).
