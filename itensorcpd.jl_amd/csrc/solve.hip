@@ -738,6 +738,16 @@ __global__ __launch_bounds__(256) void k_finalize_1rt(const double* __restrict__
     }
 }
 
+// NoCheck's state after a sweep.
+__device__ __forceinline__ void count_sweep(DevCheck* chk) {
+    chk->iter += 1;
+    chk->sweeps += 1;
+    if (chk->iter == chk->max_counter) {
+        chk->iter = 0;
+        chk->done = 1;
+    }
+}
+
 // After the last mode of a sweep: the fit from <T,X> (sum of the finalize blocks'
 // partials, fixed order) and ||X||^2 = lambda^T (G_0 .* ... .* G_{N-1}) lambda, then
 // the check update (FitCheck) or the sweep count (NoCheck).
@@ -749,14 +759,7 @@ __global__ __launch_bounds__(256) void k_fit(const double* __restrict__ inner_pa
     __shared__ double red[256];
     const int t = threadIdx.x;
     if (chk->kind == ITCPD_CHECK_NONE) {
-        if (t == 0) {
-            chk->iter += 1;
-            chk->sweeps += 1;
-            if (chk->iter == chk->max_counter) {
-                chk->iter = 0;
-                chk->done = 1;
-            }
-        }
+        if (t == 0) count_sweep(chk);
         return;
     }
     double fs = 0.0;
@@ -790,6 +793,197 @@ __global__ __launch_bounds__(256) void k_fit(const double* __restrict__ inner_pa
     if (t == 0) {
         const double inner = sum_parts_at(inner_part, 1, nbf, 0);
         check_update(chk, inner, fact_square, scal, trace, trace_cap);
+    }
+}
+
+// The whole update of a short mode in one workgroup, R <= RT <= 32: row solve, Gram, row_norm
+// and after the last mode the fit.  Wave w takes rows 16w..16w+15 with their tile of X in
+// registers throughout: as the product's result it is both operands of X^T X (k0 = 4v), so
+// only the waves' Gram tiles meet in LDS.  Otherwise the same as k_solve_mfma, k_finalize and
+// k_fit, whose launches cost more than their work here.
+template <int RT>
+__global__ __launch_bounds__(RT == 16 ? 1024 : 512) void k_update_small(
+    const double* __restrict__ Msrc, int nparts, int64_t pstride, int In, int R, int Rp,
+    const double* __restrict__ Vinv, const int* __restrict__ finfo, const double* __restrict__ W,
+    const double* __restrict__ qtau, const double* __restrict__ ztau, const int* __restrict__ jpvt, double* X,
+    double* __restrict__ A, double* __restrict__ At, double* __restrict__ lam, double* __restrict__ Gout,
+    int mode, GramSet gs, int fit, double* __restrict__ scal, DevCheck* __restrict__ chk,
+    double* __restrict__ trace, int trace_cap) {
+    constexpr int NT = RT / 16, KS = RT / 4, NP = NT * (NT + 1) / 2, LDS_ = RT + 1, NH = RT * RT / 256;
+    __shared__ double part[(RT == 16 ? 16 : 8) * NP * 256];
+    __shared__ double S[RT * LDS_];
+    __shared__ double lamS[RT];
+    __shared__ double red[32];
+    const int t = threadIdx.x, nthr = blockDim.x, l = t & 63, c = l & 15, g = l >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nt = (In + 15) / 16;
+    const bool active = w < nt;
+    // every load of the usual path is requested before the first wait
+    const int done = chk->done, kind = chk->kind, gfb = finfo[1];
+    const bool want_fit = fit && kind != ITCPD_CHECK_NONE;
+    const int ia = 16 * w + c;
+    auto sum_m = [&](int row, int k) {   // M(row, k): the partials in increasing order
+        const bool ok = row < In && k < R;
+        const double* src = Msrc + (ok ? row + (int64_t)In * k : 0);
+        double v = src[0];
+        for (int b = 1; b < nparts; ++b) v += src[b * pstride];
+        return ok ? v : 0.0;
+    };
+    double av[KS], bv[NT][KS], md[NT][4], h[NH];
+    d4 acc[NT];
+#pragma unroll
+    for (int tb = 0; tb < NT; ++tb) acc[tb] = (d4){0.0, 0.0, 0.0, 0.0};
+    if (active) {
+        const double* src[KS];
+        bool ok[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int k = 4 * ks + g;
+            ok[ks] = ia < In && k < R;
+            src[ks] = Msrc + (ok[ks] ? ia + (int64_t)In * k : 0);
+            av[ks] = src[ks][0];
+#pragma unroll
+            for (int tb = 0; tb < NT; ++tb) {
+                const int col = 16 * tb + c;
+                const double v = Vinv[k < R && col < R ? k * R + col : 0];
+                bv[tb][ks] = k < R && col < R ? v : 0.0;
+            }
+        }
+        int b = 1;
+        for (; b + 4 <= nparts; b += 4) {
+            double v[KS][4];
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int z = 0; z < 4; ++z) v[ks][z] = src[ks][(b + z) * pstride];
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int z = 0; z < 4; ++z) av[ks] += v[ks][z];
+        }
+        for (; b < nparts; ++b)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) av[ks] += src[ks][b * pstride];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) av[ks] = ok[ks] ? av[ks] : 0.0;
+    }
+    if (want_fit) {
+#pragma unroll
+        for (int q = 0; q < NH; ++q) h[q] = 1.0;
+        for (int m = 0; m < gs.N; ++m) {
+            if (m == mode) continue;
+#pragma unroll
+            for (int q = 0; q < NH; ++q) {
+                const int x = t + nthr * q;
+                h[q] *= gs.G[m][x < R * R ? x : 0];
+            }
+        }
+#pragma unroll
+        for (int tb = 0; tb < NT; ++tb)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) md[tb][v] = active ? sum_m(16 * w + g + 4 * v, 16 * tb + c) : 0.0;
+    }
+    if (done) return;
+    if (!gfb) {
+        if (active) {
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int tb = 0; tb < NT; ++tb) acc[tb] = mfma_f64(av[ks], bv[tb][ks], acc[tb]);
+        }
+    } else {   // QR fallback, row by row: lane k holds column k; then the tile as above
+        const int rk = finfo[2], pk = l < R ? jpvt[l] : 0;
+        for (int rr = 0; rr < 16; ++rr) {
+            const int row = 16 * w + rr;
+            if (row >= In) break;
+            double y[1] = {sum_m(row, l)};
+            fallback_apply<1>(y, l, R, rk, W, qtau, ztau);
+            if (l < R) X[row + (int64_t)In * pk] = y[0];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int tb = 0; tb < NT; ++tb)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int row = 16 * w + g + 4 * v, col = 16 * tb + c;
+                acc[tb][v] = row < In && col < R ? X[row + (int64_t)In * col] : 0.0;
+            }
+    }
+    if (active) {   // rows >= In and columns >= R of acc are zero
+        d4 ga[NP];
+#pragma unroll
+        for (int q = 0; q < NP; ++q) ga[q] = (d4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int tb = 0, q = 0; tb < NT; ++tb)
+#pragma unroll
+                for (int ta = 0; ta <= tb; ++ta, ++q) ga[q] = mfma_f64(acc[ta][v], acc[tb][v], ga[q]);
+#pragma unroll
+        for (int q = 0; q < NP; ++q)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) part[(w * NP + q) * 256 + 64 * v + l] = ga[q][v];
+    }
+    __syncthreads();
+    for (int x = t; x < NP * 256; x += nthr) {
+        double s = 0.0;
+        for (int k = 0; k < nt; ++k) s += part[k * NP * 256 + x];
+        const int q = x >> 8, tb = q > 0, ta = q > 1;   // tiles (0, 0), (0, 1), (1, 1)
+        const int r = 16 * ta + ((x >> 4) & 3) + 4 * ((x >> 6) & 3), r2 = 16 * tb + (x & 15);
+        S[r * LDS_ + r2] = s;
+        if (ta != tb) S[r2 * LDS_ + r] = s;
+    }
+    __syncthreads();
+    if (t < R) {
+        lamS[t] = sqrt(S[t * LDS_ + t]);
+        lam[t] = lamS[t];
+    }
+    __syncthreads();
+    double fs = 0.0, inner = 0.0;
+#pragma unroll
+    for (int q = 0; q < NH; ++q) {
+        const int x = t + nthr * q;
+        if (x >= R * R) continue;
+        const int r = x % R, r2 = x / R;
+        const double ll = lamS[r] * lamS[r2], gx = S[r * LDS_ + r2] / ll;
+        Gout[x] = gx;
+        if (want_fit) fs += h[q] * gx * ll;
+    }
+    if (active) {
+#pragma unroll
+        for (int tb = 0; tb < NT; ++tb) {
+            const int col = 16 * tb + c;
+            if (col >= R) continue;
+            const double lc = lamS[col];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int row = 16 * w + g + 4 * v;
+                if (row >= In) continue;
+                const double a = acc[tb][v] / lc;
+                A[row + (int64_t)In * col] = a;
+                At[(int64_t)row * Rp + col] = a;
+                if (want_fit) inner += md[tb][v] * (a * lc);
+            }
+        }
+    }
+    if (!fit) return;
+    if (want_fit) {
+        fs = wave_sum_dpp(fs);
+        inner = wave_sum_dpp(inner);
+        if (l == 0) {
+            red[w] = fs;
+            red[16 + w] = inner;
+        }
+        __syncthreads();
+        if (t == 0) {
+            for (int k = 1; k < nthr / 64; ++k) {
+                fs += red[k];
+                inner += red[16 + k];
+            }
+            check_update(chk, inner, fs, scal, trace, trace_cap);
+        }
+    } else if (t == 0) {
+        count_sweep(chk);
     }
 }
 
@@ -1008,14 +1202,7 @@ __global__ __launch_bounds__(256) void k_gram_final(const double* __restrict__ g
     __threadfence_block();
     __syncthreads();
     if (chk->kind == ITCPD_CHECK_NONE) {
-        if (t == 0) {
-            chk->iter += 1;
-            chk->sweeps += 1;
-            if (chk->iter == chk->max_counter) {
-                chk->iter = 0;
-                chk->done = 1;
-            }
-        }
+        if (t == 0) count_sweep(chk);
         return;
     }
     // ||X||^2 = lambda^T (G_0 .* ... .* G_{N-1}) lambda   (converge_checks.jl:5-11)
@@ -1425,6 +1612,26 @@ int run_apply(itcpd_plan* p, int mode, const double* Msrc, int nparts, int64_t s
     return run_solve_k<16>(p, mode, Msrc);
 }
 
+// One workgroup for the whole update: while its matrix products (In RT) and M's partials
+// through one CU stay below what the separate launches cost.
+bool update_small_ok(const itcpd_plan* p, int mode, int nparts) {
+    const int64_t In = p->dims[mode];
+    return p->RT && p->RT <= 32 && In * p->RT <= 4096 && In * p->R * nparts <= ((int64_t)1 << 15);
+}
+template <int RT>
+int run_update_small(itcpd_plan* p, int mode, const double* Msrc, int nparts, int64_t stride, bool fit) {
+    const int64_t In = p->dims[mode];
+    const int R = (int)p->R;
+    double* W = p->qr_aux;
+    hipLaunchKernelGGL((k_update_small<RT>), dim3(1), dim3(64 * std::max<unsigned>(4, (unsigned)cdiv(In, 16))), 0,
+                       p->stream, Msrc, nparts, stride, (int)In, R, (int)p->Rp, p->Upad, p->finfo, W,
+                       W + (size_t)R * R, W + (size_t)R * R + R, (const int*)(p->piv + R), p->X, p->A[mode],
+                       p->At[mode], p->lam, p->G[mode], mode, grams_of(p), fit ? 1 : 0, p->scal, p->chk,
+                       p->fit_trace, p->trace_cap);
+    ITCPD_HIP(hipGetLastError());
+    return ITCPD_OK;
+}
+
 }  // namespace
 
 int launch_solve(itcpd_plan* p, int mode, const double* Msrc, int nparts, int64_t stride,
@@ -1439,6 +1646,13 @@ int launch_solve(itcpd_plan* p, int mode, const double* Msrc, int nparts, int64_
         nparts = 1;
     }
     const bool cp_check = p->check_kind == ITCPD_CHECK_CPDIFF || p->check_kind == ITCPD_CHECK_CPANGLE;
+    if (finalize && update_small_ok(p, mode, nparts)) {
+        const bool fit = fit_after && !cp_check;
+        rc = p->RT == 16 ? run_update_small<16>(p, mode, Msrc, nparts, stride, fit)
+                         : run_update_small<32>(p, mode, Msrc, nparts, stride, fit);
+        if (!rc && fit_after && cp_check) rc = launch_cp_check(p);
+        return rc || next_factor < 0 ? rc : launch_factor(p, next_factor);
+    }
     rc = run_apply(p, mode, Msrc, nparts, stride, finalize, fit_after);
     if (rc || !finalize) return rc;
     const int64_t In = p->dims[mode];
