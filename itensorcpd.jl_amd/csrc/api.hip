@@ -455,6 +455,7 @@ int itcpd_random_factors(int32_t order, const int64_t* dims, int64_t rank, uint6
     int rc;
     hipError_t e = hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking);
     if (e != hipSuccess) return bail(hip_fail(e, "hipStreamCreate"));
+    p->stage_failed = true;   // one transfer: a pinned mirror costs more than it saves
     Arena ar;
     factor_state(p, ar);
     if ((rc = alloc_arena(p, ar))) return bail(rc);
@@ -744,15 +745,18 @@ int itcpd_sampled_solve(itcpd_plan* p, int32_t mode, int64_t nsamps, const int32
         ++q;
     }
     ITCPD_HIP(hipMemcpyAsync(p->smp_iws, h.data(), nidx * 4, hipMemcpyHostToDevice, p->stream));
-    if ((rc = launch_sampled_solve(p, mode, nsamps, p->smp_iws, normal != 0))) return rc;
-    if ((rc = launch_col_sumsq(p, mode, p->X))) return rc;
-    if ((rc = launch_normalize(p, mode, p->X, false))) return rc;
+    if ((rc = launch_sampled_gather(p, mode, nsamps, p->smp_iws))) return rc;
+    int form = normal ? SAMPLED_NORMAL : (sampled_corrected_ok(p, nsamps) ? SAMPLED_CORRECTED : SAMPLED_QR);
     int fi[4] = {0, 0, 0, 0};
-    if (normal)
-        ITCPD_HIP(hipMemcpyAsync(fi, p->finfo, sizeof(fi), hipMemcpyDeviceToHost, p->stream));
-    else
-        ITCPD_HIP(hipMemcpyAsync(fi, p->smp_iws + nidx + p->R, sizeof(int), hipMemcpyDeviceToHost, p->stream));
-    ITCPD_HIP(hipStreamSynchronize(p->stream));
+    for (;;) {
+        if ((rc = launch_sampled_solve(p, mode, nsamps, form))) return rc;
+        if (!normal && (rc = launch_row_norm(p, mode))) return rc;
+        ITCPD_HIP(hipMemcpyAsync(fi, normal ? p->finfo : p->smp_iws + nidx + p->R, sizeof(fi), hipMemcpyDeviceToHost,
+                                 p->stream));
+        ITCPD_HIP(hipStreamSynchronize(p->stream));
+        if (form != SAMPLED_CORRECTED || fi[1] == 0) break;
+        form = SAMPLED_QR;   // not certified: the update is made again from the QR
+    }
     if (info) {
         info[0] = normal ? fi[1] : 0;            // the Cholesky fell back to the QR solve
         info[1] = normal ? fi[2] : fi[0];        // rank of the solve

@@ -187,7 +187,7 @@ __device__ __forceinline__ bool sweep_inverse(double (&a)[16], int n, int grp, i
 // It stands in for the pivoted factorisation (xPSTRF, absolute tolerance tol) only
 // when that one provably keeps every pivot: each pivoted pivot is a diagonal entry
 // of a Schur complement of V, hence >= lambda_min(V), and lambda_min(V) >=
-// 1 / ||V^-1||_F.  The computed inverse is trusted while ||V||_F ||V^-1||_F < 1e12;
+// 1 / ||V^-1||_F.  The computed inverse is trusted while ||V||_F ||V^-1||_F < cond_max;
 // the bound must exceed 2 tol plus the pivots' rounding (64 R eps max V_ii); every
 // unpivoted pivot must be > 0.  Then the solution (the unique minimiser) is the
 // pivoted path's up to rounding, and V^-1 and finfo are written; otherwise it returns
@@ -201,7 +201,7 @@ __device__ __forceinline__ bool sweep_inverse(double (&a)[16], int n, int grp, i
 // 14, 17 and 28.
 __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, int R, double tol,
                                                    double* __restrict__ Vinv, int* __restrict__ finfo,
-                                                   double* S) {
+                                                   double* S, double cond_max = 1e12) {
     double* red = S + SWEEP_ROWS;   // behind the broadcast rows
     const int t = threadIdx.x, l = t & 63;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -267,7 +267,7 @@ __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, 
         }
     const double vF = sqrt(vs), zF = sqrt(zs);
     const bool cert = red[12] == 0.0 && zF > 0.0 && zF < __builtin_inf() &&
-                      1.0 / zF > 2.0 * tol + 64.0 * R * 0x1p-52 * dmax && vF * zF < 1e12;
+                      1.0 / zF > 2.0 * tol + 64.0 * R * 0x1p-52 * dmax && vF * zF < cond_max;
     if (cert && t == 0) {
         finfo[0] = R;
         finfo[1] = 0;

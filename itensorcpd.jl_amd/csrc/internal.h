@@ -230,6 +230,7 @@ int launch_cp_check(itcpd_plan* p);
 int launch_solve(itcpd_plan* p, int mode, const double* Msrc, int nparts, int64_t stride,
                  bool finalize, bool fit_after, int next_factor = -1);
 int launch_normalize(itcpd_plan* p, int mode, const double* Xsrc, bool fit_after);
+int launch_row_norm(itcpd_plan* p, int mode);   // (A_n, lambda) and G_n from p->X
 int launch_seed_grams(itcpd_plan* p);
 int launch_reset_flags(itcpd_plan* p);         // chk->done = chk->nan_flag = 0
 int launch_random_init(itcpd_plan* p, uint64_t seed);
@@ -239,7 +240,11 @@ int launch_col_sumsq(itcpd_plan* p, int mode, const double* X);
 // leverage-score-sampled ALS (sampled.hip)
 int launch_leverage_scores(itcpd_plan* p, int mode, double* probs_dev, double** probs_used);
 int sampled_ws_prepare(itcpd_plan* p, int mode, int64_t ns);
-int launch_sampled_solve(itcpd_plan* p, int mode, int64_t ns, const int* samples, bool normal);
+// form: the normal equations, the column-pivoted QR, or corrected normal equations in its place
+enum { SAMPLED_NORMAL, SAMPLED_QR, SAMPLED_CORRECTED };
+bool sampled_corrected_ok(const itcpd_plan* p, int64_t ns);
+int launch_sampled_gather(itcpd_plan* p, int mode, int64_t ns, const int* samples);
+int launch_sampled_solve(itcpd_plan* p, int mode, int64_t ns, int form);
 int launch_qr_pivots(itcpd_plan* p, int mode, bool krp, const int64_t* cols, int64_t ncols,
                      const int64_t* omega_rowptr, const int64_t* omega_cols, const double* omega_vals, int64_t l,
                      int* jpvt_dev, double* rdiag_dev);

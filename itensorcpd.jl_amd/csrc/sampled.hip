@@ -15,6 +15,7 @@
 // incremental condition estimation at rcond = min(m, n) eps, RZ reduction of the
 // trapezoid, minimum-norm solution) in one workgroup.
 #include "dense_la.h"
+#include "factor64.h"
 #include "internal.h"
 
 namespace itcpd {
@@ -78,6 +79,224 @@ __global__ __launch_bounds__(256) void k_gemm_tn(const double* __restrict__ A, c
     for (int64_t k = lane; k < ns; k += 64) s = fma(a[k], b[k], s);
     s = wave_sum(s);
     if (lane == 0) C[i + (int64_t)m * j] = s;
+}
+
+// A 16-sample chunk of a column over the four lanes g: value q is sample chunk_at(g, q), so
+// that each of the two 16-byte loads takes 64 consecutive bytes of a column (columns a power of
+// two apart share a cache set: what a load leaves of a line is evicted before the next one).
+typedef double dvu2 __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ int chunk_at(int g, int q) { return 2 * g + (q & 1) + 8 * (q >> 1); }
+__device__ __forceinline__ void ld_chunk(const double* __restrict__ p, int g, double (&x)[4]) {
+    const dvu2 a = *reinterpret_cast<const dvu2*>(p + 2 * g), b = *reinterpret_cast<const dvu2*>(p + 8 + 2 * g);
+    x[0] = a.x; x[1] = a.y; x[2] = b.x; x[3] = b.y;
+}
+
+// V = K^T K (n x n, upper tiles and their mirror) and M = B^T K (In x n, column-major) of the
+// sampled step: one workgroup per 16 x 16 tile, eight waves over 16-sample chunks of column c
+// of each operand.  ns = 1024, n = 32, In = 256: 10.3 us, bound by the latency of its two
+// rounds of loads.
+__global__ __launch_bounds__(512) void k_sampled_products(const double* __restrict__ K, const double* __restrict__ B,
+                                                          int64_t ns, int n, int64_t In, double* __restrict__ V,
+                                                          double* __restrict__ M, const DevCheck* __restrict__ chk) {
+    if (chk->done) return;
+    __shared__ double part[8][256];
+    const int t = threadIdx.x, l = t & 63, c = l & 15, g = l >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nt = (n + 15) / 16, ngram = nt * (nt + 1) / 2;
+    const bool gram = (int)blockIdx.x < ngram;
+    int tb = 0;
+    int64_t ta = blockIdx.x;
+    if (gram) {
+        while (ta > tb) { ta -= tb + 1; ++tb; }
+    } else {
+        tb = (int)((ta - ngram) % nt);
+        ta = (ta - ngram) / nt;
+    }
+    // columns past the end read a valid one: their products are not stored
+    const int64_t na = gram ? n : In, ca = 16 * ta + c < na ? 16 * ta + c : na - 1;
+    const int cb = 16 * tb + c < n ? 16 * tb + c : n - 1;
+    const double* __restrict__ pa = (gram ? K : B) + ns * ca;
+    const double* __restrict__ pb = K + ns * cb;
+    d4 acc = (d4){0.0, 0.0, 0.0, 0.0};
+    int64_t s = 16 * w;
+    for (; s + 400 <= ns; s += 512) {
+        double a[4][4], b[4][4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            ld_chunk(pa + s + 128 * u, g, a[u]);
+            ld_chunk(pb + s + 128 * u, g, b[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc = mfma_f64(a[u][q], b[u][q], acc);
+    }
+    for (; s < ns; s += 128) {
+        double a[4], b[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t sq = s + chunk_at(g, q);
+            const bool ok = sq < ns;
+            a[q] = pa[ok ? sq : ns - 1];
+            b[q] = pb[ok ? sq : ns - 1];
+            if (!ok) a[q] = b[q] = 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc = mfma_f64(a[q], b[q], acc);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) part[w][64 * v + l] = acc[v];
+    __syncthreads();
+    if (t >= 256) return;
+    double sum = 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) sum += part[k][t];
+    const int64_t r = 16 * ta + ((t >> 4) & 3) + 4 * (t >> 6);
+    const int r2 = 16 * tb + (t & 15);
+    if (r >= na || r2 >= n) return;
+    if (gram) {
+        V[r * n + r2] = sum;
+        V[(int64_t)r2 * n + r] = sum;
+    } else {
+        M[r + In * r2] = sum;
+    }
+}
+
+// V^-1 by sweeps.  info = {n, 0, n} when certified, else info[1] = 1.  Certified means
+// ||V||_F ||V^-1||_F < 1e8, so cond(K) < 1e4: k_sampled_correct's one correction then leaves
+// (eps cond(K)^2)^2, far below the rounding of the QR solve it replaces, and K has full rank
+// by the QR's test (n eps).
+__global__ __launch_bounds__(256) void k_sampled_inverse(const double* __restrict__ V, int n, double* __restrict__ Vinv,
+                                                         int* __restrict__ info, const DevCheck* __restrict__ chk) {
+    if (chk->done) return;
+    __shared__ double S[SWEEP_ROWS + 16];
+    GramSet gs{};
+    gs.G[0] = gs.G[1] = V;   // of mode 1: the other "Gram" alone
+    gs.N = 2;
+    if (!factor64_unpivoted(gs, 1, n, 0.0, Vinv, info, S, 1e8) && threadIdx.x == 0) info[1] = 1;
+}
+
+// Corrected normal equations for 16 rows of X (one workgroup): X_0 = M V^-1, the residual
+// E = B - K X_0^T of every sample in FP64, X = X_0 + (E^T K) V^-1.  The waves take
+// 16-sample chunks; a chunk of E comes out of its product as the operand of the next one
+// (sample chunk_at(g, v), row c), so it never leaves the registers.  Bound by the matrix cores of
+// the In / 16 CUs it runs on: ns = 1024, n = 32, In = 256, 21.8 us (31.7 with
+// 8-byte loads of the chunks).  The column-pivoted QR, its application and rank test took 610
+// us there (74 launches); they still solve what k_sampled_inverse does not certify.
+// four waves for RT = 64, whose two chunks in flight need more than 256 registers
+constexpr int correct_threads(int rt) { return rt == 64 ? 256 : 512; }
+template <int RT>
+__global__ __launch_bounds__(correct_threads(RT)) void k_sampled_correct(const double* __restrict__ K, const double* __restrict__ B,
+                                                         int64_t ns, int n, int64_t In, const double* __restrict__ M,
+                                                         const double* __restrict__ Vinv, const int* __restrict__ info,
+                                                         double* __restrict__ X, const DevCheck* __restrict__ chk) {
+    constexpr int NT = RT / 16, KS = RT / 4, LD = RT + 2, NTHR = correct_threads(RT), NW = NTHR / 64;
+    if (chk->done || info[1] != 0) return;
+    __shared__ double X0[16 * LD];
+    __shared__ double part[NW * NT * 256];
+    const int t = threadIdx.x, l = t & 63, c = l & 15, g = l >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int64_t i0 = 16 * (int64_t)blockIdx.x, ic = i0 + c < In ? i0 + c : In - 1;
+    // tile tb of (16 x RT operand rows `row(k)`) V^-1; zero beyond n
+    auto times_vinv = [&](auto row, int tb) {
+        d4 acc = (d4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int k = 4 * ks + g, r = 16 * tb + c;
+            const bool ok = k < n && r < n;
+            const double b = Vinv[ok ? k * n + r : 0];
+            acc = mfma_f64(k < n ? row(k) : 0.0, ok ? b : 0.0, acc);
+        }
+        return acc;
+    };
+    d4 x0 = (d4){0.0, 0.0, 0.0, 0.0};
+    if (w < NT) {
+        x0 = times_vinv([&](int k) { return M[ic + In * k]; }, w);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) X0[(g + 4 * v) * LD + 16 * w + c] = x0[v];
+    }
+    __syncthreads();
+    double xb[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) xb[ks] = X0[c * LD + 4 * ks + g];
+    d4 acc[NT];
+#pragma unroll
+    for (int tb = 0; tb < NT; ++tb) acc[tb] = (d4){0.0, 0.0, 0.0, 0.0};
+    const double* __restrict__ pB = B + ns * ic;
+    const double* __restrict__ pa[KS];   // columns past n: valid, met by zeros of xb
+    const double* __restrict__ pk[NT];   // columns past n: valid, not stored
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) pa[ks] = K + ns * (4 * ks + g < n ? 4 * ks + g : n - 1);
+#pragma unroll
+    for (int tb = 0; tb < NT; ++tb) pk[tb] = K + ns * (16 * tb + c < n ? 16 * tb + c : n - 1);
+    struct Chunk {
+        double ka[KS], kb[NT][4], b[4];
+    };
+    const int pc = chunk_at(c & 3, c >> 2);   // row g + 4v of the product is sample chunk_at(g, v)
+    auto load = [&](int64_t s0, Chunk& h) {
+        if (s0 + 16 <= ns) {
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) h.ka[ks] = pa[ks][s0 + pc];
+            ld_chunk(pB + s0, g, h.b);
+#pragma unroll
+            for (int tb = 0; tb < NT; ++tb) ld_chunk(pk[tb] + s0, g, h.kb[tb]);
+        } else {   // samples past the end: the last one
+            const int64_t sa = s0 + pc < ns ? s0 + pc : ns - 1;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) h.ka[ks] = pa[ks][sa];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int64_t s = s0 + chunk_at(g, v) < ns ? s0 + chunk_at(g, v) : ns - 1;
+                h.b[v] = pB[s];
+#pragma unroll
+                for (int tb = 0; tb < NT; ++tb) h.kb[tb][v] = pk[tb][s];
+            }
+        }
+    };
+    auto step = [&](int64_t s0, const Chunk& h) {
+        d4 pr = (d4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) pr = mfma_f64(h.ka[ks], xb[ks], pr);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const double e = s0 + chunk_at(g, v) < ns ? h.b[v] - pr[v] : 0.0;
+#pragma unroll
+            for (int tb = 0; tb < NT; ++tb) acc[tb] = mfma_f64(e, h.kb[tb][v], acc[tb]);
+        }
+    };
+    Chunk h0, h1;   // the next chunk's loads in flight behind the current one's products
+    int64_t s0 = 16 * (int64_t)w;
+    if (s0 < ns) load(s0, h0);
+    for (; s0 < ns; s0 += 32 * NW) {
+        const int64_t s1 = s0 + 16 * NW, s2 = s0 + 32 * NW;
+        if (s1 < ns) load(s1, h1);
+        step(s0, h0);
+        if (s1 >= ns) break;
+        if (s2 < ns) load(s2, h0);
+        step(s1, h1);
+    }
+#pragma unroll
+    for (int tb = 0; tb < NT; ++tb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) part[(w * NT + tb) * 256 + 64 * v + l] = acc[tb][v];
+    __syncthreads();
+    // the waves' sums, as the next product's rows: X0 is read no more
+    for (int x = t; x < NT * 256; x += NTHR) {
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < NW; ++k) s += part[k * NT * 256 + x];
+        X0[(((x >> 4) & 3) + 4 * ((x >> 6) & 3)) * LD + 16 * (x >> 8) + (x & 15)] = s;
+    }
+    __syncthreads();
+    if (w < NT) {
+        const d4 dx = times_vinv([&](int k) { return X0[c * LD + k]; }, w);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int64_t i = i0 + g + 4 * v;
+            const int r = 16 * w + c;
+            if (i < In && r < n) X[i + In * r] = x0[v] + dx[v];
+        }
+    }
 }
 
 // Householder reflector of x = (x[0], x[1 .. len)) (xLARFG): x[0] <- beta,
@@ -582,9 +801,8 @@ __global__ __launch_bounds__(256) void k_lev_rows(const double* __restrict__ A, 
 }
 
 // The same for n <= 64: k_gram_chol64 factors G = U^T U with the Schur complement in
-// registers and writes U; k_lev_rows64 solves U^T y = a_i per row (a lane per row, U
-// broadcast from LDS) and p(i) = ||y||^2 / n, the same a_i^T G^-1 a_i / n without
-// forming G^-1.
+// registers and writes U; k_lev_rows64 solves U^T y = a_i and p(i) = ||y||^2 / n, the
+// same a_i^T G^-1 a_i / n without forming G^-1.
 constexpr int LEV64_LD = 65;
 // One workgroup of 256 threads, the Schur complement in registers: thread (w, l)
 // holds rows 16w..16w+15 of column l.  Step j: the wave owning row j hands it over
@@ -623,7 +841,12 @@ __global__ __launch_bounds__(256) void k_gram_chol64(const double* __restrict__ 
             bad = true;
             break;
         }
-        const double ujj = sqrt(d), inv = 1.0 / ujj;
+        // 1/sqrt(d) from the hardware estimate (relative error < 2^-22) and two Newton steps
+        const double dc = fmax(d, 0x1p-1020), h = 0.5 * dc;
+        double inv = __builtin_amdgcn_rsq(dc);
+        inv = fma(inv, fma(-h * inv, inv, 0.5), inv);
+        inv = fma(inv, fma(-h * inv, inv, 0.5), inv);
+        const double ujj = dc * inv;
         const double ul = rb[l] * inv;
         if (w == 0 && l < n) U[j + (int64_t)n * l] = l > j ? ul : (l == j ? ujj : 0.0);
 #pragma unroll
@@ -637,36 +860,67 @@ __global__ __launch_bounds__(256) void k_gram_chol64(const double* __restrict__ 
     if (t == 0) *need = bad ? 1 : 0;
 }
 
-__global__ __launch_bounds__(64) void k_lev_rows64(const double* __restrict__ A, int m, int n,
+// p(i) = ||U^-T a_i||^2 / n by blocks of 16 on MFMA, transposed: Y_j = D_j^T (A_j^T - sum_{k<j}
+// U_kj^T Y_k), D_j the inverse of the diagonal block (wave j, lane c: column c by substitution).
+// A wave takes 16 rows of A; its finished block of Y is the next ones' operand as it stands.
+// 256 rows, n = 32: 6.4 us (35.3 with a lane per row, whose chain of n^2 / 2 steps was code
+// that ran once).
+__global__ __launch_bounds__(256) void k_lev_rows64(const double* __restrict__ A, int m, int n,
                                                    const double* __restrict__ U, const int* __restrict__ need,
                                                    double* __restrict__ probs, const DevCheck* __restrict__ chk) {
     if (chk->done || *need != 0) return;
-    __shared__ double S[64 * LEV64_LD];
-    __shared__ double dinv[64];
-    const int t = threadIdx.x;
-    for (int x = t; x < n * n; x += 64) S[(x % n) * LEV64_LD + x / n] = U[x];
+    __shared__ double S[64 * LEV64_LD];       // U by rows, the identity beyond n
+    __shared__ double Di[4][16 * 17];
+    const int t = threadIdx.x, l = t & 63, c = l & 15, g = l >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nt = (n + 15) / 16, np = 16 * nt;
+    const int i = (int)blockIdx.x * 64 + 16 * w + c, ic = i < m ? i : m - 1;
+    d4 y[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int k = 16 * j + g + 4 * v;
+            const double a = A[ic + (int64_t)m * (k < n ? k : 0)];
+            y[j][v] = k < n ? a : 0.0;
+        }
+    for (int x = t; x < np * np; x += 256) {
+        const int r = x % np, q = x / np;
+        S[r * LEV64_LD + q] = r < n && q < n ? U[r + n * q] : (r == q ? 1.0 : 0.0);
+    }
     __syncthreads();
-    if (t < n) dinv[t] = 1.0 / S[t * LEV64_LD + t];
-    __syncthreads();
-    const int i = blockIdx.x * 64 + t;
-    if (i >= m) return;
-    double y[64];
+    if (w < nt && l < 16) {
+        double xv[16];
+        const double* D = S + 16 * w * (LEV64_LD + 1);
 #pragma unroll
-    for (int k = 0; k < 64; ++k) y[k] = k < n ? A[i + (int64_t)m * k] : 0.0;
-    // U^T y = a by columns of U^T (rows of U): y_j /= U(j,j), y_k -= U(j,k) y_j
+        for (int r = 15; r >= 0; --r) {
+            double acc = r == l ? 1.0 : 0.0;
 #pragma unroll
-    for (int j = 0; j < 64; ++j) {
-        if (j < n) {
-            y[j] *= dinv[j];
-#pragma unroll
-            for (int k = j + 1; k < 64; ++k)
-                if (k < n) y[k] -= S[j * LEV64_LD + k] * y[j];
+            for (int k = r + 1; k < 16; ++k) acc -= D[r * LEV64_LD + k] * xv[k];
+            xv[r] = acc / D[r * LEV64_LD + r];
+            Di[w][r * 17 + l] = xv[r];
         }
     }
+    __syncthreads();
     double s = 0.0;
 #pragma unroll
-    for (int k = 0; k < 64; ++k) s += y[k] * y[k];
-    probs[i] = s / (double)n;
+    for (int j = 0; j < 4; ++j) {
+        if (j >= nt) break;
+#pragma unroll
+        for (int k = 0; k < j; ++k)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                y[j] = mfma_f64(-S[(16 * k + g + 4 * v) * LEV64_LD + 16 * j + c], y[k][v], y[j]);
+        d4 o = (d4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int v = 0; v < 4; ++v) o = mfma_f64(Di[j][(g + 4 * v) * 17 + c], y[j][v], o);
+        y[j] = o;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) s = fma(o[v], o[v], s);
+    }
+    s += __shfl_xor(s, 16);
+    s += __shfl_xor(s, 32);
+    if (g == 0 && i < m) probs[i] = s / (double)n;
 }
 
 // p(i) = 1 / m for m <= n (Q is square and orthogonal: every row has norm 1)
@@ -1115,7 +1369,7 @@ int launch_leverage_scores(itcpd_plan* p, int mode, double* probs_dev, double** 
     if (n <= 64) {
         hipLaunchKernelGGL(k_gram_chol64, dim3(1), dim3(256), 0, p->stream, G, n, Ui, need, p->chk);
         ITCPD_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_lev_rows64, dim3((unsigned)cdiv(m, 64)), dim3(64), 0, p->stream, p->A[mode], m, n, Ui,
+        hipLaunchKernelGGL(k_lev_rows64, dim3((unsigned)cdiv(m, 64)), dim3(256), 0, p->stream, p->A[mode], m, n, Ui,
                            need, probs, p->chk);
     } else {
         hipLaunchKernelGGL(k_gram_chol_inv<256>, dim3(1), dim3(256), 0, p->stream, G, n, Ui, Gi, need, p->chk);
@@ -1130,46 +1384,89 @@ int launch_leverage_scores(itcpd_plan* p, int mode, double* probs_dev, double** 
     return ITCPD_OK;
 }
 
-// samples: device, ns x (N-1) column-major.  X (I_n x R) is left in p->X; info[0] =
-// rank of K_s (QR form) or the factorisation's finfo (normal form) is copied by the caller.
-int launch_sampled_solve(itcpd_plan* p, int mode, int64_t ns, const int* samples, bool normal) {
+namespace {
+
+// Views of the sampled step's workspace.
+struct SampledWs {
+    double *Ks, *B, *W, *Vs, *tau, *ztau, *vwork;
+    int *jpvt, *info;
+};
+SampledWs sampled_ws(const itcpd_plan* p, int mode, int64_t ns) {
+    const size_t R = (size_t)p->R;
+    SampledWs w;
+    w.Ks = p->smp_ws;                                   // ns x R
+    w.B = w.Ks + (size_t)ns * R;                        // ns x In
+    w.W = w.B + (size_t)ns * (size_t)p->dims[mode];     // ns x R (QR form)
+    w.Vs = w.W + (size_t)ns * R;                        // R x R
+    w.tau = w.Vs + R * R;                               // R
+    w.ztau = w.tau + R;                                 // R
+    w.vwork = w.ztau + R;                               // 2 R
+    w.jpvt = p->smp_iws + (size_t)ns * (p->N - 1);
+    w.info = w.jpvt + R;
+    return w;
+}
+
+}  // namespace
+
+bool sampled_corrected_ok(const itcpd_plan* p, int64_t ns) { return p->R <= 64 && ns >= p->R; }
+
+// samples: device, ns x (N-1) column-major.  K_s and the sampled fibers, into the workspace.
+int launch_sampled_gather(itcpd_plan* p, int mode, int64_t ns, const int* samples) {
     const int R = (int)p->R;
     const int64_t In = p->dims[mode];
     const OtherModes om = other_modes(p, mode);
-    double* Ks = p->smp_ws;                       // ns x R
-    double* B = Ks + (size_t)ns * R;              // ns x In
-    double* W = B + (size_t)ns * In;              // ns x R (QR form)
-    double* Vs = W + (size_t)ns * R;              // R x R
-    double* tau = Vs + (size_t)R * R;             // R
-    double* ztau = tau + R;                       // R
-    double* vwork = ztau + R;                     // 2 R
-    int* jpvt = p->smp_iws + (size_t)ns * (p->N - 1);
-    int* info = jpvt + R;
+    const SampledWs w = sampled_ws(p, mode, ns);
     const int64_t nk = ns * R, nb = ns * In;
     hipLaunchKernelGGL(k_pivot_hadamard, dim3((unsigned)cdiv(nk, 256)), dim3(256), 0, p->stream, om, samples,
-                       ns, R, Ks, p->chk);
+                       ns, R, w.Ks, p->chk);
     ITCPD_HIP(hipGetLastError());
     const int64_t ms = tensor_stride(p, mode);
     if (p->elt_bytes == 8)
         hipLaunchKernelGGL(k_sample_fibers<double>, dim3((unsigned)cdiv(nb, 256)), dim3(256), 0, p->stream,
-                           (const double*)p->T, om, ms, In, samples, ns, B, p->chk);
+                           (const double*)p->T, om, ms, In, samples, ns, w.B, p->chk);
     else
         hipLaunchKernelGGL(k_sample_fibers<float>, dim3((unsigned)cdiv(nb, 256)), dim3(256), 0, p->stream,
-                           (const float*)p->T, om, ms, In, samples, ns, B, p->chk);
+                           (const float*)p->T, om, ms, In, samples, ns, w.B, p->chk);
     ITCPD_HIP(hipGetLastError());
-    if (normal) {
-        // V = K_s^T K_s, M = B^T K_s, then the plan's factorisation and row solves on V
-        hipLaunchKernelGGL(k_gemm_tn, dim3((unsigned)cdiv((int64_t)R * R * 64, 256)), dim3(256), 0, p->stream,
-                           Ks, Ks, ns, R, R, Vs, p->chk);
+    return ITCPD_OK;
+}
+
+// The solve on the gathered samples: X (I_n x R) is left in p->X (with the normal equations
+// also row-normed).  info[0] = rank of K_s and, for the corrected form, info[1] != 0 when it
+// is not certified and X is not set; or the factorisation's finfo (normal form).
+int launch_sampled_solve(itcpd_plan* p, int mode, int64_t ns, int form) {
+    const int R = (int)p->R;
+    const int64_t In = p->dims[mode];
+    const SampledWs ws = sampled_ws(p, mode, ns);
+    double *const Ks = ws.Ks, *const B = ws.B, *const W = ws.W, *const Vs = ws.Vs, *const tau = ws.tau,
+           *const ztau = ws.ztau, *const vwork = ws.vwork;
+    int *const jpvt = ws.jpvt, *const info = ws.info;
+    const int64_t nk = ns * R;
+    if (form != SAMPLED_QR) {   // V = K_s^T K_s, M = B^T K_s
+        const unsigned nt = (unsigned)cdiv(R, 16);
+        hipLaunchKernelGGL(k_sampled_products, dim3((unsigned)(nt * (nt + 1) / 2 + cdiv(In, 16) * nt)), dim3(512), 0,
+                           p->stream, Ks, B, ns, R, In, Vs, p->M, p->chk);
         ITCPD_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_gemm_tn, dim3((unsigned)cdiv(In * R * 64, 256)), dim3(256), 0, p->stream, B, Ks,
-                           ns, (int)In, R, p->M, p->chk);
-        ITCPD_HIP(hipGetLastError());
+    }
+    if (form == SAMPLED_NORMAL) {   // the plan's factorisation and update on V
         p->v_override = Vs;
         int rc = launch_factor(p, mode);
         p->v_override = nullptr;
         if (rc) return rc;
-        return launch_solve(p, mode, p->M, 1, In * R, false, false);
+        return launch_solve(p, mode, p->M, 1, In * R, true, false);
+    }
+    if (form == SAMPLED_CORRECTED) {
+        hipLaunchKernelGGL(k_sampled_inverse, dim3(1), dim3(256), 0, p->stream, Vs, R, p->Upad, info, p->chk);
+        ITCPD_HIP(hipGetLastError());
+        auto run = [&](auto kern, int threads) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)cdiv(In, 16)), dim3(threads), 0, p->stream, Ks, B, ns, R, In, p->M,
+                               p->Upad, info, p->X, p->chk);
+        };
+        if (R <= 16) run(k_sampled_correct<16>, correct_threads(16));
+        else if (R <= 32) run(k_sampled_correct<32>, correct_threads(32));
+        else run(k_sampled_correct<64>, correct_threads(64));
+        ITCPD_HIP(hipGetLastError());
+        return ITCPD_OK;
     }
     ITCPD_HIP(hipMemcpyAsync(W, Ks, (size_t)nk * 8, hipMemcpyDeviceToDevice, p->stream));
     // tall samples: the column-pivoted QR as grid-wide steps (a wave per column instead

@@ -1632,7 +1632,34 @@ int run_update_small(itcpd_plan* p, int mode, const double* Msrc, int nparts, in
     return ITCPD_OK;
 }
 
+// row_norm of X from nb Gram partials, with <M, X> for the fit when asked
+int run_finalize(itcpd_plan* p, int mode, int nb, const double* Mkept, bool fit) {
+    const int64_t In = p->dims[mode];
+    const int R = (int)p->R;
+    const int nbf = finalize_nb(In, R);
+    const bool one_rt = nb <= 32 && R <= 256 && cdiv((int64_t)R * R, nbf) <= 256 && cdiv(In, nbf) * R <= 2048;
+    hipLaunchKernelGGL(one_rt ? k_finalize_1rt : k_finalize, dim3(nbf), dim3(256), one_rt ? 0 : (size_t)R * 8,
+                       p->stream, p->gram_part, nb, p->X, Mkept, In, R, (int)p->Rp, p->A[mode], p->At[mode],
+                       p->lam, p->G[mode], fit ? p->inner_part : (double*)nullptr, p->chk);
+    ITCPD_HIP(hipGetLastError());
+    return ITCPD_OK;
+}
+// the same with X's Gram by a launch of its own
+int run_gram_finalize(itcpd_plan* p, int mode, const double* Mkept, bool fit) {
+    const int R = (int)p->R;
+    GramJobs gj{};
+    gj.X[0] = p->X;
+    gj.S[0] = p->gram_part;
+    gj.I[0] = p->dims[mode];
+    const int nb = gram_parts(p->dims[mode], R);
+    hipLaunchKernelGGL(k_gram_mfma, dim3(gram_tiles(R), (unsigned)nb), dim3(256), 0, p->stream, gj, R, nb, p->chk);
+    ITCPD_HIP(hipGetLastError());
+    return run_finalize(p, mode, nb, Mkept, fit);
+}
+
 }  // namespace
+
+int launch_row_norm(itcpd_plan* p, int mode) { return run_gram_finalize(p, mode, p->X, false); }
 
 int launch_solve(itcpd_plan* p, int mode, const double* Msrc, int nparts, int64_t stride,
                  bool finalize, bool fit_after, int next_factor) {
@@ -1656,23 +1683,12 @@ int launch_solve(itcpd_plan* p, int mode, const double* Msrc, int nparts, int64_
     rc = run_apply(p, mode, Msrc, nparts, stride, finalize, fit_after);
     if (rc || !finalize) return rc;
     const int64_t In = p->dims[mode];
-    int nb = solve_nb(In, R);
-    const double* Mkept = p->Msum;
-    if (!p->RT) {   // R > 64: the Gram of X by its own launch; M is still where the solve read it
-        GramJobs gj{};
-        gj.X[0] = p->X;
-        gj.S[0] = p->gram_part;
-        gj.I[0] = In;
-        nb = gram_parts(In, R);
-        hipLaunchKernelGGL(k_gram_mfma, dim3(gram_tiles(R), (unsigned)nb), dim3(256), 0, p->stream, gj, R, nb, p->chk);
-        Mkept = Msrc;
-    }
+    const bool fit = fit_after && !cp_check;
+    // R > 64: the Gram of X by its own launch; M is still where the solve read it
+    if ((rc = p->RT ? run_finalize(p, mode, solve_nb(In, R), p->Msum, fit)
+                    : run_gram_finalize(p, mode, Msrc, fit)))
+        return rc;
     const int nbf = finalize_nb(In, R);
-    const bool one_rt = nb <= 32 && R <= 256 && cdiv((int64_t)R * R, nbf) <= 256 && cdiv(In, nbf) * R <= 2048;
-    hipLaunchKernelGGL(one_rt ? k_finalize_1rt : k_finalize, dim3(nbf), dim3(256), one_rt ? 0 : (size_t)R * 8,
-                       p->stream, p->gram_part, nb, p->X, Mkept, In, R, (int)p->Rp, p->A[mode], p->At[mode],
-                       p->lam, p->G[mode], (fit_after && !cp_check) ? p->inner_part : (double*)nullptr, p->chk);
-    ITCPD_HIP(hipGetLastError());
     if (fit_after && cp_check) {
         if ((rc = launch_cp_check(p))) return rc;
     } else if (fit_after) {
