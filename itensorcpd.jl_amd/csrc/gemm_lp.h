@@ -5,7 +5,15 @@
 //
 // with FP32 MFMA (v_mfma_f32_16x16x4_f32) or BF16x3 (v_mfma_f32_16x16x32_bf16 on hi hi +
 // hi lo + lo hi, x = hi + lo, hi = bf16(x), lo = bf16(x - hi)).  Kt is the side's Khatri-Rao
-// product from k_krp_lp: rank-major, rows padded with zeros to a multiple of 32 indices.
+// product from k_krp_lp: rank-major, rows padded with zeros to a multiple of 32 indices, in
+// one part (FP32), two (BF16x3: hi, lo) or four.
+//
+// Four parts: BF16x3 where the factor, not the product, is what is rounded to two parts, x = (a_hi
+// + a_lo) w with w the other modes' weight.  Rounding the product instead moves the CPD by a
+// factor's rounding times the conditioning of its solves (up to 6.7e-5 over drawn order-4
+// problems, of which 6.6e-5 is the factor's rounding against 64 bits).  The parts are h, m, r
+// of x with h = bf16(a_hi w), and l = bf16(a_hi w - h): T_hi (h + m + r) + T_lo (h + l), the
+// tensor's lo part meeting a_hi alone.
 //
 // As in gemm64.h each tensor element goes from global memory to the registers of the one
 // wave that uses it, from addresses that are always valid, with the next stage's loads issued
@@ -16,9 +24,10 @@
 // ones every 128 reduction indices.  MFMA 16x16x4 step s takes k = k0 + 4 g + s; result:
 // lane (c, g), register v holds rank 4 g + v, output c.
 //
-// Measured per launch (left / right, us) on 150 x 130 x 110 x 90 FP32-stored, rank 48:
-// FP32 256 / 304, BF16x3 280 / 306 (741 / 994 and 1128 / 1534 for the masked register-staged
-// kernels that these replace); 301 x 257 x 199 rank 40 35 / 40 and 40 / 31 (97 / 78, 99 / 101).  Bound by the
+// Measured per launch (left / right, us) on 150 x 130 x 110 x 90 FP32-stored, rank 48: FP32
+// 256 / 304, BF16x3 in four parts 397 / 429 (280 / 306 in two, where the fourfold operand is not
+// read) against 741 / 994 and 1128 / 1534 for the masked register-staged kernels that these
+// replace; 301 x 257 x 199 rank 40, FP32 35 / 40 (97 / 78).  Bound by the
 // tensor's stream (0.77 GB, 127 us at 6.06 TB/s) and, in FP32, the matrix cores (122 us at 152
 // TFLOP/s).
 #pragma once
@@ -63,29 +72,33 @@ __device__ __forceinline__ void ld_float(const TT* __restrict__ p, float* x) {
     }
 }
 
-// The Khatri-Rao operand of one rank row and stage.
-template <bool BF>
+// The Khatri-Rao operand of one rank row and stage, in KP parts.
+template <int KP>
 struct KrpRun {
+    bf8 hi, lo, r, l;   // r, l: of four parts (h, m, r, l)
+    __device__ __forceinline__ void load(const void* row, int64_t part, int64_t k) {
+        const __bf16* p = reinterpret_cast<const __bf16*>(row) + k;
+        hi = *reinterpret_cast<const bf8*>(p);
+        lo = *reinterpret_cast<const bf8*>(p + part);
+        if constexpr (KP == 4) {
+            r = *reinterpret_cast<const bf8*>(p + 2 * part);
+            l = *reinterpret_cast<const bf8*>(p + 3 * part);
+        }
+    }
+};
+template <>
+struct KrpRun<1> {
     float v[4];
     __device__ __forceinline__ void load(const void* row, int64_t, int64_t k) {
         const f4 x = *reinterpret_cast<const f4*>(reinterpret_cast<const float*>(row) + k);
         v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
     }
 };
-template <>
-struct KrpRun<true> {
-    bf8 hi, lo;
-    __device__ __forceinline__ void load(const void* row, int64_t lo_off, int64_t k) {
-        const __bf16* p = reinterpret_cast<const __bf16*>(row) + k;
-        hi = *reinterpret_cast<const bf8*>(p);
-        lo = *reinterpret_cast<const bf8*>(p + lo_off);
-    }
-};
 
 // acc += Kt-rows x T over one stage; x[b] holds the lane's E values of output tile b.
-template <bool BF, int RB, int MB, int E>
-__device__ __forceinline__ void lp_stage(const KrpRun<BF> (&kr)[RB], const float (&x)[MB][E], f4 (&acc)[RB * MB]) {
-    if constexpr (BF) {
+template <int KP, int RB, int MB, int E>
+__device__ __forceinline__ void lp_stage(const KrpRun<KP> (&kr)[RB], const float (&x)[MB][E], f4 (&acc)[RB * MB]) {
+    if constexpr (KP > 1) {
 #pragma unroll
         for (int b = 0; b < MB; ++b) {
             bf8 bh, bl;
@@ -93,6 +106,10 @@ __device__ __forceinline__ void lp_stage(const KrpRun<BF> (&kr)[RB], const float
 #pragma unroll
             for (int a = 0; a < RB; ++a) {
                 f4 s = acc[a * MB + b];
+                if constexpr (KP == 4) {
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kr[a].r, bh, s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kr[a].l, bl, s, 0, 0, 0);
+                }
                 s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kr[a].lo, bh, s, 0, 0, 0);
                 s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kr[a].hi, bl, s, 0, 0, 0);
                 acc[a * MB + b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kr[a].hi, bh, s, 0, 0, 0);
@@ -122,12 +139,13 @@ __device__ __forceinline__ void lp_flush(f4 (&acc)[N], d4 (&tot)[N]) {
 // LEFT: outputs are rows (VEC of them consecutive per lane, the tile moved back to end at the
 // last row when VEC > 1, which then needs outs >= 16 MB); else columns.  Grid: x rank blocks
 // (the workgroups that share a tensor tile run together) times tiles, z reduction splits.
-template <bool LEFT, typename TT, bool BF, int RB, int MB, int KW, int VEC, int D, int OCC>
+template <bool LEFT, typename TT, int KP, int RB, int MB, int KW, int VEC, int D, int OCC>
 __global__ __launch_bounds__(256, OCC) void k_gemm_lp(const TT* __restrict__ T, int64_t outs, int64_t K,
-                                                    const void* __restrict__ Kt, int64_t Kp, int64_t lo_off,
+                                                    const void* __restrict__ Kt, int64_t Kp, int64_t part,
                                                     int64_t stages_per_split, int ny, int R,
                                                     double* __restrict__ out, int64_t split_stride,
                                                     const DevCheck* __restrict__ chk) {
+    constexpr bool BF = KP > 1;
     constexpr int E = BF ? 8 : 4, ST = 4 * E, FLUSH = 128 / ST;
     constexpr int NB = MB / VEC;
     if (chk->done) return;
@@ -167,7 +185,7 @@ __global__ __launch_bounds__(256, OCC) void k_gemm_lp(const TT* __restrict__ T, 
         acc[a] = (f4){0.f, 0.f, 0.f, 0.f};
         tot[a] = (d4){0.0, 0.0, 0.0, 0.0};
     }
-    KrpRun<BF> kr[D][RB];
+    KrpRun<KP> kr[D][RB];
     float x[D][MB][E];
     auto load = [&](int buf, int64_t st) {
         const int64_t k = st * ST + E * g;
@@ -186,11 +204,11 @@ __global__ __launch_bounds__(256, OCC) void k_gemm_lp(const TT* __restrict__ T, 
             for (int b = 0; b < NB; ++b) ld_float<TT, E>(base[b] + k, x[buf][b]);
         }
 #pragma unroll
-        for (int a = 0; a < RB; ++a) kr[buf][a].load(krow[a], lo_off, k);
+        for (int a = 0; a < RB; ++a) kr[buf][a].load(krow[a], part, k);
     };
     int flush = 0;
     auto compute = [&](int buf) {
-        lp_stage<BF, RB, MB, E>(kr[buf], x[buf], acc);
+        lp_stage<KP, RB, MB, E>(kr[buf], x[buf], acc);
         if (++flush == FLUSH) {
             lp_flush<RB * MB>(acc, tot);
             flush = 0;
@@ -226,8 +244,8 @@ __global__ __launch_bounds__(256, OCC) void k_gemm_lp(const TT* __restrict__ T, 
                 }
         }
 #pragma unroll
-        for (int a = 0; a < RB; ++a) kr[0][a].load(krow[a], lo_off, k);
-        lp_stage<BF, RB, MB, E>(kr[0], x[0], acc);
+        for (int a = 0; a < RB; ++a) kr[0][a].load(krow[a], part, k);
+        lp_stage<KP, RB, MB, E>(kr[0], x[0], acc);
     }
     lp_flush<RB * MB>(acc, tot);
 

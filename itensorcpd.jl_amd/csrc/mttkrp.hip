@@ -93,33 +93,47 @@ __device__ __forceinline__ int lpr_chunk(int j, int q) {
     return (j >> 1) * 256 + 16 * ((((j & 1) << 3) | q) ^ ((j >> 1) & 15));
 }
 
-template <bool BF>
+// KP parts of Mp x Rk: the value in FP32 (1), BF16 hi and lo (2), or h, m, r, l of gemm_lp.h (4).
+template <int KP>
 __global__ __launch_bounds__(256) void k_krp_lp(Side sd, int64_t M, int64_t Mp, int R, int Rk,
                                                 void* __restrict__ Kt,
                                                 const DevCheck* __restrict__ chk) {
     if (chk->done) return;
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= Mp * Rk) return;
+    const int64_t part = Mp * Rk;
+    if (idx >= part) return;
     const int r = (int)(idx / Mp);
     const int64_t m = idx - (int64_t)r * Mp;
-    double w = 0.0;
+    double a = 0.0, w = 1.0;   // the product; of four parts, the fastest mode's factor and the others' weight
     if (r < R && m < M) {
-        w = 1.0;
-        int64_t t = m;
-        for (int q = 0; q < sd.nm; ++q) {
+        int64_t t = m / sd.dim[0];
+        a = sd.fac[0][m - t * sd.dim[0] + sd.dim[0] * r];
+        for (int q = 1; q < sd.nm; ++q) {
             const int64_t d = t % sd.dim[q];
             t /= sd.dim[q];
-            w *= sd.fac[q][d + sd.dim[q] * r];
+            (KP == 4 ? w : a) *= sd.fac[q][d + sd.dim[q] * r];
         }
     }
-    const float x = (float)w;
-    if constexpr (BF) {
+    if constexpr (KP == 1) {
+        reinterpret_cast<float*>(Kt)[idx] = (float)a;
+    } else if constexpr (KP == 2) {
         __bf16* o = reinterpret_cast<__bf16*>(Kt);
+        const float x = (float)a;
         const __bf16 hi = (__bf16)x;
         o[idx] = hi;
-        o[Mp * Rk + idx] = (__bf16)(x - (float)hi);
+        o[part + idx] = (__bf16)(x - (float)hi);
     } else {
-        reinterpret_cast<float*>(Kt)[idx] = x;
+        __bf16* o = reinterpret_cast<__bf16*>(Kt);
+        const float af = (float)a;
+        const __bf16 ah = (__bf16)af, al = (__bf16)(af - (float)ah);
+        const double wf = (double)(float)w, xh = (double)(float)ah * wf;
+        const __bf16 h = (__bf16)(float)xh;
+        const double rest = fma((double)(float)al, wf, xh) - (double)(float)h;
+        const __bf16 mid = (__bf16)(float)rest;
+        o[idx] = h;
+        o[part + idx] = mid;
+        o[2 * part + idx] = (__bf16)(float)(rest - (double)(float)mid);
+        o[3 * part + idx] = (__bf16)(float)(xh - (double)(float)h);
     }
 }
 
@@ -872,60 +886,65 @@ int run_gemm64(itcpd_plan* p, Gemm64& q, double* dst) {
 }
 
 // ---- the direct reduced-precision GEMMs (gemm_lp.h)
-// Rank blocks of 16 per wave (at most 4: FP32 sums, their FP64 totals and two stages of
-// operands share 256 registers) and tile heights, as gemm64_rb / left64_big.
-int lp_rb(int64_t R) {
+// Rank blocks of 16 per wave (at most 4, or 3 with four parts: FP32 sums, their FP64 totals and
+// two stages of operands share 256 registers) and tile heights, as gemm64_rb / left64_big.
+int lp_rb(int64_t R, int kp) {
     const int64_t nb = cdiv(R, 16);
     int best = 1;
     int64_t bestc = INT64_MAX;
-    for (int rb = 4; rb >= 1; --rb) {
+    for (int rb = kp == 4 ? 3 : 4; rb >= 1; --rb) {
         const int64_t ny = cdiv(nb, rb), c = 2 * rb * ny + ny;
         if (c < bestc) { bestc = c; best = rb; }
     }
     return best;
 }
-constexpr int lp_big(bool bf, int rb) { return rb <= (bf ? 2 : 3) ? 4 : 2; }
+constexpr int lp_big(int kp, int rb) { return rb <= (kp > 1 ? 2 : 3) ? 4 : 2; }
 
 // Register stages: three where they fit (160^4-like shapes, FP32, us with two / three: rank 32
 // 231 / 208, rank 64 397 / 360); at rank 48 the third costs more than it hides (252 / 263).
-constexpr int lp_depth(bool bf, int rb) { return !bf && (rb == 2 || rb == 4) ? 3 : 2; }
+constexpr int lp_depth(int kp, int rb) { return kp == 1 && (rb == 2 || rb == 4) ? 3 : 2; }
 
 struct GemmLp {
     bool left;
-    int64_t outs, K, Kp, lo;
-    int rb, ny;
+    int64_t outs, K, Kp, part;
+    int kp, rb, ny;
     Gemm64Cfg c;
     double* out;
 };
-template <bool LEFT, typename TT, bool BF, int RB, int MB, int KW, int VEC>
+template <bool LEFT, typename TT, int KP, int RB, int MB, int KW, int VEC>
 void launch_lp(itcpd_plan* p, const GemmLp& q) {
     const int64_t nt = cdiv(q.outs, 16 * MB);
     const dim3 grid((unsigned)((KW == 1 ? cdiv(nt, 4) : nt) * q.ny), 1, (unsigned)q.c.nz);
-    hipLaunchKernelGGL((k_gemm_lp<LEFT, TT, BF, RB, MB, KW, VEC, lp_depth(BF, RB), 2>), grid, dim3(256), 0, p->stream, (const TT*)p->T,
-                       q.outs, q.K, (const void*)p->Kt, q.Kp, q.lo, q.c.per, q.ny, (int)p->R, q.out, q.outs * p->R,
+    hipLaunchKernelGGL((k_gemm_lp<LEFT, TT, KP, RB, MB, KW, VEC, lp_depth(KP, RB), 2>), grid, dim3(256), 0, p->stream, (const TT*)p->T,
+                       q.outs, q.K, (const void*)p->Kt, q.Kp, q.part, q.c.per, q.ny, (int)p->R, q.out, q.outs * p->R,
                        p->chk);
 }
-template <bool LEFT, typename TT, bool BF, int RB>
+template <bool LEFT, typename TT, int KP, int RB>
 void run_lp(itcpd_plan* p, const GemmLp& q) {
-    constexpr int B = lp_big(BF, RB), V = LEFT ? B : 1;
-    if (q.c.KW == 1) launch_lp<LEFT, TT, BF, RB, B, 1, V>(p, q);
-    else if (q.c.MB == B) launch_lp<LEFT, TT, BF, RB, B, 4, V>(p, q);
-    else launch_lp<LEFT, TT, BF, RB, 1, 4, 1>(p, q);
+    constexpr int B = lp_big(KP, RB), V = LEFT ? B : 1;
+    if (q.c.KW == 1) launch_lp<LEFT, TT, KP, RB, B, 1, V>(p, q);
+    else if (q.c.MB == B) launch_lp<LEFT, TT, KP, RB, B, 4, V>(p, q);
+    else launch_lp<LEFT, TT, KP, RB, 1, 4, 1>(p, q);
 }
-template <bool LEFT, typename TT, bool BF>
+template <bool LEFT, typename TT, int KP>
 void dispatch_lp(itcpd_plan* p, const GemmLp& q) {
     switch (q.rb) {
-        case 1: return run_lp<LEFT, TT, BF, 1>(p, q);
-        case 2: return run_lp<LEFT, TT, BF, 2>(p, q);
-        case 3: return run_lp<LEFT, TT, BF, 3>(p, q);
-        default: return run_lp<LEFT, TT, BF, 4>(p, q);
+        case 1: return run_lp<LEFT, TT, KP, 1>(p, q);
+        case 2: return run_lp<LEFT, TT, KP, 2>(p, q);
+        case 3: return run_lp<LEFT, TT, KP, 3>(p, q);
+        default:
+            if constexpr (KP < 4) run_lp<LEFT, TT, KP, 4>(p, q);
     }
+}
+template <bool LEFT, typename TT>
+void dispatch_lp(itcpd_plan* p, const GemmLp& q) {
+    if (q.kp == 1) dispatch_lp<LEFT, TT, 1>(p, q);
+    else if (q.kp == 2) dispatch_lp<LEFT, TT, 2>(p, q);
+    else dispatch_lp<LEFT, TT, 4>(p, q);
 }
 template <bool LEFT>
 void dispatch_lp(itcpd_plan* p, const GemmLp& q) {
-    const bool bf = p->prec == ITCPD_BF16X3;
-    if (p->elt_bytes == 4) bf ? dispatch_lp<LEFT, float, true>(p, q) : dispatch_lp<LEFT, float, false>(p, q);
-    else bf ? dispatch_lp<LEFT, double, true>(p, q) : dispatch_lp<LEFT, double, false>(p, q);
+    p->elt_bytes == 4 ? dispatch_lp<LEFT, float>(p, q) : dispatch_lp<LEFT, double>(p, q);
 }
 
 }  // namespace
@@ -1118,44 +1137,51 @@ int launch_right_gemm_impl(itcpd_plan* p, MSrc* ms, int factor_mode) {
 // left GEMM, us (ring / direct): FP32 rank 32 1342 / 581, rank 64 1346 / 1169, rank 128 1372 /
 // 2160; BF16x3 rank 16 530 / 491, rank 32 543 / 548, rank 64 545 / 1055.  512^3 rank 64, right
 // GEMM (2 tiles): FP32 4268 / 276, BF16x3 1597 / 231.
-static bool lp_ring_ok(const itcpd_plan* p, bool left) {
+static bool lp_ring_ok(const itcpd_plan* p, bool left, int prec) {
     const int64_t M = left ? p->ML : p->MR, K = left ? p->MR : p->ML;
     const int64_t nb = cdiv(p->R, 16), ny = cdiv(p->R, 128);
     return p->elt_bytes == 4 && M % 256 == 0 && K % 32 == 0 && M / 256 * ny * 8 >= p->num_cu &&
-           nb >= (p->prec == ITCPD_BF16X3 ? 3 : 5) * ny;
+           nb >= (prec == ITCPD_BF16X3 ? 3 : 5) * ny;
 }
 
-// Rows (ranks, padded to the GEMM's blocks) and row length (a multiple of 32) of a side's
-// Khatri-Rao product in Kt.
-static void lp_krp_geometry(const itcpd_plan* p, bool left, int* Rk, int64_t* Kp) {
-    const int rb = lp_rb(p->R);
-    *Rk = lp_ring_ok(p, left) ? 128 * (int)cdiv(p->R, 128) : 16 * rb * (int)cdiv(cdiv(p->R, 16), rb);
-    *Kp = cdiv(left ? p->MR : p->ML, 32) * 32;
+// A side's Khatri-Rao product in Kt: kp parts of Rk rows (ranks, padded to the GEMM's blocks)
+// of Kp elements (a multiple of 32).  Four parts (the factor is rounded, gemm_lp.h) unless the
+// side is one mode, whose product is the factor, or the tensor is whole tiles of the ring form,
+// which rounds the product: each shape keeps the rounding that its BF16x3 results have had.
+struct LpKrp {
+    int kp, Rk;
+    int64_t Kp;
+};
+static LpKrp lp_krp(const itcpd_plan* p, bool left, int prec) {
+    const int64_t M = left ? p->ML : p->MR, K = left ? p->MR : p->ML;
+    const bool one = (left ? p->N - p->s : p->s) == 1, whole = p->elt_bytes == 4 && M % 256 == 0 && K % 32 == 0;
+    LpKrp k;
+    k.kp = prec != ITCPD_BF16X3 ? 1 : (one || whole ? 2 : 4);
+    const int rb = lp_rb(p->R, k.kp);
+    k.Rk = lp_ring_ok(p, left, prec) ? 128 * (int)cdiv(p->R, 128) : 16 * rb * (int)cdiv(cdiv(p->R, 16), rb);
+    k.Kp = cdiv(K, 32) * 32;
+    return k;
 }
+// for either precision: a plan keeps the buffer when it changes between them
 int64_t lp_krp_elems(const itcpd_plan* p) {
     int64_t n = 0;
-    for (int left = 0; left < 2; ++left) {
-        int Rk;
-        int64_t Kp;
-        lp_krp_geometry(p, left != 0, &Rk, &Kp);
-        n = std::max(n, Kp * Rk);
-    }
+    for (int prec : {ITCPD_FP32, ITCPD_BF16X3})
+        for (int left = 0; left < 2; ++left) {
+            const LpKrp k = lp_krp(p, left != 0, prec);
+            n = std::max(n, k.Kp * k.Rk * (k.kp == 4 ? 2 : 1));
+        }
     return n;
 }
-// Forms the reduction side's Khatri-Rao product in Kt; *lo = elements from the BF16 hi array
-// to the lo array.
-static int launch_krp_lp(itcpd_plan* p, bool left, int64_t* Kp, int64_t* lo) {
+static int launch_krp_lp(itcpd_plan* p, bool left, const LpKrp& k) {
     const Side sd = left ? make_side(p, p->s, p->N - p->s, /*rank_fast=*/false)
                          : make_side(p, 0, p->s, /*rank_fast=*/false);
-    int Rk;
-    lp_krp_geometry(p, left, &Rk, Kp);
-    *lo = *Kp * Rk;
-    const dim3 grid((unsigned)cdiv(*lo, 256));
-    const int64_t K = left ? p->MR : p->ML;
-    if (p->prec == ITCPD_BF16X3)
-        hipLaunchKernelGGL(k_krp_lp<true>, grid, dim3(256), 0, p->stream, sd, K, *Kp, (int)p->R, Rk, (void*)p->Kt, p->chk);
-    else
-        hipLaunchKernelGGL(k_krp_lp<false>, grid, dim3(256), 0, p->stream, sd, K, *Kp, (int)p->R, Rk, (void*)p->Kt, p->chk);
+    auto run = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)cdiv(k.Kp * k.Rk, 256)), dim3(256), 0, p->stream, sd,
+                           left ? p->MR : p->ML, k.Kp, (int)p->R, k.Rk, (void*)p->Kt, p->chk);
+    };
+    if (k.kp == 1) run(k_krp_lp<1>);
+    else if (k.kp == 2) run(k_krp_lp<2>);
+    else run(k_krp_lp<4>);
     ITCPD_HIP(hipGetLastError());
     return ITCPD_OK;
 }
@@ -1165,8 +1191,9 @@ static int launch_lp_ring(itcpd_plan* p, MSrc* ms, bool left) {
     const int64_t M = left ? p->ML : p->MR;    // output rows
     const int64_t Mk = left ? p->MR : p->ML;   // reduction length
     const int ny = (int)cdiv(p->R, 128);
-    int64_t Kp, lo;
-    if (int rc = launch_krp_lp(p, left, &Kp, &lo)) return rc;
+    const LpKrp kr = lp_krp(p, left, p->prec);
+    const int64_t lo = kr.Kp * kr.Rk;   // hi to lo
+    if (int rc = launch_krp_lp(p, left, kr)) return rc;
 
     // split-K factor: one workgroup per CU, so the fewest rounds per unit of work,
     // plus a small charge per partial for summing them
@@ -1208,16 +1235,19 @@ static int launch_lp_ring(itcpd_plan* p, MSrc* ms, bool left) {
 
 // Reduced-precision forms of the two GEMMs (FP32 or BF16x3 arithmetic, FP64 output).
 static int launch_gemm_lp(itcpd_plan* p, MSrc* ms, bool left) {
-    if (lp_ring_ok(p, left)) return launch_lp_ring(p, ms, left);
-    const bool bf = p->prec == ITCPD_BF16X3;
+    if (lp_ring_ok(p, left, p->prec)) return launch_lp_ring(p, ms, left);
     GemmLp q{};
     q.left = left;
     q.outs = left ? p->ML : p->MR;
     q.K = left ? p->MR : p->ML;
-    if (int rc = launch_krp_lp(p, left, &q.Kp, &q.lo)) return rc;
-    q.rb = lp_rb(p->R);
+    const LpKrp kr = lp_krp(p, left, p->prec);
+    if (int rc = launch_krp_lp(p, left, kr)) return rc;
+    q.kp = kr.kp;
+    q.Kp = kr.Kp;
+    q.part = kr.Kp * kr.Rk;
+    q.rb = lp_rb(p->R, q.kp);
     q.ny = (int)cdiv(cdiv(p->R, 16), q.rb);
-    q.c = gemm64_cfg(p, q.outs, 1, cdiv(q.K, bf ? 32 : 16), 2, q.ny, lp_big(bf, q.rb));
+    q.c = gemm64_cfg(p, q.outs, 1, cdiv(q.K, q.kp > 1 ? 32 : 16), 2, q.ny, lp_big(q.kp, q.rb));
     const int nout = left ? p->s : p->N - p->s;
     double* dst = nout > 1 ? (left ? p->PL : p->PR) : p->M;
     q.out = q.c.nz > 1 ? p->parts : dst;
