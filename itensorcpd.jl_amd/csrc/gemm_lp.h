@@ -21,11 +21,13 @@
 // lane (c, g) takes the E = 4 or 8 consecutive ones from E g on, a 16-byte run of each of
 // its rows of Kt.  The left form reads VEC consecutive output rows at each index, the right
 // form an E-element run of each of its columns.  The FP32 accumulators are added into FP64
-// ones every 128 reduction indices.  MFMA 16x16x4 step s takes k = k0 + 4 g + s; result:
-// lane (c, g), register v holds rank 4 g + v, output c.
+// ones every stage (FP32) or every 128 indices (BF16x3, whose parts round at 2^-18).  FP32, the
+// relative error of M on Gaussian data and the GEMMs' times below: 16 indices 7.8e-8, 243 / 281;
+// 8 indices 5.9e-8, 279 / 306; 32 1.05e-7, 250 / 301; 128 2.0e-7, 253 / 298.  MFMA 16x16x4
+// step s takes k = k0 + 4 g + s; result: lane (c, g), register v holds rank 4 g + v, output c.
 //
 // Measured per launch (left / right, us) on 150 x 130 x 110 x 90 FP32-stored, rank 48: FP32
-// 256 / 304, BF16x3 in four parts 397 / 429 (280 / 306 in two, where the fourfold operand is not
+// 243 / 281, BF16x3 in four parts 397 / 429 (280 / 306 in two, where the fourfold operand is not
 // read) against 741 / 994 and 1128 / 1534 for the masked register-staged kernels that these
 // replace; 301 x 257 x 199 rank 40, FP32 35 / 40 (97 / 78).  Bound by the
 // tensor's stream (0.77 GB, 127 us at 6.06 TB/s) and, in FP32, the matrix cores (122 us at 152
@@ -95,9 +97,21 @@ struct KrpRun<1> {
     }
 };
 
-// acc += Kt-rows x T over one stage; x[b] holds the lane's E values of output tile b.
+template <int N>
+__device__ __forceinline__ void lp_flush(f4 (&acc)[N], d4 (&tot)[N]) {
+#pragma unroll
+    for (int a = 0; a < N; ++a) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) tot[a][v] += (double)acc[a][v];
+        acc[a] = (f4){0.f, 0.f, 0.f, 0.f};
+    }
+}
+
+// One stage of Kt-rows x T, x[b] the lane's E values of output tile b: BF16x3 into acc, FP32
+// through acc into tot.
 template <int KP, int RB, int MB, int E>
-__device__ __forceinline__ void lp_stage(const KrpRun<KP> (&kr)[RB], const float (&x)[MB][E], f4 (&acc)[RB * MB]) {
+__device__ __forceinline__ void lp_stage(const KrpRun<KP> (&kr)[RB], const float (&x)[MB][E], f4 (&acc)[RB * MB],
+                                         d4 (&tot)[RB * MB]) {
     if constexpr (KP > 1) {
 #pragma unroll
         for (int b = 0; b < MB; ++b) {
@@ -123,16 +137,7 @@ __device__ __forceinline__ void lp_stage(const KrpRun<KP> (&kr)[RB], const float
 #pragma unroll
                 for (int b = 0; b < MB; ++b)
                     acc[a * MB + b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[a].v[s], x[b][s], acc[a * MB + b], 0, 0, 0);
-    }
-}
-
-template <int N>
-__device__ __forceinline__ void lp_flush(f4 (&acc)[N], d4 (&tot)[N]) {
-#pragma unroll
-    for (int a = 0; a < N; ++a) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) tot[a][v] += (double)acc[a][v];
-        acc[a] = (f4){0.f, 0.f, 0.f, 0.f};
+        lp_flush<RB * MB>(acc, tot);
     }
 }
 
@@ -208,8 +213,8 @@ __global__ __launch_bounds__(256, OCC) void k_gemm_lp(const TT* __restrict__ T, 
     };
     int flush = 0;
     auto compute = [&](int buf) {
-        lp_stage<KP, RB, MB, E>(kr[buf], x[buf], acc);
-        if (++flush == FLUSH) {
+        lp_stage<KP, RB, MB, E>(kr[buf], x[buf], acc, tot);
+        if (BF && ++flush == FLUSH) {
             lp_flush<RB * MB>(acc, tot);
             flush = 0;
         }
@@ -245,9 +250,9 @@ __global__ __launch_bounds__(256, OCC) void k_gemm_lp(const TT* __restrict__ T, 
         }
 #pragma unroll
         for (int a = 0; a < RB; ++a) kr[0][a].load(krow[a], part, k);
-        lp_stage<KP, RB, MB, E>(kr[0], x[0], acc);
+        lp_stage<KP, RB, MB, E>(kr[0], x[0], acc, tot);
     }
-    lp_flush<RB * MB>(acc, tot);
+    if (BF) lp_flush<RB * MB>(acc, tot);
 
     if constexpr (KW > 1) {
         __shared__ d4 red[RB * MB][64];
