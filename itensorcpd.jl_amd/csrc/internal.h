@@ -93,6 +93,15 @@ struct KernelTimer {
 
 }  // namespace itcpd
 
+namespace itcpd {
+// An MTTKRP result: M(i, r) = sum_{z < nparts} ptr[z * stride + i + I_n * r].
+struct MSrc {
+    const double* ptr;
+    int nparts;
+    int64_t stride;
+};
+}  // namespace itcpd
+
 struct itcpd_plan {
     int device = 0;
     int num_cu = 256;                          // compute units of the device
@@ -135,6 +144,7 @@ struct itcpd_plan {
     unsigned* counters = nullptr;              // arrival counters of last-block reductions
     int* piv = nullptr;                        // R
     int* finfo = nullptr;                      // [0] = rank, [1] = used fallback, [2] = QR rank
+    itcpd::MSrc side{};                        // the current side's partial: PL, PR or its GEMM's parts
     double* PL = nullptr;                      // ML x Rp partial of the left side (if s > 1)
     float* Kt = nullptr;                       // reduced precision: a side's Khatri-Rao product, rank-major
     double* Wrest = nullptr;                   // a side's Khatri-Rao product or rest weights (rank fastest)
@@ -182,13 +192,6 @@ struct itcpd_plan {
 };
 
 namespace itcpd {
-
-// An MTTKRP result: M(i, r) = sum_{z < nparts} ptr[z * stride + i + I_n * r].
-struct MSrc {
-    const double* ptr;
-    int nparts;
-    int64_t stride;
-};
 
 // error plumbing (api.hip)
 void set_error(const std::string& msg);

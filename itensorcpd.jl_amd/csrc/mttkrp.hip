@@ -296,7 +296,8 @@ __global__ __launch_bounds__(512, 1) void k_lp_ring(const float* __restrict__ T,
 // ------------------------------------------------------- Hadamard-reduce (ttv)
 // M(i, r) = sum_{a<A, b<B} P(a + A*i + A*In*b, r) * Wa(a, r) * Wb(b, r)
 // Wa = product over the side's modes before `pos`, Wb over the modes after it
-// (column-major factors).  P has leading dimension MS.
+// (column-major factors).  P has leading dimension MS and is the sum of np partials, pstride
+// apart, when its GEMM left them (added in increasing order, as k_sum_parts).
 // w[k] *= the product over the side's modes [q0, q1) at the flattened index x[k] (x is used
 // up), mode by mode so that the U loads of one are in flight together.
 template <int U, typename I>
@@ -319,9 +320,9 @@ __device__ __forceinline__ void side_weights(const Side& sd, int q0, int q1, int
 // The side's fastest mode: thread per (i, r), split over b; 8 steps of b in flight.  Bound by
 // HBM when large (512 x 512 x 64: 32 us, 4.2 TB/s).  When small, by the factorisation in the
 // same launch: In = 20, B = 342, R = 24 takes 11.1 us, 14.1 with the steps one by one.
-template <typename I>
-__global__ __launch_bounds__(256) void k_ttv_lead(const double* __restrict__ P, int64_t MS,
-                                                  int64_t In, int R, Side sd, I B, I b_per_split,
+template <bool PARTS, typename I>
+__global__ __launch_bounds__(256) void k_ttv_lead(const double* __restrict__ P, int np, int64_t pstride,
+                                                  int64_t MS, int64_t In, int R, Side sd, I B, I b_per_split,
                                                   double* __restrict__ out, int64_t split_stride,
                                                   FactorJob fj, const DevCheck* __restrict__ chk) {
     if (factor_block(fj)) return;
@@ -343,6 +344,11 @@ __global__ __launch_bounds__(256) void k_ttv_lead(const double* __restrict__ P, 
             pv[k] = Pc[In * x[k]];
             w[k] = 1.0;
         }
+        if constexpr (PARTS)
+#pragma unroll 2
+            for (int z = 1; z < np; ++z)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) pv[k] += Pc[z * pstride + In * x[k]];
         side_weights<8, I>(sd, 1, sd.nm, r, x, w);
 #pragma unroll
         for (int k = 0; k < 8; ++k)
@@ -356,9 +362,9 @@ __global__ __launch_bounds__(256) void k_ttv_lead(const double* __restrict__ P, 
 // the rows.  Bound as k_ttv_lead (512 x 512 x 64: 30 us).  Lanes over a alone, b one by one,
 // left most lanes idle behind one load at a time where A is short: A = 20, In = 19, B = 18,
 // R = 24 took 18.6 us, now 10.8 with its factorisation.
-template <int JW, int U, typename I>
-__global__ __launch_bounds__(256) void k_ttv_inner(const double* __restrict__ P, int64_t MS,
-                                                   int64_t In, int R, Side sd, int pos, I A, I B,
+template <bool PARTS, int JW, int U, typename I>
+__global__ __launch_bounds__(256) void k_ttv_inner(const double* __restrict__ P, int np, int64_t pstride,
+                                                   int64_t MS, int64_t In, int R, Side sd, int pos, I A, I B,
                                                    double* __restrict__ out, FactorJob fj,
                                                    const DevCheck* __restrict__ chk) {
     if (factor_block(fj)) return;
@@ -380,17 +386,25 @@ __global__ __launch_bounds__(256) void k_ttv_inner(const double* __restrict__ P,
     const int64_t skip = (int64_t)A * (In - 1);   // x = a + A b is at x + skip b
     for (I x0 = lane; x0 < n; x0 += 64 * U) {
         I xa[U], xb[U];
+        int64_t off[U];
         double w[U], pv[JW][U];
 #pragma unroll
         for (int k = 0; k < U; ++k) {
             const I x = x0 + 64 * k < n ? x0 + 64 * k : n - 1;
             xb[k] = B > 1 ? x / A : (I)0;
             xa[k] = x - xb[k] * A;
-            const int64_t off = x + skip * xb[k];
+            off[k] = x + skip * xb[k];
 #pragma unroll
-            for (int j = 0; j < JW; ++j) pv[j][k] = Pr[j][off];
+            for (int j = 0; j < JW; ++j) pv[j][k] = Pr[j][off[k]];
             w[k] = 1.0;
         }
+        if constexpr (PARTS)
+#pragma unroll 2
+            for (int z = 1; z < np; ++z)
+#pragma unroll
+                for (int k = 0; k < U; ++k)
+#pragma unroll
+                    for (int j = 0; j < JW; ++j) pv[j][k] += Pr[j][off[k] + z * pstride];
         side_weights<U, I>(sd, 0, pos, r, xa, w);
         side_weights<U, I>(sd, pos + 1, sd.nm, r, xb, w);
 #pragma unroll
@@ -728,6 +742,17 @@ int gemm64_rb(int64_t R, int64_t Rp) {
     return best;
 }
 
+// Split-K partials (n elements each) of a GEMM whose output side has nout modes that need no
+// launch to sum them.  One mode: what the row solves sum as they read M.  More: what its
+// Hadamard-reduces sum as they read the side, when a factorisation runs in their launch and
+// hides it (R <= 64): at most 8, at most 32 MB in all.  Per sweep of
+// 96x88x80x72 rank 16: one sum launch of 5.0 us instead of two of 6.6.
+int64_t unsummed_parts(const itcpd_plan* p, int nout, int64_t n, int factor_mode) {
+    if (nout == 1) return p->RT ? SOLVE_MAX_PARTS : 1;
+    if (p->R > 64 || p->v_override || factor_mode >= 0) return 1;
+    return std::max<int64_t>(1, std::min<int64_t>(8, ((int64_t)1 << 22) / n));
+}
+
 struct Gemm64Cfg {
     int MB, KW;
     int64_t per, nz;    // reduction units (4-steps / 16-index stages) per split, splits
@@ -735,13 +760,14 @@ struct Gemm64Cfg {
 // Tiles of 16 MB outputs.  With at least three workgroups of four such tiles per CU every
 // wave takes its own tile and no reduction is split (KW = 1).  Otherwise the four waves of a
 // workgroup split one tile's reduction, and so do nz workgroups, for the fewest rounds of
-// two workgroups per CU per unit of work plus a charge for the partials' traffic; a wave
+// two workgroups per CU per unit of work plus a charge for the partials' traffic and, above
+// `unsummed` of them, 6 us (30 MB of the tensor's stream) for the launch that sums them; a wave
 // keeps at least `min_units`.  16-output tiles are taken when the large ones cannot give
 // every CU a workgroup, or when a slab has fewer rows than one (the large left tile is moved
 // back to end at the slab's last row).  Measured, us (KW = 1 / KW = 4): 301 x (257) x 199
 // rank 37, 398 workgroups, 60 / 42; 512 x (512) x 512 rank 64, 1024 workgroups, 338 / 347.
 Gemm64Cfg gemm64_cfg(const itcpd_plan* p, int64_t M, int64_t slabs, int64_t units, int64_t min_units, int ny,
-                     int big) {
+                     int big, int64_t unsummed) {
     Gemm64Cfg c{};
     const int64_t slots = 2 * (int64_t)p->num_cu;
     const int64_t out_elems = M * slabs * p->R;
@@ -756,7 +782,7 @@ Gemm64Cfg gemm64_cfg(const itcpd_plan* p, int64_t M, int64_t slabs, int64_t unit
         for (int64_t z = 1; z <= 512; ++z) {
             if (z > 1 && (units < 4 * min_units * z || (size_t)(z * out_elems) > p->parts_elems)) break;
             const double cost = (double)cdiv(base * z, slots) * (double)slots / (double)(base * z) +
-                                (z > 1 ? 16.0 * (double)(z * out_elems) / tbytes : 0.0);
+                                (z > 1 ? 16.0 * (double)(z * out_elems) / tbytes : 0.0) + (z > unsummed ? 3e7 / tbytes : 0.0);
             if (cost < best - 1e-9) { best = cost; nz = z; }
         }
         c = Gemm64Cfg{mb, 4, cdiv(units, nz), nz};
@@ -799,6 +825,7 @@ struct Gemm64 {
     int64_t M, slabs, K;   // outputs per slab, slabs (1 for the right form)
     Krp64 kp;
     int nm, rb, ny;
+    int64_t unsummed;      // splits whose partials no launch sums
     Gemm64Cfg c;
     double* out;
 };
@@ -874,8 +901,8 @@ void dispatch_gemm64(itcpd_plan* p, const Gemm64& q) {
 int run_gemm64(itcpd_plan* p, Gemm64& q, double* dst) {
     q.rb = gemm64_rb(p->R, p->Rp);
     q.ny = (int)cdiv(cdiv(p->R, 16), q.rb);
-    q.c = q.left ? gemm64_cfg(p, q.M, q.slabs, cdiv(q.K, 4), 4, q.ny, left64_big(q.rb))
-                 : gemm64_cfg(p, q.M, 1, cdiv(q.K, 16), 2, q.ny, right64_big(q.rb));
+    q.c = q.left ? gemm64_cfg(p, q.M, q.slabs, cdiv(q.K, 4), 4, q.ny, left64_big(q.rb), q.unsummed)
+                 : gemm64_cfg(p, q.M, 1, cdiv(q.K, 16), 2, q.ny, right64_big(q.rb), q.unsummed);
     q.out = q.c.nz > 1 ? p->parts : dst;
     Timed tm(p, q.left ? 0 : 1, 2.0 * (double)p->ML * (double)p->MR * (double)p->R,
              (double)p->ML * (double)p->MR * p->elt_bytes);
@@ -967,9 +994,20 @@ namespace {
 // Hands split partials to the consumer, or sums them into dst when there are many.
 // factor_mode >= 0: that mode's factorisation rides the partial-sum launch, else
 // (no sum launched, R > 64) runs as its own launch after the producer.
+//
+// The partials of a side with more modes (consumer_sums false) stay as they are up to
+// unsummed_parts.
 int finish_parts(itcpd_plan* p, double* parts, int64_t nz, int64_t n, double* dst, MSrc* ms,
                  bool consumer_sums, int factor_mode = -1, bool fallback_only = false) {
     MSrc pm{parts, (int)nz, n};
+    if (!consumer_sums) {
+        const bool keep = nz > 1 && nz <= unsummed_parts(p, 2, n, factor_mode);
+        p->side = keep ? pm : MSrc{dst, 1, n};
+        if (keep) {
+            *ms = pm;
+            return ITCPD_OK;
+        }
+    }
     if (nz == 1 || (consumer_sums && nz <= MAX_CONSUMER_PARTS)) {
         *ms = nz == 1 ? MSrc{dst, 1, n} : pm;
         return factor_mode >= 0 ? launch_factor(p, factor_mode) : ITCPD_OK;
@@ -981,7 +1019,7 @@ int finish_parts(itcpd_plan* p, double* parts, int64_t nz, int64_t n, double* ds
 
 // Left GEMM: rows = left multi-index (ML), reduction = right side.  Produces PL
 // (s > 1) or the M of mode 0 (s == 1).
-static int launch_ttv(itcpd_plan* p, const double* P, int64_t MS, const Side& sd, int pos, MSrc* ms,
+static int launch_ttv(itcpd_plan* p, const MSrc& P, int64_t MS, const Side& sd, int pos, MSrc* ms,
                       int factor_mode);
 int launch_left_gemm_lp(itcpd_plan* p, MSrc* ms);
 int launch_right_gemm_lp(itcpd_plan* p, MSrc* ms);
@@ -1016,6 +1054,7 @@ static int launch_gemm64(itcpd_plan* p, MSrc* ms, bool left, int factor_mode) {
     q.K = left ? p->MR : p->ML;
     int rc;
     if ((rc = krp64_of(p, sd, q.K, &q.kp, &q.nm))) return rc;
+    q.unsummed = unsummed_parts(p, nout, q.M * p->R, factor_mode);
     double* dst = nout > 1 ? (left ? p->PL : p->PR) : p->M;
     if ((rc = run_gemm64(p, q, dst))) return rc;
     return finish_parts(p, p->parts, q.c.nz, q.M * p->R, dst, ms, nout == 1, factor_mode);
@@ -1051,6 +1090,7 @@ int launch_tree3_gemm(itcpd_plan* p, int c) {
     q.K = p->dims[c];
     q.kp = Krp64{p->At[c], p->At[c], p->dims[c], (int)p->Rp};
     q.nm = 1;
+    q.unsummed = 1;
     int rc;
     if ((rc = run_gemm64(p, q, p->P3))) return rc;
     if (q.c.nz == 1) return ITCPD_OK;
@@ -1068,7 +1108,7 @@ int launch_tree3_ttv(itcpd_plan* p, int mode, int c, MSrc* ms, int factor_mode) 
         sd.fac[q] = p->A[m];
         ++q;
     }
-    return launch_ttv(p, p->P3, sd.dim[0] * sd.dim[1], sd, pos, ms, factor_mode);
+    return launch_ttv(p, MSrc{p->P3, 1, 0}, sd.dim[0] * sd.dim[1], sd, pos, ms, factor_mode);
 }
 
 int launch_left_gemm_impl(itcpd_plan* p, MSrc* ms) {
@@ -1245,10 +1285,11 @@ static int launch_gemm_lp(itcpd_plan* p, MSrc* ms, bool left) {
     q.kp = kr.kp;
     q.Kp = kr.Kp;
     q.part = kr.Kp * kr.Rk;
+    const int nout = left ? p->s : p->N - p->s;
     q.rb = lp_rb(p->R, q.kp);
     q.ny = (int)cdiv(cdiv(p->R, 16), q.rb);
-    q.c = gemm64_cfg(p, q.outs, 1, cdiv(q.K, q.kp > 1 ? 32 : 16), 2, q.ny, lp_big(q.kp, q.rb));
-    const int nout = left ? p->s : p->N - p->s;
+    q.c = gemm64_cfg(p, q.outs, 1, cdiv(q.K, q.kp > 1 ? 32 : 16), 2, q.ny, lp_big(q.kp, q.rb),
+                     unsummed_parts(p, nout, q.outs * p->R, -1));
     double* dst = nout > 1 ? (left ? p->PL : p->PR) : p->M;
     q.out = q.c.nz > 1 ? p->parts : dst;
     {
@@ -1266,13 +1307,13 @@ int launch_side_ttv(itcpd_plan* p, int mode, MSrc* ms, int factor_mode) {
     const bool left = mode < p->s;
     const int first = left ? 0 : p->s;
     const Side sd = make_side(p, first, left ? p->s : p->N - p->s, /*rank_fast=*/false);
-    return launch_ttv(p, left ? p->PL : p->PR, left ? p->ML : p->MR, sd, mode - first, ms, factor_mode);
+    return launch_ttv(p, p->side, left ? p->ML : p->MR, sd, mode - first, ms, factor_mode);
 }
 
 // M of the side's mode `pos` from the partial P (leading dimension MS) by a
 // Hadamard-reduce.  With factor_mode >= 0 that mode's factorisation runs in an extra
 // workgroup of the same launch when it can (R <= 64), else it is launched right after.
-static int launch_ttv(itcpd_plan* p, const double* P, int64_t MS, const Side& sd, int pos, MSrc* ms,
+static int launch_ttv(itcpd_plan* p, const MSrc& P, int64_t MS, const Side& sd, int pos, MSrc* ms,
                       int factor_mode) {
     const int nm = sd.nm;
     int64_t A = 1, B = 1;
@@ -1287,29 +1328,36 @@ static int launch_ttv(itcpd_plan* p, const double* P, int64_t MS, const Side& sd
     if (pos == 0) {
         int64_t nz = 1;
         const int64_t blocks = cdiv(nout, 256);
-        while (blocks * nz < 2048 && B / (nz * 2) >= 16 && (size_t)(nz * 2 * nout) <= p->parts_elems &&
+        // behind the side's own partials, which the next modes still read
+        const int64_t taken = P.nparts > 1 ? P.nparts * P.stride : 0;
+        double* const parts = p->parts + taken;
+        while (blocks * nz < 2048 && B / (nz * 2) >= 16 && (size_t)(taken + nz * 2 * nout) <= p->parts_elems &&
                nz * 2 <= MAX_CONSUMER_PARTS)
             nz *= 2;
         const int64_t bper = cdiv(B, nz);
         nz = cdiv(B, bper);
-        double* out = nz > 1 ? p->parts : p->M;
+        double* out = nz > 1 ? parts : p->M;
         const dim3 grid((unsigned)(blocks + fj.on), (unsigned)nz);
-        if (small)
-            hipLaunchKernelGGL(k_ttv_lead<int>, grid, dim3(256), lds, p->stream, P, MS, In, (int)p->R, sd, (int)B,
-                               (int)bper, out, nout, fj, p->chk);
-        else
-            hipLaunchKernelGGL(k_ttv_lead<int64_t>, grid, dim3(256), lds, p->stream, P, MS, In, (int)p->R, sd, B,
-                               bper, out, nout, fj, p->chk);
+        auto run = [&](auto kern, auto b, auto per) {
+            hipLaunchKernelGGL(kern, grid, dim3(256), lds, p->stream, P.ptr, P.nparts, P.stride, MS, In, (int)p->R, sd,
+                               b, per, out, nout, fj, p->chk);
+        };
+        if (!small) run(k_ttv_lead<true, int64_t>, B, bper);
+        else if (P.nparts > 1) run(k_ttv_lead<true, int>, (int)B, (int)bper);
+        else run(k_ttv_lead<false, int>, (int)B, (int)bper);
         ITCPD_HIP(hipGetLastError());
-        rc = finish_parts(p, p->parts, nz, nout, p->M, ms, true);
+        rc = finish_parts(p, parts, nz, nout, p->M, ms, true);
     } else {
         auto run = [&](auto kern, int jw, auto a, auto b) {
             hipLaunchKernelGGL(kern, dim3((unsigned)(cdiv(cdiv(In, jw) * p->R, 4) + fj.on)), dim3(256), lds,
-                               p->stream, P, MS, In, (int)p->R, sd, pos, a, b, p->M, fj, p->chk);
+                               p->stream, P.ptr, P.nparts, P.stride, MS, In, (int)p->R, sd, pos, a, b, p->M, fj, p->chk);
         };
-        if (!small) run(k_ttv_inner<4, 4, int64_t>, 4, A, B);
-        else if (A * B <= 128) run(k_ttv_inner<4, 2, int>, 4, (int)A, (int)B);
-        else run(k_ttv_inner<4, 4, int>, 4, (int)A, (int)B);
+        const bool shrt = A * B <= 128, parts = P.nparts > 1;
+        if (!small) run(k_ttv_inner<true, 4, 4, int64_t>, 4, A, B);
+        else if (shrt && parts) run(k_ttv_inner<true, 4, 2, int>, 4, (int)A, (int)B);
+        else if (shrt) run(k_ttv_inner<false, 4, 2, int>, 4, (int)A, (int)B);
+        else if (parts) run(k_ttv_inner<true, 4, 4, int>, 4, (int)A, (int)B);
+        else run(k_ttv_inner<false, 4, 4, int>, 4, (int)A, (int)B);
         ITCPD_HIP(hipGetLastError());
         *ms = MSrc{p->M, 1, nout};
     }
