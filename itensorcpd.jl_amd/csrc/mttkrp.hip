@@ -1067,8 +1067,8 @@ static int launch_gemm64(itcpd_plan* p, MSrc* ms, bool left, int factor_mode) {
 // Contracting mode 2 or mode 1 is a left GEMM (mode 1: a batch of K slabs), mode 0 a right
 // one, each against one factor.  The price is one and a half partials written and three read
 // per sweep instead of one and two: taken when half a pass over T (the tensor's read or
-// 2 n R flops, at the rates the GEMMs reach) costs more than that.  Per sweep, us: 512^3
-// rank 64 684 (755 with two passes); 301 x 257 x 199 rank 37 166 (206).
+// 2 n R flops, at the rates the GEMMs reach) costs more than that.  A sweep with and
+// without, us: 512^3 rank 64 653 / 759; 301 x 257 x 199 rank 37 178 / 201.
 bool tree3_pays(const itcpd_plan* p) {
     if (p->N != 3 || p->prec != ITCPD_FP64) return false;
     const double n = (double)p->ML * (double)p->MR;
