@@ -327,8 +327,7 @@ int itcpd_plan_create(itcpd_plan** out, int32_t order, const int64_t* dims, int6
     } else {
         const int64_t nb = cdiv(R, 64);
         ar.add(&p->inv_buf, (size_t)(2 * 4096 * nb * nb));
-        ar.add(&p->inv_P, (size_t)2 * 4096);
-        ar.add(&p->inv_stat, (size_t)(3 * nb * nb + nb));
+        ar.add(&p->inv_stat, inv_stat_elems(R));
     }
     ar.add(&p->invdiag, (size_t)R);
     ar.add(&p->qr_aux, (size_t)(R * R + 4 * R));

@@ -7,8 +7,9 @@
 namespace itcpd {
 
 constexpr size_t FACTOR64_LDS = (size_t)(2 * 64 * 66) * 8;
-// LDS of the unpivoted form alone: four broadcast rows and 16 doubles of reductions
-constexpr size_t FACTOR64_UNPIV_LDS = (size_t)(4 * 128 + 16) * 8;
+// LDS of the unpivoted form alone: W (the sweeps' rows before it), D^-1, 16 doubles of reductions
+constexpr int FACTOR64_UNPIV = 64 * 64 + 64 + 16;
+constexpr size_t FACTOR64_UNPIV_LDS = (size_t)FACTOR64_UNPIV * 8;
 
 // LDS written by lanes of one wave, then read by other lanes of the same wave: the wave's LDS
 // operations complete in order, so only the compiler must keep them so.
@@ -18,33 +19,43 @@ __device__ __forceinline__ void lds_wave_order() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Inverse of a symmetric positive definite n x n matrix by symmetric sweeps, in registers.
-// A thread holds 16 rows (16 grp ..) of one column col; rows and columns >= n are zero.
-// Sweeping index k, with r the k-th row (= column) and d = r_k: the element (i, l) takes
-// a - r_i r_l / d, row and column k become r / d and (k, k) -1 / d.  After n sweeps the matrix
-// is -A^-1; it stays symmetric throughout, so the rows being swept, handed to every thread
-// through LDS, are all that a step needs.  The d are the pivots of the unpivoted
-// factorisation; false when one was not > 0.
+// The triangular half of the inverse of a symmetric positive definite n x n matrix A = L D L^T:
+// W = L^-1 and the reciprocals of D, in registers.  A thread holds 16 rows (16 grp ..) of one
+// column col; rows and columns >= n are zero.  Eliminating index k, with r the k-th row and d =
+// r_k: the rows i > k take a_il - r_i r_l / d (r_i, their column k, is their row k by symmetry),
+// where column k counts as the identity's (r_k = 1, a_ik = 0 before).  So the columns below k
+// collect W and those above the Schur complement, row k is final, and the row being eliminated,
+// handed to every thread through LDS, is all that a step needs.  false when a pivot was not > low.
 //
-// A step sweeps k and k + 1 together: p, q their rows, B = [d1 c; c e] their 2 x 2 block, (T1,
-// T2) = B^-1 (p_l, q_l): the element (i, l) takes a - p_i T1 - q_i T2, rows k and k + 1 become
-// T1 and T2.  With an odd n the index n is a 1 on the diagonal.  The step's critical chain is
-// 1 / det B, the next two rows' multiply-adds and their way through LDS: those rows go first
-// and their reads are issued before the other rows are updated; d1 and e come from a running
-// copy of the diagonal by readlane, not from the rows.
+// Rows already eliminated take no part.  Updating them too (Gauss-Jordan) would leave A^-1 in
+// place without a product, but its rows of size 1 / lambda_min then pass through every later
+// update and the error of M A^-1, M = X A, grows with cond(A)^2: 1e-7 at cond(A) = 1e6 and
+// wrong in the first digit at 1e9, where W^T D^-1 W, as the triangular inverse of a Cholesky
+// factor, has 5e-11 and 4e-7.
+//
+// A step eliminates k and k + 1 together: p, q their rows, d1 = p_k, c = p_{k+1}, q' = q - (c /
+// d1) p, the second pivot e' = q'_{k+1} = det / d1, det = d1 e - c^2, so that both reciprocals
+// start at once: the element (i, l) takes a - p_i p_l / d1 - q'_i q'_l / e'.  With an odd n the
+// index n is a 1 on the diagonal.  The step's critical chain is 1 / det, the next two rows'
+// multiply-adds and their way through LDS: those rows go first and their reads are issued
+// before the other rows are updated; d1 and e come from a running copy of the diagonal by
+// readlane, not from the rows.
 //
 // The loop body is short on purpose: unrolled over all steps it is straight-line code that
 // every launch fetches anew (27 us at n = 64).  So that registers are not indexed by k, every
 // step rotates the rows by two (position j holds row 16 grp + (j + k) mod 16, the rows being
-// swept sit at positions 0 and 1, the next ones at 2 and 3), and each row in LDS keeps its
-// 16-entry groups twice in a row, so a rotated group is one run.
+// eliminated sit at positions 0 and 1, the next ones at 2 and 3).  Each row is in LDS by column,
+// and once more with its 16-entry groups twice in a row, so a rotated group is one run, and with
+// zeros for the rows already eliminated.
 //
 // WAVES = 1: one wave, n <= 32, grp = lane >> 5, col = lane & 31, rows in LDS order, no
 // barrier; WAVES = 4: a 256-thread workgroup, n <= 64, grp = wave, col = lane, one barrier a
 // step (two row buffers), and p_i, q_i, which a wave's lanes share, by readlane from one
 // LDS read (delivered to every lane they would take 512 cycles of the LDS port a step).
-// rows: SWEEP_ROWS doubles of LDS.  On return position j holds row sweep_row(n, grp, j).
-constexpr int SWEEP_ROWS = 4 * 128;
+// rows: SWEEP_ROWS doubles of LDS.  KEEP_L: Lt[k ld + i] = L_ik, i > k, in LDS.  On return position
+// j holds row sweep_row(n, grp, j) of W and rd the reciprocal of pivot col.
+constexpr int SWEEP_BUF = 384;   // rows p, q by column and their runs of 128
+constexpr int SWEEP_ROWS = 2 * SWEEP_BUF;
 
 __device__ __forceinline__ int sweep_row(int n, int grp, int j) { return 16 * grp + ((j + n + (n & 1)) & 15); }
 
@@ -79,16 +90,19 @@ __device__ __forceinline__ double newton_rcp(double d) {
     return fma(y, fma(e, e, e), y);
 }
 
-template <int WAVES>
-__device__ __forceinline__ bool sweep_inverse(double (&a)[16], int n, int grp, int col, double* rows) {
+template <int WAVES, bool KEEP_L>
+__device__ __forceinline__ bool sweep_triangular(double (&a)[16], int n, int grp, int col, double low, double* rows,
+                                                 double& rd, double* Lt = nullptr, int ld = 0) {
     auto sync = [] {
         if (WAVES == 1) lds_wave_order();
         else __syncthreads();
     };
-    const int at = 32 * (col >> 4) + (col & 15);   // this column's place in a row in LDS
-    auto put = [&](double* row, double v) {
-        row[at] = v;
-        row[at + 16] = v;
+    const int at = 32 * (col >> 4) + (col & 15);   // this column's place in a row's runs
+    auto put = [&](double* buf, int q, int k, double v) {   // row q of the pair k, k + 1
+        const double run = col > k + 1 ? v : 0.0;
+        buf[64 * q + col] = v;
+        buf[128 + 128 * q + at] = run;
+        buf[128 + 128 * q + at + 16] = run;
     };
     double dg = 0.0;
 #pragma unroll
@@ -97,22 +111,24 @@ __device__ __forceinline__ bool sweep_inverse(double (&a)[16], int n, int grp, i
         a[i] = here && (n & 1) && col == n ? 1.0 : a[i];
         dg = here ? a[i] : dg;
     }
-    if (col >> 4 == grp) rows[256 + at] = dg;
+    if (col >> 4 == grp) rows[SWEEP_BUF + col] = dg;
     if (grp == 0) {
-        put(rows, a[0]);
-        put(rows + 128, a[1]);
+        put(rows, 0, 0, a[0]);
+        put(rows, 1, 0, a[1]);
     }
     sync();
-    dg = rows[256 + at];
+    dg = rows[SWEEP_BUF + col];
+    rd = 0.0;
     const int lane = threadIdx.x & 63;
     // the rows' entries of this column and of this group
     double pl, ql;
-    auto fetch = [&](const double* row, int k, double (&p)[16], double (&q)[16]) {
-        const double* run = row + 32 * grp + (k & 15);
-        pl = row[at];
-        ql = row[128 + at];
+    auto fetch = [&](const double* buf, int k, double (&p)[16], double (&q)[16]) {
+        const double* run = buf + 128 + 32 * grp + (k & 15);
+        pl = buf[col];
+        ql = buf[64 + col];
         if (WAVES == 4) {
-            p[0] = run[(lane & 15) + 8 * (lane & 16)];   // lane j: p_j, lane 16 + j: q_j
+            p[0] = run[lane & 15];
+            q[0] = run[128 + (lane & 15)];
         } else {
 #pragma unroll
             for (int j = 0; j < 16; ++j) {
@@ -129,34 +145,56 @@ __device__ __forceinline__ bool sweep_inverse(double (&a)[16], int n, int grp, i
     auto step = [&](int k, double (&p)[16], double (&q)[16], double (&pn)[16], double (&qn)[16]) {
         const double d1 = lane_double(dg, k), e = lane_double(dg, k + 1), c = lane_double(pl, k + 1);
         const double det = fma(d1, e, -c * c);
-        pos = pos && d1 > 0.0 && det > 0.0;
-        const double inv = newton_rcp(det);
-        double t1 = fma(e, pl, -c * ql) * inv, t2 = fma(d1, ql, -c * pl) * inv;
-        dg = fma(-pl, t1, fma(-ql, t2, dg));
+        pos = pos && d1 > low && det > low * d1;
+        const double r1 = newton_rcp(d1), r2 = d1 * newton_rcp(det), m = c * r1;
+        const double q2 = fma(-m, pl, ql);
+        double t1 = pl * r1, t2 = q2 * r2;
         const bool c1 = col == k, c2 = col == k + 1;
-        t1 = c1 ? -e * inv : (c2 ? c * inv : t1);
-        t2 = c1 ? c * inv : (c2 ? -d1 * inv : t2);
+        const double l0 = t1, l1 = t2;   // above the diagonal, L's columns k and k + 1
+        // the diagonal as the rows' own updates; four waves after the next rows, which wait for less
+        if (WAVES == 1) dg = fma(-q2, l1, fma(-pl, l0, dg));
+        t1 = c1 ? r1 : (c2 ? 0.0 : t1);
+        t2 = c1 ? -m * r2 : (c2 ? r2 : t2);
         const double keep = c1 || c2 ? 0.0 : 1.0;
-        if (WAVES == 4) {
-            const double pq = p[0];
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                p[j] = lane_double(pq, j);
-                q[j] = lane_double(pq, 16 + j);
+        const double ps = p[0], qs = fma(-m, p[0], q[0]);
+        auto multiplier = [&](int j) {
+            if (WAVES == 4) {
+                p[j] = lane_double(ps, j);
+                q[j] = lane_double(qs, j);
+            } else {
+                q[j] = fma(-m, p[j], q[j]);
             }
-        }
-        double* next = rows + 256 * ((k / 2 + 1) & 1);
+        };
+        multiplier(2);
+        multiplier(3);
+        double* next = rows + SWEEP_BUF * ((k / 2 + 1) & 1);
         if ((k + 2) >> 4 == grp) {
             const double v2 = fma(-p[2], t1, a[2] * keep), v3 = fma(-p[3], t1, a[3] * keep);
-            put(next, fma(-q[2], t2, v2));
-            put(next + 128, fma(-q[3], t2, v3));
+            put(next, 0, k + 2, fma(-q[2], t2, v2));
+            put(next, 1, k + 2, fma(-q[3], t2, v3));
+        }
+        if (WAVES == 4) {
+            __builtin_amdgcn_sched_barrier(0);
+            dg = fma(-q2, l1, fma(-pl, l0, dg));
+        }
+        // rows k and k + 1 of W: their multipliers are zero, so they are final from here on
+        const bool own = k >> 4 == grp, below = col < k;
+        a[0] = own ? (c1 ? 1.0 : (below ? pl : 0.0)) : a[0] * keep;
+        a[1] = own ? (c1 ? -m : (c2 ? 1.0 : (below ? q2 : 0.0))) : a[1] * keep;
+        rd = c1 ? r1 : (c2 ? r2 : rd);
+        if (KEEP_L && own) {
+            Lt[k * ld + col] = l0;
+            Lt[(k + 1) * ld + col] = l1;
         }
         sync();
         fetch(next, k + 2, pn, qn);
         // a <- a keep - p t1 - q t2 in passes of 16 independent operations
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) a[j] *= keep;
+        for (int j = 0; j < 16; ++j)
+            if (j != 2 && j != 3) multiplier(j);
+#pragma unroll
+        for (int j = 2; j < 16; ++j) a[j] *= keep;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < 16; ++j) a[j] = fma(-p[j], t1, a[j]);
@@ -164,12 +202,11 @@ __device__ __forceinline__ bool sweep_inverse(double (&a)[16], int n, int grp, i
 #pragma unroll
         for (int j = 0; j < 16; ++j) a[j] = fma(-q[j], t2, a[j]);
         __builtin_amdgcn_sched_barrier(0);
-        const bool own = k >> 4 == grp;
-        const double r0 = own ? t1 : a[0], r1 = own ? t2 : a[1];
+        const double x0 = a[0], x1 = a[1];
 #pragma unroll
         for (int j = 0; j < 14; ++j) a[j] = a[j + 2];
-        a[14] = r0;
-        a[15] = r1;
+        a[14] = x0;
+        a[15] = x1;
     };
 #pragma unroll 1
     for (int k = 0;; k += 4) {
@@ -181,6 +218,11 @@ __device__ __forceinline__ bool sweep_inverse(double (&a)[16], int n, int grp, i
     return pos;
 }
 
+// W = L^-1 in LDS as the operand of W^T D^-1 W: entry (r, k) of rows of ld (32 or 64) doubles,
+// odd rows with their 16-column groups swapped in pairs, so that two rows of a read meet
+// distinct banks.
+__device__ __forceinline__ int tri_at(int ld, int r, int k) { return r * ld + (k ^ ((r & 1) << 4)); }
+
 // Unpivoted V^-1 for the R <= 64 row solves (one 256-thread workgroup; the first wave alone
 // up to R = 32).
 //
@@ -190,22 +232,23 @@ __device__ __forceinline__ bool sweep_inverse(double (&a)[16], int n, int grp, i
 // 1 / ||V^-1||_F.  The computed inverse is trusted while ||V||_F ||V^-1||_F < cond_max;
 // the bound must exceed 2 tol plus the pivots' rounding (64 R eps max V_ii); every
 // unpivoted pivot must be > 0.  Then the solution (the unique minimiser) is the
-// pivoted path's up to rounding, and V^-1 and finfo are written; otherwise it returns
+// pivoted path's up to rounding (eps cond(V), the form's backward error), and V^-1 and finfo are written; otherwise it returns
 // false and writes nothing but V^-1 (which the caller's pivoted path overwrites or leaves
 // unused).  Uniform result.
 //
-// Bound by its chain of R / 2 steps on one wave per SIMD (about 165 instructions of 5 cycles).
-// Gram loads to V^-1, us: R = 1 3.9, 10 5.2, 24 7.7, 37 13.6, 64 19.7; the blocked Cholesky,
-// triangular inverse and product of them that this replaces took 11 (R = 10), 17 (R = 24), 19
-// (R = 37), 29 (R = 64) in the Hadamard-reduce launch that carries them, where this takes 7,
-// 14, 17 and 28.
+// Bound by its chain of R / 2 steps, 0.5 us each, on one wave per SIMD.  The Hadamard-reduce of
+// 64 x 64 x 64 that carries it takes, us: R = 10 7.2, 16 8.6, 24 11.5, 37 17.9, 64 25.5 (Gauss-Jordan
+// 6.6, 7.8, 9.4, 16.2, 22.8; the blocked Cholesky, triangular inverse and product of them
+// before that 11 at R = 10, 17 at 24, 19 at 37, 29 at 64).
+// SMALL = false: R > 32 only, in a kernel whose registers the one-wave form would not fit.
+template <bool SMALL = true>
 __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, int R, double tol,
                                                    double* __restrict__ Vinv, int* __restrict__ finfo,
                                                    double* S, double cond_max = 1e12) {
-    double* red = S + SWEEP_ROWS;   // behind the broadcast rows
+    double* red = S + 64 * 64 + 64;   // behind W (before it the sweeps' rows) and D^-1
     const int t = threadIdx.x, l = t & 63;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-    const bool one = R <= 32;
+    const bool one = SMALL && R <= 32;
     if (!one || w == 0) {
         const int grp = one ? l >> 5 : w, col = one ? l & 31 : l;
         // V in the mode order of the pivoted path's Hadamard; two modes' loads in flight
@@ -238,13 +281,90 @@ __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, 
             vsq = fma(a[i], a[i], vsq);
             if (r == col) dmax = fmax(dmax, a[i]);
         }
-        const bool pos = one ? sweep_inverse<1>(a, R, grp, col, S) : sweep_inverse<4>(a, R, grp, col, S);
+        double rd;
+        const bool pos = one ? sweep_triangular<1, false>(a, R, grp, col, 0.0, S, rd)
+                             : sweep_triangular<4, false>(a, R, grp, col, 0.0, S, rd);
+        // V^-1 = W^T D^-1 W by upper tiles, 16 rows of W (4 k-steps) read ahead of their products
+        double* dinv = S + 64 * 64;
+        const int ld = one ? 32 : 64, c = l & 15, g = l >> 4;
+        auto sync = [&] {
+            if (one) lds_wave_order();
+            else __syncthreads();
+        };
+        sync();
+        if (grp == 0) dinv[col] = rd;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int r = sweep_row(R, grp, i);
-            if (r < R && col < R) {
-                Vinv[r * R + col] = -a[i];
-                zsq = fma(a[i], a[i], zsq);
+        for (int i = 0; i < 16; ++i) S[tri_at(ld, sweep_row(R, grp, i), col)] = a[i];
+        sync();
+        auto tile = [&](int ta, int tb, const d4& z) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int ra = 16 * ta + g + 4 * v, rb = 16 * tb + c;
+                if (ra >= R || rb >= R) continue;
+                Vinv[ra * R + rb] = z[v];
+                if (ta != tb) Vinv[rb * R + ra] = z[v];
+                zsq = fma(ta == tb ? z[v] : 2.0 * z[v], z[v], zsq);
+            }
+        };
+        // rows 16 kb .. of a column block of W, and the same times D^-1
+        auto load = [&](double (&x)[4], int kb, int t) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) x[s] = S[tri_at(ld, 16 * kb + 4 * s + g, 16 * t + c)];
+        };
+        auto scaled = [&](const double (&x)[4], int kb, double (&y)[4]) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) y[s] = x[s] * dinv[16 * kb + 4 * s + g];
+        };
+        auto product = [&](const double (&x)[4], const double (&y)[4], d4& z) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) z = mfma_f64(x[s], y[s], z);
+        };
+        const d4 zero = (d4){0.0, 0.0, 0.0, 0.0};
+        if (one) {
+            double x00[4], x10[4], x11[4], y[4];
+            d4 z00 = zero, z01 = zero, z11 = zero;
+            load(x00, 0, 0);
+            load(x10, 1, 0);
+            load(x11, 1, 1);
+            scaled(x00, 0, y);
+            product(x00, y, z00);
+            if (R > 16) {
+                scaled(x11, 1, y);
+                product(x10, y, z01);
+                product(x11, y, z11);
+                scaled(x10, 1, y);
+                product(x10, y, z00);
+                tile(0, 1, z01);
+                tile(1, 1, z11);
+            }
+            tile(0, 0, z00);
+        } else {
+            constexpr int ZT[4][3][2] = {{{0, 0}, {0, 3}, {-1, -1}},
+                                         {{0, 1}, {1, 3}, {2, 3}},
+                                         {{1, 1}, {0, 2}, {-1, -1}},
+                                         {{1, 2}, {2, 2}, {3, 3}}};   // 20 k-steps a wave
+            const int nt = (R + 15) / 16;
+#pragma unroll 1
+            for (int q = 0; q < 3; ++q) {
+                const int ta = ZT[w][q][0], tb = ZT[w][q][1];
+                if (ta < 0 || tb >= nt) continue;
+                d4 z = zero;
+                double x0[4], w0[4], x1[4], w1[4], y[4];
+                load(x0, tb, ta);
+                load(w0, tb, tb);
+                for (int kb = tb; kb < nt; kb += 2) {
+                    const int k1 = kb + 1 < 4 ? kb + 1 : 3, k2 = kb + 2 < 4 ? kb + 2 : 3;   // past the last: not used
+                    load(x1, k1, ta);
+                    load(w1, k1, tb);
+                    scaled(w0, kb, y);
+                    product(x0, y, z);
+                    if (kb + 1 >= nt) break;
+                    load(x0, k2, ta);
+                    load(w0, k2, tb);
+                    scaled(w1, k1, y);
+                    product(x1, y, z);
+                }
+                tile(ta, tb, z);
             }
         }
         vsq = wave_sum_dpp(vsq);

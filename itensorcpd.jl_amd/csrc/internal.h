@@ -137,7 +137,6 @@ struct itcpd_plan {
     double* invdiag = nullptr;                 // R: 1 / U(j,j) of the pivoted Cholesky
     double* Upad = nullptr;                    // R <= 64: V^-1 (R x R) from the factor kernel
     double* inv_buf = nullptr;                 // R > 64: two (64 nb)^2 buffers of the blocked inverse
-    double* inv_P = nullptr;                   // the pivot block's inverse (two of 64 x 64)
     double* inv_stat = nullptr;                // norms and flags of the certificate
     int RT = 0;                                // 16, 32 or 64 for R <= 64, else 0
     double* Msum = nullptr;                    // maxI x R: summed MTTKRP of the last mode (fit)
@@ -227,6 +226,7 @@ int launch_update_mode(itcpd_plan* p, int mode, bool fit_after, const double* Ms
                        int64_t stride);  // factor + solve + row_norm + post_solve (+ fit)
 int launch_factor(itcpd_plan* p, int mode);
 int launch_factor_on(itcpd_plan* p, int mode, hipStream_t st);
+size_t inv_stat_elems(int64_t R);              // doubles of p->inv_stat
 int launch_cp_check(itcpd_plan* p);
 // solve + row_norm + Gram refresh of `mode` (finalize), the fit after the last mode
 // (fit_after), then next_factor's factorisation (>= 0), all on the plan's stream

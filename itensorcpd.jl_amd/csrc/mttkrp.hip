@@ -294,6 +294,9 @@ __global__ __launch_bounds__(512, 1) void k_lp_ring(const float* __restrict__ T,
 }
 
 // ------------------------------------------------------- Hadamard-reduce (ttv)
+// Two waves a SIMD are asked for: the factorisation that rides along wants a register more than
+// they leave, and with one wave the reduces of 200 x 200 x 150 take 21 us instead of 14.
+//
 // M(i, r) = sum_{a<A, b<B} P(a + A*i + A*In*b, r) * Wa(a, r) * Wb(b, r)
 // Wa = product over the side's modes before `pos`, Wb over the modes after it
 // (column-major factors).  P has leading dimension MS and is the sum of np partials, pstride
@@ -321,7 +324,7 @@ __device__ __forceinline__ void side_weights(const Side& sd, int q0, int q1, int
 // HBM when large (512 x 512 x 64: 32 us, 4.2 TB/s).  When small, by the factorisation in the
 // same launch: In = 20, B = 342, R = 24 takes 11.1 us, 14.1 with the steps one by one.
 template <bool PARTS, typename I>
-__global__ __launch_bounds__(256) void k_ttv_lead(const double* __restrict__ P, int np, int64_t pstride,
+__global__ __launch_bounds__(256, 2) void k_ttv_lead(const double* __restrict__ P, int np, int64_t pstride,
                                                   int64_t MS, int64_t In, int R, Side sd, I B, I b_per_split,
                                                   double* __restrict__ out, int64_t split_stride,
                                                   FactorJob fj, const DevCheck* __restrict__ chk) {
@@ -363,7 +366,7 @@ __global__ __launch_bounds__(256) void k_ttv_lead(const double* __restrict__ P, 
 // left most lanes idle behind one load at a time where A is short: A = 20, In = 19, B = 18,
 // R = 24 took 18.6 us, now 10.8 with its factorisation.
 template <bool PARTS, int JW, int U, typename I>
-__global__ __launch_bounds__(256) void k_ttv_inner(const double* __restrict__ P, int np, int64_t pstride,
+__global__ __launch_bounds__(256, 2) void k_ttv_inner(const double* __restrict__ P, int np, int64_t pstride,
                                                    int64_t MS, int64_t In, int R, Side sd, int pos, I A, I B,
                                                    double* __restrict__ out, FactorJob fj,
                                                    const DevCheck* __restrict__ chk) {
@@ -423,7 +426,7 @@ __global__ __launch_bounds__(256) void k_ttv_inner(const double* __restrict__ P,
 
 // out[x] = sum_{z < nz} parts[z*stride + x] (fixed order); with fj on, block 0
 // runs that factorisation instead
-__global__ __launch_bounds__(256) void k_sum_parts(const double* __restrict__ parts, int nz,
+__global__ __launch_bounds__(256, 2) void k_sum_parts(const double* __restrict__ parts, int nz,
                                                    int64_t stride, int64_t n,
                                                    double* __restrict__ out, FactorJob fj,
                                                    const DevCheck* __restrict__ chk) {
@@ -544,9 +547,9 @@ __global__ __launch_bounds__(NW * 64, 4) void k_tr_ring(const double* __restrict
     constexpr int CPL = KS / 2;           // 16-byte chunks a lane reads per run
     extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
     if (fj.on && blockIdx.x == 0) {
-        // the unpivoted factorisation of mode fj.mode in this launch's LDS (no
-        // done test, as factor_block)
-        const bool ok = factor64_unpivoted(fj.gs, fj.mode, fj.R, fj.tol, fj.Vinv, fj.finfo, reinterpret_cast<double*>(ring));
+        // the unpivoted factorisation of mode fj.mode (R > 32: whole 64-rank tiles) in this
+        // launch's LDS (no done test, as factor_block)
+        const bool ok = factor64_unpivoted<false>(fj.gs, fj.mode, fj.R, fj.tol, fj.Vinv, fj.finfo, reinterpret_cast<double*>(ring));
         if (threadIdx.x == 0) fj.finfo[3] = ok ? 1 : 0;
         return;
     }

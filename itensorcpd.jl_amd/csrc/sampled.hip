@@ -169,7 +169,7 @@ __global__ __launch_bounds__(512) void k_sampled_products(const double* __restri
 __global__ __launch_bounds__(256) void k_sampled_inverse(const double* __restrict__ V, int n, double* __restrict__ Vinv,
                                                          int* __restrict__ info, const DevCheck* __restrict__ chk) {
     if (chk->done) return;
-    __shared__ double S[SWEEP_ROWS + 16];
+    __shared__ double S[FACTOR64_UNPIV];
     GramSet gs{};
     gs.G[0] = gs.G[1] = V;   // of mode 1: the other "Gram" alone
     gs.N = 2;

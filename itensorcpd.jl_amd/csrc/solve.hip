@@ -1508,13 +1508,14 @@ int launch_factor_on(itcpd_plan* p, int mode_in, hipStream_t st) {
         // V^-1 by blocks; the pivoted factorisation only when it is not certified
         const int nb = (int)cdiv(R, 64);
         const size_t half = (size_t)(64 * nb) * (64 * nb);
-        const dim3 grid((unsigned)nb, (unsigned)nb);
-        hipLaunchKernelGGL(k_inv_first, grid, dim3(256), (size_t)(INV_TILE + SWEEP_ROWS) * 8, st, gs, mode, R, nb, p->inv_buf,
-                           p->inv_P, p->inv_stat, p->chk);
-        for (int k = 0; k < nb; ++k)
-            hipLaunchKernelGGL(k_inv_step, grid, dim3(256), INV_LDS, st, k, R, nb, p->inv_buf + (k & 1) * half,
-                               p->inv_buf + ((k + 1) & 1) * half, p->inv_P + (k & 1) * 4096,
-                               p->inv_P + ((k + 1) & 1) * 4096, p->inv_stat, p->chk);
+        hipLaunchKernelGGL(k_inv_first, dim3((unsigned)nb, (unsigned)nb), dim3(256), INV_LDS, st, gs, mode, R, nb, p->inv_buf,
+                           p->inv_stat, p->chk);
+        for (int k = 1; k < nb; ++k)
+            hipLaunchKernelGGL(k_inv_step, dim3((unsigned)(nb - k), (unsigned)nb), dim3(256), INV_LDS, st, k, R, nb,
+                               p->inv_buf + ((k - 1) & 1) * half, p->inv_buf + (k & 1) * half, p->inv_stat, p->chk);
+        // into U: the pivoted kernels write it only when they do not exit on the certificate
+        hipLaunchKernelGGL(k_inv_product, dim3((unsigned)inv_tiles(R)), dim3(256), 0, st, R, nb, p->inv_buf, p->U,
+                           p->inv_stat, p->chk);
         ITCPD_HIP(hipGetLastError());
         if (R <= 128)
             hipLaunchKernelGGL(k_factor128, dim3(1), dim3(1024), F128_LDS, st, gs, mode, R, 1e-6, p->U, p->invdiag,
@@ -1570,11 +1571,8 @@ template <int RQ>
 int run_solve_k(itcpd_plan* p, int mode, const double* Msrc) {
     const int64_t In = p->dims[mode];
     const int R = (int)p->R;
-    const int nbq = (int)cdiv(R, 64);
-    const int64_t Rq = 64 * (int64_t)nbq;
     hipLaunchKernelGGL(k_solve_inv, dim3((unsigned)cdiv(In, 16), (unsigned)cdiv(cdiv(R, 16), 4)), dim3(256), 0,
-                       p->stream, Msrc, In, R, p->inv_buf + (nbq & 1) * (size_t)(Rq * Rq), Rq, p->finfo, p->X,
-                       p->chk);
+                       p->stream, Msrc, In, R, p->U, p->finfo, p->X, p->chk);
     const bool u_lds = R <= 128;
     constexpr int RPW = rpw_of<RQ>();
     const size_t lds = (size_t)4 * RPW * R * 8 + (u_lds ? (size_t)R * (R + 1) * 8 : 0);
