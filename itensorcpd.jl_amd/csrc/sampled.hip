@@ -162,10 +162,11 @@ __global__ __launch_bounds__(512) void k_sampled_products(const double* __restri
     }
 }
 
-// V^-1 by sweeps.  info = {n, 0, n} when certified, else info[1] = 1.  Certified means
-// ||V||_F ||V^-1||_F < 1e8, so cond(K) < 1e4: k_sampled_correct's one correction then leaves
-// (eps cond(K)^2)^2, far below the rounding of the QR solve it replaces, and K has full rank
-// by the QR's test (n eps).
+// V^-1 of the normal equations.  info = {n, 0, n} when certified, else info[1] = 1.  Certified
+// means ||V||_F ||V^-1||_F < 1e8, so cond(K) < 1e4, and V^-1 = W^T D^-1 W (factor64.h) solves to
+// at worst 1e-7 there: k_sampled_correct's one correction squares that, below the rounding of
+// the QR solve it replaces (1e-13; both sides of the certificate measure 6e-14 .. 1.5e-13 on
+// low-rank tensors), and K has full rank by the QR's test (n eps).
 __global__ __launch_bounds__(256) void k_sampled_inverse(const double* __restrict__ V, int n, double* __restrict__ Vinv,
                                                          int* __restrict__ info, const DevCheck* __restrict__ chk) {
     if (chk->done) return;
