@@ -1147,7 +1147,9 @@ int launch_right_gemm_impl(itcpd_plan* p, MSrc* ms, int factor_mode) {
         // Mode s's unpivoted factorisation rides in workgroup 0 (in the GEMM's LDS
         // budget, all workgroups resident at once) when a partial-sum launch follows
         // to run the pivoted fallback.  Its dependent steps then overlap the GEMM.
+        // With tiles for every slot nothing is split and no such launch follows.
         FactorJob fj = factor_job_for(p, factor_mode);
+        if (slots <= tiles) fj.on = 0;
         int64_t nz = split_for(fj.on ? slots - tiles : slots);
         if (fj.on && !(nz > 1 && !(consumer_sums && nz <= MAX_CONSUMER_PARTS) && slots - tiles * nz >= 1)) {
             fj.on = 0;
