@@ -747,10 +747,12 @@ int itcpd_sampled_solve(itcpd_plan* p, int32_t mode, int64_t nsamps, const int32
     if ((rc = launch_sampled_gather(p, mode, nsamps, p->smp_iws))) return rc;
     int form = normal ? SAMPLED_NORMAL : (sampled_corrected_ok(p, nsamps) ? SAMPLED_CORRECTED : SAMPLED_QR);
     int fi[4] = {0, 0, 0, 0};
+    const int* const status = p->smp_iws + nidx + p->R;
     for (;;) {
         if ((rc = launch_sampled_solve(p, mode, nsamps, form))) return rc;
-        if (!normal && (rc = launch_row_norm(p, mode))) return rc;
-        ITCPD_HIP(hipMemcpyAsync(fi, normal ? p->finfo : p->smp_iws + nidx + p->R, sizeof(fi), hipMemcpyDeviceToHost,
+        // the CPD takes no X that the corrected form has not certified
+        if (!normal && (rc = launch_row_norm(p, mode, form == SAMPLED_CORRECTED ? status + 1 : nullptr))) return rc;
+        ITCPD_HIP(hipMemcpyAsync(fi, normal ? p->finfo : status, sizeof(fi), hipMemcpyDeviceToHost,
                                  p->stream));
         ITCPD_HIP(hipStreamSynchronize(p->stream));
         if (form != SAMPLED_CORRECTED || fi[1] == 0) break;

@@ -233,7 +233,8 @@ int launch_cp_check(itcpd_plan* p);
 int launch_solve(itcpd_plan* p, int mode, const double* Msrc, int nparts, int64_t stride,
                  bool finalize, bool fit_after, int next_factor = -1);
 int launch_normalize(itcpd_plan* p, int mode, const double* Xsrc, bool fit_after);
-int launch_row_norm(itcpd_plan* p, int mode);   // (A_n, lambda) and G_n from p->X
+// (A_n, lambda) and G_n from p->X, unless *hold (device, nullable) is nonzero
+int launch_row_norm(itcpd_plan* p, int mode, const int* hold);
 int launch_seed_grams(itcpd_plan* p);
 int launch_reset_flags(itcpd_plan* p);         // chk->done = chk->nan_flag = 0
 int launch_random_init(itcpd_plan* p, uint64_t seed);

@@ -598,7 +598,7 @@ __global__ __launch_bounds__(256) void k_solve_mfma(const double* __restrict__ M
 // lambda_r = sqrt(sum_b gram_part[b](r,r)) (every block, fixed order); block k
 // writes its slice of G = S ./ (lambda lambda^T) (S = sum_b gram_part[b]) and of the
 // rows A = X ./ lambda, At; with `inner_part` it also sums <M, A .* lambda> over
-// its rows.
+// its rows.  hold (nullable): nonzero when X was not set, and the CPD stays as it is.
 __global__ __launch_bounds__(256) void k_finalize(const double* __restrict__ gram_part, int nb,
                                                   const double* __restrict__ X,
                                                   const double* __restrict__ Msum, int64_t In, int R,
@@ -606,8 +606,9 @@ __global__ __launch_bounds__(256) void k_finalize(const double* __restrict__ gra
                                                   double* __restrict__ At, double* __restrict__ lam,
                                                   double* __restrict__ Gout,
                                                   double* __restrict__ inner_part,
+                                                  const int* __restrict__ hold,
                                                   const DevCheck* __restrict__ chk) {
-    if (chk->done) return;
+    if (chk->done || (hold && *hold)) return;
     extern __shared__ double lamS[];
     __shared__ double red[256];
     const int t = threadIdx.x;
@@ -671,11 +672,12 @@ __global__ __launch_bounds__(256) void k_finalize_1rt(const double* __restrict__
                                                       double* __restrict__ At, double* __restrict__ lam,
                                                       double* __restrict__ Gout,
                                                       double* __restrict__ inner_part,
+                                                      const int* __restrict__ hold,
                                                       const DevCheck* __restrict__ chk) {
     __shared__ double lamS[256];
     __shared__ double red[256];
     const int t = threadIdx.x;
-    const int done = chk->done;
+    const int done = chk->done | (hold ? *hold : 0);
     const int64_t RR = (int64_t)R * R;
     const bool dr = t < R;
     const int64_t xd = dr ? (int64_t)t * R + t : 0;
@@ -1635,19 +1637,19 @@ int run_update_small(itcpd_plan* p, int mode, const double* Msrc, int nparts, in
 }
 
 // row_norm of X from nb Gram partials, with <M, X> for the fit when asked
-int run_finalize(itcpd_plan* p, int mode, int nb, const double* Mkept, bool fit) {
+int run_finalize(itcpd_plan* p, int mode, int nb, const double* Mkept, bool fit, const int* hold = nullptr) {
     const int64_t In = p->dims[mode];
     const int R = (int)p->R;
     const int nbf = finalize_nb(In, R);
     const bool one_rt = nb <= 32 && R <= 256 && cdiv((int64_t)R * R, nbf) <= 256 && cdiv(In, nbf) * R <= 2048;
     hipLaunchKernelGGL(one_rt ? k_finalize_1rt : k_finalize, dim3(nbf), dim3(256), one_rt ? 0 : (size_t)R * 8,
                        p->stream, p->gram_part, nb, p->X, Mkept, In, R, (int)p->Rp, p->A[mode], p->At[mode],
-                       p->lam, p->G[mode], fit ? p->inner_part : (double*)nullptr, p->chk);
+                       p->lam, p->G[mode], fit ? p->inner_part : (double*)nullptr, hold, p->chk);
     ITCPD_HIP(hipGetLastError());
     return ITCPD_OK;
 }
 // the same with X's Gram by a launch of its own
-int run_gram_finalize(itcpd_plan* p, int mode, const double* Mkept, bool fit) {
+int run_gram_finalize(itcpd_plan* p, int mode, const double* Mkept, bool fit, const int* hold = nullptr) {
     const int R = (int)p->R;
     GramJobs gj{};
     gj.X[0] = p->X;
@@ -1656,12 +1658,14 @@ int run_gram_finalize(itcpd_plan* p, int mode, const double* Mkept, bool fit) {
     const int nb = gram_parts(p->dims[mode], R);
     hipLaunchKernelGGL(k_gram_mfma, dim3(gram_tiles(R), (unsigned)nb), dim3(256), 0, p->stream, gj, R, nb, p->chk);
     ITCPD_HIP(hipGetLastError());
-    return run_finalize(p, mode, nb, Mkept, fit);
+    return run_finalize(p, mode, nb, Mkept, fit, hold);
 }
 
 }  // namespace
 
-int launch_row_norm(itcpd_plan* p, int mode) { return run_gram_finalize(p, mode, p->X, false); }
+int launch_row_norm(itcpd_plan* p, int mode, const int* hold) {
+    return run_gram_finalize(p, mode, p->X, false, hold);
+}
 
 int launch_solve(itcpd_plan* p, int mode, const double* Msrc, int nparts, int64_t stride,
                  bool finalize, bool fit_after, int next_factor) {

@@ -37,3 +37,25 @@ def test_step_on_a_low_rank_tensor(itcpd, dims, R, ns, near):
         got = plan.get_cpd()
     err = np.linalg.norm(got.factors[0] * got.lam - fac[0]) / np.linalg.norm(fac[0])
     assert err <= 2 * 8 * ns * EPS * np.linalg.cond(K)
+
+
+@pytest.mark.parametrize("dims,R,ns", [((20, 40, 30), 10, 300), ((300, 40, 30), 10, 300), ((17, 60, 50), 47, 900),
+                                       ((2100, 30, 40), 64, 1100)])
+def test_uncertified_step_sets_the_whole_cpd(itcpd, dims, R, ns):
+    """Equal columns: the corrected form leaves the CPD alone and the QR's solution sets factor,
+    lambda and Gram, also on a new plan whose solution buffer holds nothing yet.  Rank and
+    residual as least squares has them; V of mode 1 = G_0 .* G_2 within the rounding of its sums."""
+    T, fac, smp, K = problem(dims, R, ns, 0.0)
+    B = S.fused_flatten_sample(T, 0, smp)
+    rank = np.linalg.matrix_rank(K)
+    assert rank < R
+    with itcpd.ALSPlan(T, R) as plan:
+        plan.set_cpd(itcpd.CPD([np.ones((dims[0], R))] + fac[1:], np.ones(R)))
+        info = plan.sampled_solve(0, smp, False)
+        got = plan.get_cpd()
+        V = plan.compute_krp(1)
+    A, F = got.factors[0], fac[2]
+    assert info[1] == rank
+    assert np.linalg.norm(B.T - K @ (A * got.lam).T) <= 16 * ns * EPS * np.linalg.norm(K, 2) * np.linalg.norm(fac[0])
+    bound = 2 * (dims[0] + dims[2] + 8) * EPS * (np.abs(A).T @ np.abs(A)) * (np.abs(F).T @ np.abs(F))
+    assert (np.abs(V - (A.T @ A) * (F.T @ F)) / bound).max() <= 1.0
