@@ -23,7 +23,8 @@
 // form an E-element run of each of its columns.  The FP32 accumulators are added into FP64
 // ones every stage (FP32) or every 128 indices (BF16x3, whose parts round at 2^-18).  FP32, the
 // relative error of M on Gaussian data and the GEMMs' times below: 16 indices 7.8e-8, 243 / 281;
-// 8 indices 5.9e-8, 279 / 306; 32 1.05e-7, 250 / 301; 128 2.0e-7, 253 / 298.  MFMA 16x16x4
+// 8 indices 5.9e-8, 279 / 306; 32 1.05e-7, 250 / 301; 128 2.0e-7, 253 / 298 (the LDS ring form's
+// sums still run over 128).  MFMA 16x16x4
 // step s takes k = k0 + 4 g + s; result: lane (c, g), register v holds rank 4 g + v, output c.
 //
 // Measured per launch (left / right, us) on 150 x 130 x 110 x 90 FP32-stored, rank 48: FP32
