@@ -7,10 +7,7 @@ import oracle as O
 pytestmark = pytest.mark.gpu
 
 
-def workgroups():
-    """Workgroups of the ring form resident at once: four per compute unit."""
-    import torch
-    return 4 * torch.cuda.get_device_properties(0).multi_processor_count
+WORKGROUPS = 4 * 256   # of the ring form resident at once: four per compute unit
 
 
 @pytest.mark.parametrize("R", [33, 48])
@@ -19,7 +16,7 @@ def test_one_right_mode_of_whole_tiles(itcpd, per, R):
     """A matrix whose second mode has `per` tiles of 64 columns for every resident workgroup (the
     factorisation that may ride along takes one's place), one sweep against the oracle: a solve's
     8 R eps cond(V) on either side, V the Gram of the first mode's new factor."""
-    dims = (64, 64 * int(per * workgroups()))
+    dims = (64, 64 * int(per * WORKGROUPS))
     rng = np.random.default_rng(51)
     T = np.asfortranarray(rng.standard_normal((64, R)) @ rng.standard_normal((R, dims[1]))
                           + 1e-3 * rng.standard_normal(dims))
