@@ -376,7 +376,7 @@ int itcpd_plan_destroy(itcpd_plan* p) {
     dfree(p->lamprev);
     dfree(p->smp_ws);
     dfree(p->sk_ws);
-    dfree(p->P3);
+    dfree(p->P3_owned);
     dfree(p->smp_iws);
     dfree(p->xg_part);
     if (p->chk_host) (void)hipHostFree(p->chk_host);
@@ -524,10 +524,18 @@ int itcpd_run(itcpd_plan* p, itcpd_check* c, double* fit_trace) {
     c->converged = 0;
     if (nsweeps <= 0) return ITCPD_OK;
     p->tree3 = nsweeps > 1 && tree3_pays(p);
-    if (p->tree3 && !p->P3 && hipMalloc((void**)&p->P3, (size_t)tree3_elems(p) * 8) != hipSuccess) {
-        (void)hipGetLastError();   // no memory for it: the plain tree
-        p->P3 = nullptr;
-        p->tree3 = false;
+    if (p->tree3 && !p->P3) {
+        // the plain tree's partial, which a shared run does not use, where it is large enough
+        double* const side = p->s > 1 ? p->PL : p->PR;
+        if (tree3_elems(p) <= (p->s > 1 ? p->ML : p->MR) * p->R) {
+            p->P3 = side;
+        } else if (hipMalloc((void**)&p->P3_owned, (size_t)tree3_elems(p) * 8) == hipSuccess) {
+            p->P3 = p->P3_owned;
+        } else {
+            (void)hipGetLastError();   // no memory for it: the plain tree
+            p->P3_owned = nullptr;
+            p->tree3 = false;
+        }
     }
     if (nsweeps > p->trace_cap) {
         dfree(p->trace_owned);

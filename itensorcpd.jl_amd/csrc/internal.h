@@ -147,7 +147,8 @@ struct itcpd_plan {
     double* PL = nullptr;                      // ML x Rp partial of the left side (if s > 1)
     float* Kt = nullptr;                       // reduced precision: a side's Khatri-Rao product, rank-major
     double* Wrest = nullptr;                   // a side's Khatri-Rao product or rest weights (rank fastest)
-    double* P3 = nullptr;                      // order 3: the partial that serves two mode updates (tree3)
+    double* P3 = nullptr;                      // order 3: the partial that serves two mode updates (tree3):
+    double* P3_owned = nullptr;                // PL or PR, or this where neither is large enough
     bool tree3 = false;                        // order 3: partials shared across sweeps
     double* PR = nullptr;                      // MR x Rp partial of the right side (if N-s > 1)
     double* parts = nullptr;                   // split-K partial buffer

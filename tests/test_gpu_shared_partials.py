@@ -1,5 +1,7 @@
 """Order-3 sweeps on partials shared across updates, with the form that ran told by its GEMM
 launches: three for every two sweeps, the plain tree's two for each."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -31,3 +33,28 @@ def test_shared_partials_run_and_match_the_oracle(itcpd, dims, R, sweeps):
     for a, b in zip(got.factors, ref.factors):
         assert np.linalg.norm(a - b) <= 1e-10 * np.linalg.norm(b)
     assert np.linalg.norm(got.lam - ref.lam) <= 1e-10 * np.linalg.norm(ref.lam)
+
+
+def test_a_cube_needs_no_further_partial(itcpd):
+    """The shared partial of equal modes is no larger than the plain tree's, which the run does
+    not use: a run allocates nothing on the device."""
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free():
+        n, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(n), ctypes.byref(total)) == 0
+        return n.value
+
+    R = 48
+    T = np.asfortranarray(np.random.default_rng(63).standard_normal((256, 256, 256)))
+    init = itcpd.random_CPD(T, R, 64)
+    used = []
+    for _ in range(2):   # the first run loads the kernels
+        with itcpd.ALSPlan(T, R) as plan:
+            plan.set_cpd(init)
+            plan.set_profiling(True)
+            before = free()
+            plan.run(itcpd.NoCheck(4))
+            used.append(before - free())
+            assert plan.kernel_stats()["launches"] == 6
+    assert used[1] == 0
