@@ -223,6 +223,65 @@ __device__ __forceinline__ bool sweep_triangular(double (&a)[16], int n, int grp
 // distinct banks.
 __device__ __forceinline__ int tri_at(int ld, int r, int k) { return r * ld + (k ^ ((r & 1) << 4)); }
 
+// One Newton step Z <- Z + Z (I - V Z) for the inverse Z of V = Hadamard of the Grams of modes !=
+// mode, by the 256 threads of a workgroup on MFMA; returns the thread's share of ||I - V Z||_F^2.
+// D: 64 x 64 doubles of LDS.
+//
+// W is a left inverse of L to rounding (each of its columns is a substitution) and a right one only
+// to eps cond(V), so V W^T D^-1 W is off the identity by up to eps cond(V)^1.5; after the step
+// by that squared plus the step's own eps cond(V).  X from M = X V, worst of 6 seeds, without / with / by
+// the pivoted substitution: cond(V) 1e6 1e-10 / 1e-11 / 2e-11; 5e7 9e-8 / 5e-10 / 1e-9; 1e9 4e-6 / 2e-8 /
+// 2e-8.  Up to NEWTON_COND the two are alike.
+constexpr double NEWTON_COND = 1e4;
+__device__ __forceinline__ double newton_inverse(const GramSet& gs, int mode, int R, double* Z, double* D) {
+    const int l = threadIdx.x & 63, c = l & 15, g = l >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = 16 * w + c;   // this lane's row of the left operands
+    d4 acc[4];
+    double dsq = 0.0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[b][v] = 16 * w + g + 4 * v == 16 * b + c ? 1.0 : 0.0;
+    for (int k0 = 0; k0 < R; k0 += 4) {
+        const int k = k0 + g;
+        double a = k < R && i < R ? -1.0 : 0.0;
+        for (int m = 0; m < gs.N; ++m)
+            if (m != mode) a *= gs.G[m][k < R && i < R ? k * R + i : 0];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const int j = 16 * b + c;
+            const double z = Z[k < R && j < R ? k * R + j : 0];
+            acc[b] = mfma_f64(a, k < R && j < R ? z : 0.0, acc[b]);
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int r = 16 * w + g + 4 * v, j = 16 * b + c;
+            if (r < R && j < R) dsq = fma(acc[b][v], acc[b][v], dsq);
+            D[r * 64 + j] = acc[b][v];
+            acc[b][v] = r < R && j < R ? Z[r * R + j] : 0.0;
+        }
+    __syncthreads();
+    for (int k0 = 0; k0 < R; k0 += 4) {
+        const int k = k0 + g;
+        const double z = Z[k < R && i < R ? i * R + k : 0], a = k < R && i < R ? z : 0.0;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc[b] = mfma_f64(a, D[k * 64 + 16 * b + c], acc[b]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int r = 16 * w + g + 4 * v, j = 16 * b + c;
+            if (r < R && j < R) Z[r * R + j] = acc[b][v];
+        }
+    return dsq;
+}
+
 // Unpivoted V^-1 for the R <= 64 row solves (one 256-thread workgroup; the first wave alone
 // up to R = 32).
 //
@@ -231,10 +290,11 @@ __device__ __forceinline__ int tri_at(int ld, int r, int k) { return r * ld + (k
 // of a Schur complement of V, hence >= lambda_min(V), and lambda_min(V) >=
 // 1 / ||V^-1||_F.  The computed inverse is trusted while ||V||_F ||V^-1||_F < cond_max;
 // the bound must exceed 2 tol plus the pivots' rounding (64 R eps max V_ii); every
-// unpivoted pivot must be > 0.  Then the solution (the unique minimiser) is the
-// pivoted path's up to rounding (eps cond(V), the form's backward error), and V^-1 and finfo are written; otherwise it returns
-// false and writes nothing but V^-1 (which the caller's pivoted path overwrites or leaves
-// unused).  Uniform result.
+// unpivoted pivot must be > 0; and past NEWTON_COND, where a Newton step follows, the
+// ||I - V V^-1||_F^2 before it must be below eps cond(V).  Then the solution (the unique
+// minimiser) is the pivoted path's up to rounding (eps cond(V)), and V^-1 and finfo are
+// written; otherwise it returns false and writes nothing but V^-1 (which the caller's
+// pivoted path overwrites or leaves unused).  Uniform result.
 //
 // Bound by its chain of R / 2 steps, 0.5 us each, on one wave per SIMD.  The Hadamard-reduce of
 // 64 x 64 x 64 that carries it takes, us: R = 10 7.2, 16 8.6, 24 11.5, 37 17.9, 64 25.5 (Gauss-Jordan
@@ -386,8 +446,14 @@ __device__ __forceinline__ bool factor64_unpivoted(const GramSet& gs, int mode, 
             zs += red[8 + q];
         }
     const double vF = sqrt(vs), zF = sqrt(zs);
-    const bool cert = red[12] == 0.0 && zF > 0.0 && zF < __builtin_inf() &&
-                      1.0 / zF > 2.0 * tol + 64.0 * R * 0x1p-52 * dmax && vF * zF < cond_max;
+    bool cert = red[12] == 0.0 && zF > 0.0 && zF < __builtin_inf() &&
+                1.0 / zF > 2.0 * tol + 64.0 * R * 0x1p-52 * dmax && vF * zF < cond_max;
+    if (cert && vF * zF > NEWTON_COND) {
+        const double d = wave_sum_dpp(newton_inverse(gs, mode, R, Vinv, S));
+        if (l == 0) red[w] = d;
+        __syncthreads();
+        cert = (red[0] + red[1]) + (red[2] + red[3]) < 0x1p-52 * vF * zF;
+    }
     if (cert && t == 0) {
         finfo[0] = R;
         finfo[1] = 0;

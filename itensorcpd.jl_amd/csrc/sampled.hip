@@ -163,17 +163,15 @@ __global__ __launch_bounds__(512) void k_sampled_products(const double* __restri
 }
 
 // V^-1 of the normal equations.  info = {n, 0, n} when certified, else info[1] = 1.  Certified
-// means ||V||_F ||V^-1||_F < 1e8, so cond(K) < 1e4, and V^-1 = W^T D^-1 W (factor64.h) solves to
-// at worst 1e-7 there: k_sampled_correct's one correction squares that, below the rounding of
-// the QR solve it replaces (1e-13; both sides of the certificate measure 6e-14 .. 1.5e-13 on
-// low-rank tensors), and K has full rank by the QR's test (n eps).
-__global__ __launch_bounds__(256) void k_sampled_inverse(const double* __restrict__ V, int n, double* __restrict__ Vinv,
+// means ||V||_F ||V^-1||_F < 1e8, so cond(K) < 1e4, and V^-1 solves to eps cond(V), 1e-8 at
+// worst: k_sampled_correct's one correction squares that, below the rounding of the QR solve
+// it replaces (1e-13; both sides of the certificate measure 6e-14 .. 1.5e-13 on low-rank
+// tensors), and K has full rank by the QR's test (n eps).
+// gs: V as the only Gram of a mode 0, beside a mode 1.
+__global__ __launch_bounds__(256) void k_sampled_inverse(GramSet gs, int n, double* __restrict__ Vinv,
                                                          int* __restrict__ info, const DevCheck* __restrict__ chk) {
     if (chk->done) return;
     __shared__ double S[FACTOR64_UNPIV];
-    GramSet gs{};
-    gs.G[0] = gs.G[1] = V;   // of mode 1: the other "Gram" alone
-    gs.N = 2;
     if (!factor64_unpivoted(gs, 1, n, 0.0, Vinv, info, S, 1e8) && threadIdx.x == 0) info[1] = 1;
 }
 
@@ -1457,7 +1455,10 @@ int launch_sampled_solve(itcpd_plan* p, int mode, int64_t ns, int form) {
         return launch_solve(p, mode, p->M, 1, In * R, true, false);
     }
     if (form == SAMPLED_CORRECTED) {
-        hipLaunchKernelGGL(k_sampled_inverse, dim3(1), dim3(256), 0, p->stream, Vs, R, p->Upad, info, p->chk);
+        GramSet gs{};
+        gs.G[0] = gs.G[1] = Vs;
+        gs.N = 2;
+        hipLaunchKernelGGL(k_sampled_inverse, dim3(1), dim3(256), 0, p->stream, gs, R, p->Upad, info, p->chk);
         ITCPD_HIP(hipGetLastError());
         auto run = [&](auto kern, int threads) {
             hipLaunchKernelGGL(kern, dim3((unsigned)cdiv(In, 16)), dim3(threads), 0, p->stream, Ks, B, ns, R, In, p->M,
