@@ -322,7 +322,7 @@ __device__ __forceinline__ void side_weights(const Side& sd, int q0, int q1, int
 
 // The side's fastest mode: thread per (i, r), split over b; 8 steps of b in flight.  Bound by
 // HBM when large (512 x 512 x 64: 32 us, 4.2 TB/s).  When small, by the factorisation in the
-// same launch: In = 20, B = 342, R = 24 takes 11.1 us, 14.1 with the steps one by one.
+// same launch: In = 20, B = 342, R = 24 takes 14.0 us.
 template <bool PARTS, typename I>
 __global__ __launch_bounds__(256, 2) void k_ttv_lead(const double* __restrict__ P, int np, int64_t pstride,
                                                   int64_t MS, int64_t In, int R, Side sd, I B, I b_per_split,
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(256, 2) void k_ttv_lead(const double* __restrict__ 
 // (a, b) with U steps and the JW rows' loads in flight together, and share the weights over
 // the rows.  Bound as k_ttv_lead (512 x 512 x 64: 30 us).  Lanes over a alone, b one by one,
 // left most lanes idle behind one load at a time where A is short: A = 20, In = 19, B = 18,
-// R = 24 took 18.6 us, now 10.8 with its factorisation.
+// R = 24 took 18.6 us, now 13.1 with its factorisation.
 template <bool PARTS, int JW, int U, typename I>
 __global__ __launch_bounds__(256, 2) void k_ttv_inner(const double* __restrict__ P, int np, int64_t pstride,
                                                    int64_t MS, int64_t In, int R, Side sd, int pos, I A, I B,
