@@ -231,8 +231,9 @@ __device__ __forceinline__ int tri_at(int ld, int r, int k) { return r * ld + (k
 // to eps cond(V), so V W^T D^-1 W is off the identity by up to eps cond(V)^1.5; after the step
 // by that squared plus the step's own eps cond(V).  X from M = X V, worst of 6 seeds, without / with / by
 // the pivoted substitution: cond(V) 1e6 1e-10 / 1e-11 / 2e-11; 5e7 9e-8 / 5e-10 / 1e-9; 1e9 4e-6 / 2e-8 /
-// 2e-8.  Up to NEWTON_COND the two are alike.
-constexpr double NEWTON_COND = 1e4;
+// 2e-8.  Up to NEWTON_COND all are within a few units of eps cond(V), and the step would cost, us: R =
+// 10 3.6, 24 6.0, 37 8.6, 64 11.6.
+constexpr double NEWTON_COND = 1e5;
 __device__ __forceinline__ double newton_inverse(const GramSet& gs, int mode, int R, double* Z, double* D) {
     const int l = threadIdx.x & 63, c = l & 15, g = l >> 4;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -243,17 +244,29 @@ __device__ __forceinline__ double newton_inverse(const GramSet& gs, int mode, in
     for (int b = 0; b < 4; ++b)
 #pragma unroll
         for (int v = 0; v < 4; ++v) acc[b][v] = 16 * w + g + 4 * v == 16 * b + c ? 1.0 : 0.0;
-    for (int k0 = 0; k0 < R; k0 += 4) {
-        const int k = k0 + g;
-        double a = k < R && i < R ? -1.0 : 0.0;
-        for (int m = 0; m < gs.N; ++m)
-            if (m != mode) a *= gs.G[m][k < R && i < R ? k * R + i : 0];
+    for (int k0 = 0; k0 < R; k0 += 16) {   // four k-steps' loads in flight
+        double a[4], z[4][4];
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int j = 16 * b + c;
-            const double z = Z[k < R && j < R ? k * R + j : 0];
-            acc[b] = mfma_f64(a, k < R && j < R ? z : 0.0, acc[b]);
+        for (int s = 0; s < 4; ++s) {
+            const int k = k0 + 4 * s + g;
+            a[s] = k < R && i < R ? -1.0 : 0.0;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) z[s][b] = Z[k < R && 16 * b + c < R ? k * R + 16 * b + c : 0];
         }
+        for (int m = 0; m < gs.N; ++m) {
+            if (m == mode) continue;
+            const double* __restrict__ G = gs.G[m];
+            double v[4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) v[s] = G[k0 + 4 * s + g < R && i < R ? (k0 + 4 * s + g) * R + i : 0];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) a[s] *= v[s];
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+                acc[b] = mfma_f64(a[s], k0 + 4 * s + g < R && 16 * b + c < R ? z[s][b] : 0.0, acc[b]);
     }
 #pragma unroll
     for (int b = 0; b < 4; ++b)
@@ -265,11 +278,19 @@ __device__ __forceinline__ double newton_inverse(const GramSet& gs, int mode, in
             acc[b][v] = r < R && j < R ? Z[r * R + j] : 0.0;
         }
     __syncthreads();
-    for (int k0 = 0; k0 < R; k0 += 4) {
-        const int k = k0 + g;
-        const double z = Z[k < R && i < R ? i * R + k : 0], a = k < R && i < R ? z : 0.0;
+    for (int k0 = 0; k0 < R; k0 += 16) {
+        double a[4];
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[b] = mfma_f64(a, D[k * 64 + 16 * b + c], acc[b]);
+        for (int s = 0; s < 4; ++s) {
+            const int k = k0 + 4 * s + g;
+            a[s] = Z[k < R && i < R ? i * R + k : 0];
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int k = k0 + 4 * s + g;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) acc[b] = mfma_f64(k < R && i < R ? a[s] : 0.0, D[k * 64 + 16 * b + c], acc[b]);
+        }
     }
     __syncthreads();
 #pragma unroll
